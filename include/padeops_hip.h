@@ -201,6 +201,11 @@ int pdo_op_partition(pdo_op h, int kind, int bc1, int bcn, int *m, int *P);
  * single-segment tables.  Pass NULL arrays to query meta only. */
 int pdo_op_tables(pdo_op h, int kind, int bc1, int bcn, int general, int *meta, double *fac, double *spk,
                   double *G, double *sp);
+/* The same for the overlapping segments of other lengths: meta[9] = {m, P, K,
+ * nbl, nbr, q0, nd, d0, guni}, P == 0 where the variant does not take them;
+ * fac [4][m][5], spk [4][m][4], G [P][nd][2K][2K], sp [2][4][8]. */
+int pdo_op_overlap_tables(pdo_op h, int kind, int bc1, int bcn, int *meta, double *fac, double *spk, double *G,
+                          double *sp);
 
 /* ---- periodic FFT Poisson solver -----------------------------------------
  * replaces type(PoissonPeriodic), src/utilities/PoissonPeriodic.F90:

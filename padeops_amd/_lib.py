@@ -92,6 +92,7 @@ SIGNATURES = {
     "pdo_op_dims": ([_vp, _c_int, _pint, _pint], _c_int),
     "pdo_op_partition": ([_vp, _c_int, _c_int, _c_int, _pint, _pint], _c_int),
     "pdo_op_tables": ([_vp, _c_int, _c_int, _c_int, _c_int, _pint, _pdbl, _pdbl, _pdbl, _pdbl], _c_int),
+    "pdo_op_overlap_tables": ([_vp, _c_int, _c_int, _c_int, _pint, _pdbl, _pdbl, _pdbl, _pdbl], _c_int),
     "pdo_poisson_periodic_init": ([_pvp, _c_int, _c_int, _c_int, _c_double, _c_double, _c_double,
                                    _c_int, _c_int, _c_int, _c_int], _c_int),
     "pdo_poisson_periodic_init_k": ([_pvp, _c_int, _c_int, _c_int, _pdbl, _pdbl, _pdbl, _c_int], _c_int),

@@ -23,33 +23,17 @@
 //     coalesced loads, lanes are (pencil, segment) pairs reading their window
 //     from LDS (segment rows padded by one element against bank conflicts),
 //     and results go back through LDS to coalesced stores.
-// Sizes outside the register path (n not a multiple of 32 or above 512) use a
-// one-lane-per-pencil kernel with global scratch, computing in FP64.
+// Other sizes, and the x pencils the x kernel does not take, run on the
+// overlapping segments of pdo_overlap.hip; what those leave (n below 16 or
+// above 1024, epilogue operands) uses a one-lane-per-pencil kernel with
+// global scratch, computing in FP64.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
 
-#include "pdo_kernels.hpp"
+#include "pdo_stencil.hpp"
 
 namespace pdo {
-
-template <int FAM> struct Fam;
-//                                  K  R  sigma shift center
-#define PDO_FAM(ID, K_, R_, S_, H_, C_)                                                   \
-    template <> struct Fam<ID> {                                                          \
-        static constexpr int K = K_, R = R_, SIGMA = S_, SHIFT = H_;                      \
-        static constexpr bool CENTER = C_;                                                \
-    };
-PDO_FAM(0, 1, 2, -1, 0, false)   // cd06 d1
-PDO_FAM(1, 1, 2, +1, 0, true)    // cd06 d2, staggered d2
-PDO_FAM(2, 2, 3, -1, 0, false)   // cd10 d1
-PDO_FAM(3, 2, 3, +1, 0, true)    // cd10 d2
-PDO_FAM(4, 2, 4, +1, 0, true)    // cf90
-PDO_FAM(5, 1, 2, -1, +1, false)  // staggered ddz E2C
-PDO_FAM(6, 1, 2, -1, -1, false)  // staggered ddz C2E
-PDO_FAM(7, 1, 2, +1, +1, false)  // staggered interp E2C
-PDO_FAM(8, 1, 2, +1, -1, false)  // staggered interp C2E
-#undef PDO_FAM
 
 template <int MODE> struct Mode;
 template <> struct Mode<MODE_F64> { using TS = double; using TC = double; static constexpr bool REFINE = false; };
@@ -62,23 +46,6 @@ template <typename T> __device__ __forceinline__ const T *tab(const ApplyArgs &A
 template <> __device__ __forceinline__ const double *tab<double>(const ApplyArgs &A) { return A.tab_d; }
 template <> __device__ __forceinline__ const float *tab<float>(const ApplyArgs &A) { return A.tab_f; }
 
-
-// interior stencil of output row j; window index of input row (row0 + j + o)
-// is j + R + o.
-template <int FAM, typename T, typename TW, int W>
-__device__ __forceinline__ T stencil_row(const TW (&win)[W], int j, const T *c)
-{
-    using F = Fam<FAM>;
-    T acc = F::CENTER ? c[0] * (T)win[j + F::R] : T(0);
-#pragma unroll
-    for (int q = 1; q <= F::R; ++q) {
-        const int hi = j + F::R + q + (F::SHIFT < 0 ? -1 : 0);
-        const int lo = j + F::R - q + (F::SHIFT > 0 ? 1 : 0);
-        const T pr = F::SIGMA > 0 ? (T)win[hi] + (T)win[lo] : (T)win[hi] - (T)win[lo];
-        acc = fma(c[q], pr, acc);
-    }
-    return acc;
-}
 
 // right closure row against input columns [n_in - WBMAX, n_in): window index
 // MSEG + R - WBMAX + q + DN with DN = n_in - n_sys (MSEG: rows of the last
@@ -150,37 +117,6 @@ __device__ __forceinline__ T rhs_row(const TW (&win)[W], int j, const T *c, cons
 // choice.
 template <int FAM, bool PER> constexpr bool rhs1_fp64() { return PER && Fam<FAM>::R > 2; }
 
-// local banded solve, in place, factors fac[j*5 + {l1,l2,inv,u1,u2}]
-// Scheduling fence every SB rows: the row coefficients are uniform scalar
-// loads; without a fence the scheduler hoists all of them (hundreds of
-// values) and spills scalar registers into vector lanes.
-#define PDO_SCHED_FENCE(j, SB) \
-    if (((j) % (SB)) == (SB) - 1) __builtin_amdgcn_sched_barrier(0)
-
-template <int K, int MM, bool EXACT, typename T, typename PT>
-__device__ __forceinline__ void local_solve(T (&d)[MM], PT fac, int m)
-{
-#pragma unroll
-    for (int j = 1; j < MM; ++j) {
-        if (EXACT || j < m) {
-            T v = d[j] - fac[j * 5 + 0] * d[j - 1];
-            if (K == 2 && j >= 2) v -= fac[j * 5 + 1] * d[j - 2];
-            d[j] = v;
-        }
-        PDO_SCHED_FENCE(j, 8);
-    }
-#pragma unroll
-    for (int j = MM - 1; j >= 0; --j) {
-        if (EXACT || j < m) {
-            T v = d[j] * fac[j * 5 + 2];
-            if (j + 1 < MM && (EXACT || j + 1 < m)) v -= fac[j * 5 + 3] * d[j + 1];
-            if (K == 2 && j + 2 < MM && (EXACT || j + 2 < m)) v -= fac[j * 5 + 4] * d[j + 2];
-            d[j] = v;
-        }
-        PDO_SCHED_FENCE(j, 8);
-    }
-}
-
 // the same for segments of MAXM rows, or MAXM + 1 when `ext` (MM = MAXM + 1)
 template <int K, int MM, typename T, typename PT>
 __device__ __forceinline__ void local_solve_x(T (&d)[MM], PT fac, bool ext)
@@ -236,24 +172,6 @@ __device__ __forceinline__ void publish_ends(T *rb, const T (&d)[MM], int s, int
         T v = d[MAXM - K + q];
         if constexpr (MM > MAXM) v = ext ? d[MAXM + 1 - K + q] : v;
         rb[(s * 2 * K + K + q) * NPW + pl] = v;
-    }
-}
-
-template <int K, int MM, bool EXACT, typename T, typename PT>
-__device__ __forceinline__ void apply_spikes(T (&d)[MM], PT spk, const T (&yl)[2], const T (&yr)[2], int m)
-{
-#pragma unroll
-    for (int j = 0; j < MM; ++j) {
-        if (EXACT || j < m) {
-            T v = d[j];
-#pragma unroll
-            for (int q = 0; q < K; ++q) {
-                v = fma(-spk[j * 4 + q], yl[q], v);
-                v = fma(-spk[j * 4 + 2 + q], yr[q], v);
-            }
-            d[j] = v;
-        }
-        PDO_SCHED_FENCE(j, 8);
     }
 }
 

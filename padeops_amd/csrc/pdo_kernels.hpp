@@ -11,7 +11,8 @@ constexpr int NBMAX = 4;   // closure rows per end of a non-periodic system
 constexpr int WBMAX = 8;   // closure columns per end
 
 enum KMode : int { MODE_F64 = 0, MODE_F32R = 1, MODE_F32S = 2, MODE_F32 = 3 };
-enum KShape : int { SHAPE_STRIDED = 0, SHAPE_X = 1, SHAPE_GENERAL = 2 };
+enum KShape : int { SHAPE_STRIDED = 0, SHAPE_X = 1, SHAPE_GENERAL = 2, SHAPE_OVL_STRIDED = 3, SHAPE_OVL_X = 4 };
+constexpr int OVL_PMAX = 32;  // most overlapping segments per pencil (n <= 1024 on that path)
 
 // Arguments of one apply launch (passed by value).  A pencil is addressed by
 // (a, b): input element r of pencil (a,b) is f[a*sa_in + b*sb_in + r*se_in].
@@ -34,12 +35,18 @@ struct ApplyArgs {
     const double *tab_d;
     const float *tab_f;
     int o_fac, o_spk, o_lhs, o_G, o_sp;
+    // overlapping segments (SHAPE_OVL_*): rows between segment starts (q0 or
+    // q0 + 1), segments coupled to one (nd, from d0 relative to it), and
+    // whether every segment has the same coupling rows
+    int q0, nd, d0, guni;
+    unsigned smul, sdiv;  // start of segment s: s smul / D by the reciprocal sdiv = 2^31 / D + 1 (2^31: D = 1)
     double c[5];
     double band[5];    // interior LHS band (offsets -2..2), used by periodic systems
 };
 
 hipError_t launch_absmax(const void *x, bool is_double, long n, double *partial, int nblocks, hipStream_t st);
 hipError_t launch_zero_words(void *p, long words, hipStream_t st);
+hipError_t launch_overlap(int family, int shape, bool dbl, const ApplyArgs &A, hipStream_t st);
 hipError_t launch_compact(int family, int shape, int mode, const ApplyArgs &A, double *scratch, hipStream_t st);
 
 }  // namespace pdo

@@ -1,7 +1,9 @@
 // Allocation-free compact-operator entry point, pdo_op_apply_noalloc.
 //
-// The one-lane-per-pencil kernel (sizes outside the register path) keeps an
-// FP64 work area of n_sys values per pencil.  The ordinary entry points take
+// The one-lane-per-pencil kernel (sizes outside the register paths) keeps an
+// FP64 work area of n_sys values per pencil; calls that leave the fixed
+// register kernels are held to its size here, also where overlapping segments
+// serve them without a work area.  The ordinary entry points take
 // it from stream-ordered memory per call; this one takes it from `scratch`, a
 // fixed array in device memory of which every device holds its own copy for
 // the life of the process.  Nothing here calls hipMalloc or hipFree, so

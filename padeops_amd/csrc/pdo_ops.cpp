@@ -20,14 +20,12 @@ int hip_fail(hipError_t e, const char *what)
     return PDO_ERR_HIP;
 }
 
-TabSet::~TabSet()
+Variant::~Variant()
 {
-    if (d_tab) (void)hipFree(d_tab);
-    if (f_tab) (void)hipFree(f_tab);
+    if (mem) (void)hipFree(mem);
 }
 
-// one device buffer per precision: fac | spk | lhs | G | sp
-int TabSet::upload()
+std::vector<double> TabSet::pack()
 {
     const SpikeTables &t = tab;
     std::vector<double> all;
@@ -36,16 +34,53 @@ int TabSet::upload()
     o_lhs = (int)all.size(); all.insert(all.end(), t.lhs.begin(), t.lhs.end());
     o_G = (int)all.size(); all.insert(all.end(), t.G.begin(), t.G.end());
     o_sp = (int)all.size(); all.insert(all.end(), t.sp.begin(), t.sp.end());
-    std::vector<float> allf(all.begin(), all.end());
-    hipError_t e = hipMalloc(&d_tab, all.size() * sizeof(double));
+    return all;
+}
+
+// every table of the variant in one device buffer, by one copy: the FP64
+// tables, then the FP32 copies of the partitioned ones
+int Variant::upload()
+{
+    std::vector<double> a = fast.pack(), g, o;
+    const bool single = !fast.tab.general;
+    if (single) g = gen.pack();
+    if (ovl.P > 0) {
+        // per segment type: lower factors, pivots and upper factors, spikes
+        const int K = ovl.K, m = ovl.m;
+        for (int ty = 0; ty < 4; ty++) {
+            const double *F = &ovl.fac[ty * m * 5], *S = &ovl.spk[ty * m * 4];
+            for (int j = 0; j < m; j++) o.insert(o.end(), F + j * 5, F + j * 5 + K);
+            for (int j = 0; j < m; j++) o.insert(o.end(), F + j * 5 + 2, F + j * 5 + 3 + K);
+            for (int j = 0; j < m; j++) {
+                o.insert(o.end(), S + j * 4, S + j * 4 + K);
+                o.insert(o.end(), S + j * 4 + 2, S + j * 4 + 2 + K);
+            }
+        }
+        ov_G = (int)o.size(); o.insert(o.end(), ovl.G.begin(), ovl.G.end());
+        ov_sp = (int)o.size(); o.insert(o.end(), ovl.sp.begin(), ovl.sp.end());
+    }
+    // each set starts on a 256-byte boundary, as allocations of its own would
+    auto up = [](size_t words) { return (words + 31) & ~(size_t)31; };
+    const size_t wa = up(a.size()), wg = up(g.size()), wo = up(o.size()), wf = up((a.size() + 1) / 2);
+    std::vector<double> host(wa + wg + wo + wf, 0.0);
+    std::copy(a.begin(), a.end(), host.begin());
+    std::copy(g.begin(), g.end(), host.begin() + wa);
+    std::copy(o.begin(), o.end(), host.begin() + wa + wg);
+    const std::vector<float> f(a.begin(), a.end());
+    std::memcpy(host.data() + wa + wg + wo, f.data(), f.size() * sizeof(float));
+    hipError_t e = hipMalloc(&mem, host.size() * sizeof(double));
     if (e != hipSuccess) return hip_fail(e, "hipMalloc(tables)");
-    e = hipMalloc(&f_tab, allf.size() * sizeof(float));
-    if (e != hipSuccess) return hip_fail(e, "hipMalloc(tables)");
-    e = hipMemcpy(d_tab, all.data(), all.size() * sizeof(double), hipMemcpyHostToDevice);
+    e = hipMemcpy(mem, host.data(), host.size() * sizeof(double), hipMemcpyHostToDevice);
     if (e != hipSuccess) return hip_fail(e, "hipMemcpy(tables)");
-    e = hipMemcpy(f_tab, allf.data(), allf.size() * sizeof(float), hipMemcpyHostToDevice);
-    if (e != hipSuccess) return hip_fail(e, "hipMemcpy(tables)");
-    ready = true;
+    double *d = (double *)mem;
+    fast.d_tab = d;
+    fast.f_tab = (float *)(d + wa + wg + wo);
+    fast.ready = true;
+    if (single) {
+        gen.d_tab = d + wa;
+        gen.ready = true;
+    }
+    d_ovl = d + wa + wg;
     return 0;
 }
 
@@ -102,13 +137,15 @@ int OpObject::variant(int kind, int b1, int bn, Variant **out)
     }
     st = build_spike(v->sys, v->fast.tab);
     if (st) { set_error("failed to build the partitioned-solve tables"); return PDO_ERR_ARG; }
-    if ((st = v->fast.upload())) return st;
-    // the single-segment tables of the general kernel too (a few KB), so that
-    // every shape the variant can take is ready once the variant exists
-    if (!v->fast.tab.general) {
-        if (build_spike(v->sys, v->gen.tab, true)) { set_error("failed to build tables"); return PDO_ERR_ARG; }
-        if ((st = v->gen.upload())) return st;
+    // the single-segment tables of the general kernel and those of the
+    // overlapping segments too (a few KB), so that every shape the variant
+    // can take is ready once the variant exists
+    if (!v->fast.tab.general && build_spike(v->sys, v->gen.tab, true)) {
+        set_error("failed to build tables");
+        return PDO_ERR_ARG;
     }
+    build_overlap(v->sys, v->ovl);
+    if ((st = v->upload())) return st;
     *out = v.get();
     variants[key] = std::move(v);
     return 0;
@@ -123,6 +160,29 @@ int prec_mode(int prec)
     case PDO_F32: return MODE_F32;
     }
     return -1;
+}
+
+// whether the overlapping-segment kernels take a call
+static bool overlap_fits(const Variant &v, int dir, long na, long nb, size_t word)
+{
+    const SystemDesc &s = v.sys;
+    const OverlapTables &o = v.ovl;
+    const FamShape f = family_shape(s.family);
+    if (o.P <= 0) return false;
+    if (dir == 1) {
+        if (f.shift != 0 || s.n_in != s.n_sys || s.n_out != s.n_sys) return false;
+        // at least 8 pencils fit a workgroup's LDS, with the exchange values and tables
+        const size_t pen = (size_t)(s.n_sys | 1) * word + (size_t)o.P * 2 * o.K * 8;
+        return 8 * pen + (s.periodic ? 0 : 3 * (size_t)o.m * 9 * 8) <= 160 * 1024 &&
+               (size_t)na * nb < ((size_t)1 << 31);
+    }
+    if (o.P > PMAX && (f.shift != 0 || o.m != MAXM)) return false;
+    // pencils are addressed by 32-bit byte offsets within the field, or
+    // within one plane of a larger one
+    const size_t nmax = (size_t)std::max(std::max(s.n_in, s.n_out), s.n_sys + 1);
+    const size_t lim = (size_t)1 << 32;
+    if ((size_t)na * nb * nmax * word < lim) return true;
+    return dir == 3 ? (size_t)na * nb * word < lim : ((size_t)na * word < lim && nb <= 65535);
 }
 
 // Validate one apply call and fill its launch arguments; *empty is set when
@@ -175,6 +235,12 @@ static int prepare(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, 
     // an extra row in the last segment only in the tridiagonal families
     if (shape == SHAPE_STRIDED && !s.periodic && (epi || (v->fast.tab.xr && family_shape(s.family).K != 1)))
         shape = SHAPE_GENERAL;
+    // sizes and ends without a register kernel of their own: overlapping
+    // segments, where they fit (n >= 16, at most 512 rows, 1024 of the
+    // collocated operators), else one lane per pencil
+    scratch_elems = (shape == SHAPE_GENERAL) ? (size_t)s.n_sys * (size_t)(na * nb) : 0;
+    if (shape == SHAPE_GENERAL && force_shape != SHAPE_GENERAL && !epi && overlap_fits(*v, dir, na, nb, word))
+        shape = dir == 1 ? SHAPE_OVL_X : SHAPE_OVL_STRIDED;
     TabSet *ts = &v->fast;
     if (shape == SHAPE_GENERAL && !v->fast.tab.general) {
         // built with the variant
@@ -210,8 +276,25 @@ static int prepare(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, 
         A.sa_in = 1; A.sb_in = 0; A.se_in = na * nb;
         A.sa_out = 1; A.sb_out = 0; A.se_out = na * nb;
     }
-    scratch_elems = (shape == SHAPE_GENERAL) ? (size_t)s.n_sys * (size_t)(A.na * A.nb) : 0;
+    if (shape == SHAPE_OVL_X || shape == SHAPE_OVL_STRIDED) {
+        const OverlapTables &o = v->ovl;
+        A.m = o.m; A.P = o.P; A.xr = 0; A.nbl = o.nbl; A.nbr = o.nbr;
+        A.q0 = o.q0; A.nd = o.nd; A.d0 = o.d0; A.guni = o.guni;
+        const int steps = s.periodic ? o.P : std::max(o.P - 1, 1);
+        A.smul = s.periodic ? s.n_sys : (o.P > 1 ? s.n_sys - o.m : 0);
+        A.sdiv = steps > 1 ? (1u << 31) / steps + 1 : 1u << 31;
+        A.tab_d = v->d_ovl; A.tab_f = nullptr;
+        A.o_fac = 0; A.o_G = v->ov_G; A.o_sp = v->ov_sp;
+    }
     return 0;
+}
+
+// launch of a prepared call; `work` serves the general kernel
+static hipError_t launch(int family, int shape, int mode, const ApplyArgs &A, double *work, hipStream_t stream)
+{
+    if (shape == SHAPE_OVL_X || shape == SHAPE_OVL_STRIDED)
+        return launch_overlap(family, shape, mode == MODE_F64, A, stream);
+    return launch_compact(family, shape, mode, A, work, stream);
 }
 
 int apply(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, const void *f, void *out, long na, long nb,
@@ -229,11 +312,11 @@ int apply(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, const voi
     // run concurrently on different streams
     double *scratch = nullptr;
     hipError_t e = hipSuccess;
-    if (scratch_elems) {
+    if (shape == SHAPE_GENERAL) {
         e = hipMallocAsync((void **)&scratch, scratch_elems * sizeof(double), stream);
         if (e != hipSuccess) return hip_fail(e, "hipMallocAsync(general-kernel work area)");
     }
-    e = launch_compact(family, shape, mode, A, scratch, stream);
+    e = launch(family, shape, mode, A, scratch, stream);
     if (scratch) {
         const hipError_t ef = hipFreeAsync(scratch, stream);
         if (e == hipSuccess) e = ef;
@@ -273,12 +356,14 @@ int apply_noalloc(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, c
     int st = prepare(op, kind, bc1, bcn, dir, prec, f, out, na, nb, 0, nullptr, -1, A, shape, mode, family,
                      scratch_elems, &empty, true);
     if (st || empty) return st;
+    // the limit is the entry point's contract for every call outside the fixed
+    // register kernels, whichever kernel serves it
     if (scratch_elems > work_elems) {
         set_error("input too large for the fixed work area of the allocation-free entry point (" +
                   std::to_string(scratch_elems) + " > " + std::to_string(work_elems) + " FP64 words)");
         return PDO_ERR_ARG;
     }
-    const hipError_t e = launch_compact(family, shape, mode, A, scratch_elems ? work : nullptr, stream);
+    const hipError_t e = launch(family, shape, mode, A, shape == SHAPE_GENERAL ? work : nullptr, stream);
     if (e != hipSuccess) return hip_fail(e, "kernel launch");
     return 0;
 }
@@ -578,6 +663,24 @@ int pdo_op_tables(pdo_op h, int kind, int bc1, int bcn, int general, int *meta, 
     if (spk) std::memcpy(spk, t.spk.data(), t.spk.size() * sizeof(double));
     if (G) std::memcpy(G, t.G.data(), t.G.size() * sizeof(double));
     if (sp) std::memcpy(sp, t.sp.data(), t.sp.size() * sizeof(double));
+    return 0;
+}
+
+int pdo_op_overlap_tables(pdo_op h, int kind, int bc1, int bcn, int *meta, double *fac, double *spk, double *G,
+                          double *sp)
+{
+    if (!h || !meta) return PDO_ERR_ARG;
+    SystemDesc s;
+    int st = build_desc(*h, kind, h->periodic ? 0 : bc1, h->periodic ? 0 : bcn, s);
+    if (st) return st;
+    OverlapTables t;
+    build_overlap(s, t);
+    const int m[9] = {t.m, t.P, t.K, t.nbl, t.nbr, t.q0, t.nd, t.d0, t.guni};
+    std::copy(m, m + 9, meta);
+    if (fac) std::copy(t.fac.begin(), t.fac.end(), fac);
+    if (spk) std::copy(t.spk.begin(), t.spk.end(), spk);
+    if (G) std::copy(t.G.begin(), t.G.end(), G);
+    if (sp) std::copy(t.sp.begin(), t.sp.end(), sp);
     return 0;
 }
 

@@ -9,6 +9,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <vector>
 
 #include "pdo_system.hpp"
 
@@ -17,20 +18,26 @@ namespace pdo {
 void set_error(const std::string &msg);
 int hip_fail(hipError_t e, const char *what);
 
+// one set of tables in device memory: fac | spk | lhs | G | sp
 struct TabSet {
     SpikeTables tab;
     double *d_tab = nullptr;  // device: FP64 tables
     float *f_tab = nullptr;   // device: FP32 copies
     int o_fac = 0, o_spk = 0, o_lhs = 0, o_G = 0, o_sp = 0;
     bool ready = false;
-    int upload();
-    ~TabSet();
+    std::vector<double> pack();  // the set's tables in order, and its offsets
 };
 
 struct Variant {
     SystemDesc sys;
     TabSet fast;   // partitioned tables (general == true when n does not fit)
-    TabSet gen;    // single-segment tables of the general kernel, built on demand
+    TabSet gen;    // single-segment tables of the general kernel, where fast is not general itself
+    OverlapTables ovl;         // overlapping segments (P == 0: not for this system)
+    const double *d_ovl = nullptr;
+    int ov_G = 0, ov_sp = 0;
+    void *mem = nullptr;       // device memory of every table above
+    int upload();
+    ~Variant();
 };
 
 struct OpObject {

@@ -826,4 +826,157 @@ int build_spike(const SystemDesc &s, SpikeTables &t, bool force_general)
     return 0;
 }
 
+// banded LU of rows [r0, r0 + m) taken alone, and the solutions for the K
+// coupling columns on either side; the layouts of SpikeTables
+static bool local_tables(const SystemDesc &s, int r0, int m, bool has_prev, bool has_next, double *fac, double *spk)
+{
+    const int K = s.K, n = s.n_sys;
+    auto band = [&](int j, int o) { return s.lhs[(r0 + j) % n][o + 2]; };
+    std::vector<double> l1(m, 0), l2(m, 0), u0(m, 0), u1(m, 0), u2(m, 0);
+    for (int j = 0; j < m; j++) {
+        auto in = [&](int o) { return (j + o >= 0 && j + o < m) ? band(j, o) : 0.0; };
+        const double L2 = j >= 2 ? in(-2) / u0[j - 2] : 0.0;
+        const double L1 = j >= 1 ? (in(-1) - (j >= 2 ? L2 * u1[j - 2] : 0.0)) / u0[j - 1] : 0.0;
+        u0[j] = in(0) - (j >= 1 ? L1 * u1[j - 1] : 0.0) - (j >= 2 ? L2 * u2[j - 2] : 0.0);
+        u1[j] = in(1) - (j >= 1 ? L1 * u2[j - 1] : 0.0);
+        u2[j] = in(2);
+        if (u0[j] == 0.0) return false;
+        l1[j] = L1; l2[j] = L2;
+        double *F = fac + j * 5;
+        F[0] = L1; F[1] = L2; F[2] = 1.0 / u0[j]; F[3] = u1[j] / u0[j]; F[4] = u2[j] / u0[j];
+    }
+    for (int r = 0; r < 2 * K; r++) {
+        // columns -K + r (r < K) and m + r - K
+        const int col = r < K ? -K + r : m + r - K;
+        std::vector<double> v(m, 0.0);
+        if (r < K ? has_prev : has_next)
+            for (int j = 0; j < m; j++)
+                if (col - j >= -2 && col - j <= 2) v[j] = band(j, col - j);
+        for (int j = 0; j < m; j++) {
+            if (j >= 1) v[j] -= l1[j] * v[j - 1];
+            if (j >= 2) v[j] -= l2[j] * v[j - 2];
+        }
+        for (int j = m - 1; j >= 0; j--) {
+            if (j + 1 < m) v[j] -= u1[j] * v[j + 1];
+            if (j + 2 < m) v[j] -= u2[j] * v[j + 2];
+            v[j] /= u0[j];
+        }
+        for (int j = 0; j < m; j++) spk[j * 4 + (r < K ? r : 2 + r - K)] = v[j];
+    }
+    return true;
+}
+
+// 32-row segments where they fit, 16-row ones for short pencils.  A segment
+// must own at least K rows (its neighbours read K rows of it), and without
+// periodicity only the first and the last may hold closure rows, so the
+// second starts, and the last but one ends, past them.  Periodic pencils
+// take a few segments more where that makes all of them own equally many
+// rows: the coupling rows are then the same for every segment.
+// `exact`: rows beyond the period may not stand in for the first ones (an
+// edge field's last point is read as it is stored), so n is a multiple of m.
+static bool choose_overlap(int n, int K, int nb, bool periodic, bool exact, int &m, int &P)
+{
+    for (m = MAXM; m >= MAXM / 2; m /= 2) {
+        if (n < m || (exact && n % m != 0)) continue;
+        P = (n + m - 1) / m;
+        if (P > OVL_PMAX) return false;
+        if (exact) return P <= PMAX;
+        if (periodic) {
+            for (int p = P; p <= P + P / 4 && p <= (P <= PMAX ? PMAX : OVL_PMAX); p++)
+                if (n % p == 0) { P = p; break; }
+            if (n / P >= K) return true;
+        } else if (P == 1 || (n - m) / (P - 1) >= std::max(nb, K)) {
+            return true;
+        }
+    }
+    return false;
+}
+
+void build_overlap(const SystemDesc &s, OverlapTables &t)
+{
+    t = OverlapTables();
+    const int n = s.n_sys, K = s.K, K2 = 2 * K;
+    for (auto &kv : s.special) {
+        if (kv.first < n / 2) t.nbl = std::max(t.nbl, kv.first + 1);
+        else t.nbr = std::max(t.nbr, n - kv.first);
+    }
+    int m, P;
+    if (t.nbl > NBMAX || t.nbr > NBMAX || (!s.periodic && n < 2 * WBMAX)) return;
+    if (!choose_overlap(n, K, NBMAX, s.periodic, s.periodic && n_read(s) != n, m, P)) return;
+    t.m = m; t.P = P; t.K = K;
+    t.q0 = s.periodic ? n / P : (P > 1 ? (n - m) / (P - 1) : m);
+    t.fac.assign(4 * m * 5, 0.0);
+    t.spk.assign(4 * m * 4, 0.0);
+    t.sp.assign(2 * NBMAX * WBMAX, 0.0);
+    for (auto &kv : s.special) {
+        const bool left = kv.first < n / 2;
+        const int jr = left ? kv.first : kv.first - (n - t.nbr);
+        for (auto &cw : kv.second) {
+            const int c = left ? cw.first : cw.first - (s.n_in - WBMAX);
+            if (c < 0 || c >= WBMAX) { t.P = 0; return; }
+            t.sp[((left ? 0 : 1) * NBMAX + jr) * WBMAX + c] += cw.second;
+        }
+    }
+    auto type_of = [&](int sg) { return s.periodic ? 1 : (P == 1 ? 3 : (sg == 0 ? 0 : (sg == P - 1 ? 2 : 1))); };
+    auto st = [&](int sg) { return t.start(sg, n, s.periodic); };
+    bool built[4] = {false, false, false, false};
+    for (int sg = 0; sg < P; sg++) {
+        const int ty = type_of(sg);
+        if (built[ty]) continue;
+        built[ty] = true;
+        if (!local_tables(s, st(sg), m, s.periodic || sg > 0, s.periodic || sg < P - 1, &t.fac[ty * m * 5],
+                          &t.spk[ty * m * 4])) {
+            t.P = 0;
+            return;
+        }
+    }
+    // unknowns of segment s: its rows [m - own(s - 1), +K), which segment
+    // s - 1 needs beyond its end, and [own(s) - K, own(s)), which s + 1 needs
+    auto own = [&](int sg) {
+        sg = (sg + P) % P;
+        return (sg < P - 1 ? st(sg + 1) : (s.periodic ? n : st(sg) + m)) - st(sg);
+    };
+    const int NR = K2 * P;
+    std::vector<double> R((size_t)NR * NR, 0.0);
+    for (int i = 0; i < NR; i++) R[(size_t)i * NR + i] = 1.0;
+    auto prev_of = [&](int sg) { return sg > 0 ? sg - 1 : (s.periodic ? P - 1 : -1); };
+    auto next_of = [&](int sg) { return sg < P - 1 ? sg + 1 : (s.periodic ? 0 : -1); };
+    for (int sg = 0; sg < P; sg++) {
+        const int ty = type_of(sg), pv = prev_of(sg), nx = next_of(sg);
+        for (int q = 0; q < K2; q++) {
+            if (q < K ? pv < 0 : nx < 0) continue;  // nobody reads these rows
+            const int j = q < K ? m - own(sg - 1) + q : own(sg) - K2 + q;
+            for (int r = 0; r < K; r++) {
+                if (pv >= 0) R[(size_t)(sg * K2 + q) * NR + pv * K2 + K + r] += t.spk[(ty * m + j) * 4 + r];
+                if (nx >= 0) R[(size_t)(sg * K2 + q) * NR + nx * K2 + r] += t.spk[(ty * m + j) * 4 + 2 + r];
+            }
+        }
+    }
+    invert(R, NR);
+    // coupling of segment s with s + dd: rows of the inverse at its neighbours
+    auto couple = [&](int sg, int r, int tt, int c) {
+        const int o = r < K ? prev_of(sg) : next_of(sg);
+        return o < 0 ? 0.0 : R[(size_t)(o * K2 + (r < K ? K + r : r - K)) * NR + tt * K2 + c];
+    };
+    std::vector<double> blk(P, 0.0);  // largest coupling by segment offset
+    for (int sg = 0; sg < P; sg++)
+        for (int dd = 0; dd < P; dd++)
+            for (int r = 0; r < K2; r++)
+                for (int c = 0; c < K2; c++)
+                    blk[dd] = std::max(blk[dd], std::fabs(couple(sg, r, (sg + dd) % P, c)));
+    const double top = *std::max_element(blk.begin(), blk.end());
+    int D = 0;
+    for (int dd = 1; dd <= P / 2; dd++)
+        if (blk[dd] > 1e-18 * top || blk[P - dd] > 1e-18 * top) D = dd;
+    t.nd = std::min(2 * D + 1, P);
+    t.d0 = 2 * D + 1 < P ? P - D : 0;
+    t.guni = s.periodic && n % P == 0;
+    t.G.assign((size_t)P * t.nd * K2 * K2, 0.0);
+    for (int sg = 0; sg < P; sg++)
+        for (int id = 0; id < t.nd; id++)
+            for (int r = 0; r < K2; r++)
+                for (int c = 0; c < K2; c++)
+                    t.G[(((size_t)sg * t.nd + id) * K2 + r) * K2 + c] = couple(sg, r, (sg + t.d0 + id) % P, c);
+}
+
 }  // namespace pdo

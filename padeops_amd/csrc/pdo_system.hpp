@@ -97,6 +97,29 @@ struct SpikeTables {
 
 int build_spike(const SystemDesc &s, SpikeTables &t, bool force_general = false);
 
+// ---- overlapping segments -------------------------------------------------
+// Systems of any length n as P segments of exactly m (32 or 16) rows that
+// overlap: segment s covers rows [start(s), start(s) + m) and owns (stores)
+// those up to the next start, q0 or q0 + 1 of them.  Two segments solve a
+// shared row from the same equations, so the partitioned solve holds as it
+// stands, with the neighbour values of a segment taken from inside the
+// neighbours instead of from their ends.
+struct OverlapTables {
+    int m = 0, P = 0;          // P == 0: the system does not fit this path
+    int K = 1, nbl = 0, nbr = 0;
+    int q0 = 0, nd = 0, d0 = 0, guni = 0;
+    std::vector<double> fac;   // [4][m][5] as SpikeTables
+    std::vector<double> spk;   // [4][m][4]
+    std::vector<double> G;     // [P][nd][2K][2K]: yL[0..K), yR[0..K) of segment s from the values of s + d0 + id
+    std::vector<double> sp;    // closure rows as SpikeTables
+    int start(int s, int n, bool periodic) const
+    {
+        return periodic ? (int)((long)s * n / P) : (P > 1 ? (int)((long)s * (n - m) / (P - 1)) : 0);
+    }
+};
+
+void build_overlap(const SystemDesc &s, OverlapTables &t);
+
 // Choose (m, P, xr) for a system of n rows; returns false when only the
 // general kernel applies.
 bool choose_partition(int n_sys, int K, int nb, bool periodic, int &m, int &P, int &xr);
