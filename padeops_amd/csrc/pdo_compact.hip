@@ -175,36 +175,6 @@ __device__ __forceinline__ void publish_ends(T *rb, const T (&d)[MM], int s, int
     }
 }
 
-// ---------------------------------------------------------------------------
-// raw buffer access: a uniform resource over a field plus a per-lane and a
-// scalar byte offset, so that rows of a strided pencil (scalar offsets
-// row * stride) cost no vector ALU work.  Byte offsets are 32-bit: the host
-// sends fields of 4 GiB or more to the general kernel.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t field_rsrc(const void *p)
-{
-    // stride 0, no range limit, 32-bit data format (raw dword access)
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, -1, 0x00020000);
-}
-template <typename T> __device__ __forceinline__ T buf_ld(__amdgpu_buffer_rsrc_t r, unsigned vo, unsigned so);
-template <> __device__ __forceinline__ float buf_ld<float>(__amdgpu_buffer_rsrc_t r, unsigned vo, unsigned so)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)vo, (int)so, 0));
-}
-template <> __device__ __forceinline__ double buf_ld<double>(__amdgpu_buffer_rsrc_t r, unsigned vo, unsigned so)
-{
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)vo, (int)so, 0));
-}
-__device__ __forceinline__ void buf_st(float v, __amdgpu_buffer_rsrc_t r, unsigned vo, unsigned so)
-{
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, (int)vo, (int)so, 0);
-}
-__device__ __forceinline__ void buf_st(double v, __amdgpu_buffer_rsrc_t r, unsigned vo, unsigned so)
-{
-    using U2 = unsigned __attribute__((ext_vector_type(2)));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), r, (int)vo, (int)so, 0);
-}
-
 // strided pencils: periodic windows and the stores through scalar row
 // offsets (1) or per-row lane address arithmetic (0); tuning constants
 #ifndef PDO_STRIDED_WINDOW_BUFFER

@@ -39,6 +39,7 @@ struct ApplyArgs {
     // q0 + 1), segments coupled to one (nd, from d0 relative to it), and
     // whether every segment has the same coupling rows
     int q0, nd, d0, guni;
+    int glds;          // words of coupling rows the workgroup stages in LDS (0: read from memory)
     unsigned smul, sdiv;  // start of segment s: s smul / D by the reciprocal sdiv = 2^31 / D + 1 (2^31: D = 1)
     double c[5];
     double band[5];    // interior LHS band (offsets -2..2), used by periodic systems

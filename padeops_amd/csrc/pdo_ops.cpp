@@ -173,7 +173,7 @@ static bool overlap_fits(const Variant &v, int dir, long na, long nb, size_t wor
         if (f.shift != 0 || s.n_in != s.n_sys || s.n_out != s.n_sys) return false;
         // at least 8 pencils fit a workgroup's LDS, with the exchange values and tables
         const size_t pen = (size_t)(s.n_sys | 1) * word + (size_t)o.P * 2 * o.K * 8;
-        return 8 * pen + (s.periodic ? 0 : 3 * (size_t)o.m * 9 * 8) <= 160 * 1024 &&
+        return 8 * pen + (s.periodic ? 0 : 3 * (size_t)o.m * 9 * 8) + 24 * 1024 <= 160 * 1024 &&
                (size_t)na * nb < ((size_t)1 << 31);
     }
     if (o.P > PMAX && (f.shift != 0 || o.m != MAXM)) return false;
@@ -182,6 +182,7 @@ static bool overlap_fits(const Variant &v, int dir, long na, long nb, size_t wor
     const size_t nmax = (size_t)std::max(std::max(s.n_in, s.n_out), s.n_sys + 1);
     const size_t lim = (size_t)1 << 32;
     if ((size_t)na * nb * nmax * word < lim) return true;
+    if (o.P > PMAX) return false;
     return dir == 3 ? (size_t)na * nb * word < lim : ((size_t)na * word < lim && nb <= 65535);
 }
 

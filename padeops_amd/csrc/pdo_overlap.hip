@@ -23,6 +23,8 @@
 // sequence of a few workgroups per CU.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "pdo_stencil.hpp"
 
 namespace pdo {
@@ -121,23 +123,23 @@ __device__ __forceinline__ void end_rows(const ApplyArgs &A, double (&d)[M], boo
 // of them loaded ahead; s may vary between the lanes of a wave unless UNI.  All threads of the block take
 // part.
 template <int K, int M, bool UNI, int SB, typename PT>
-__device__ __forceinline__ void ovl_solve(const ApplyArgs &A, double (&d)[M], PT tb, double *red, int pitch, int s, int pl,
-                                          const Seg &g)
+__device__ __forceinline__ void ovl_solve(const ApplyArgs &A, double (&d)[M], PT tb, double *red, const double *gl, int pitch, int s,
+                                          int pl, const Seg &g)
 {
     constexpr int K2 = 2 * K;
     const int P = A.P;
     sweep<K, M, SB>(d, tb);
     // rows in registers cannot be indexed: each row in range is written under
     // its own condition, which costs less than selecting the values would
-    double *rp = red + s * K2 * pitch + pl;
+    double *rlo = red + (s * K2 - g.lo) * pitch + pl, *rhi = red + (s * K2 + K - g.hi) * pitch + pl;
 #pragma unroll
     for (int j = 0; j < M; ++j) {
-        if ((unsigned)(j - g.lo) < (unsigned)K) rp[(j - g.lo) * pitch] = d[j];
-        if ((unsigned)(j - g.hi) < (unsigned)K) rp[(K + j - g.hi) * pitch] = d[j];
+        if ((unsigned)(j - g.lo) < (unsigned)K) rlo[j * pitch] = d[j];
+        if ((unsigned)(j - g.hi) < (unsigned)K) rhi[j * pitch] = d[j];
     }
     __syncthreads();
     double yl[2] = {0, 0}, yr[2] = {0, 0};
-    auto reduce = [&](const double *G) {
+    auto reduce = [&](auto G) {
         int t = s + A.d0;
         t -= t >= P ? P : 0;
         for (int id = 0; id < A.nd; ++id) {
@@ -157,9 +159,9 @@ __device__ __forceinline__ void ovl_solve(const ApplyArgs &A, double (&d)[M], PT
             t = t == P - 1 ? 0 : t + 1;
         }
     };
-    const double *G = A.tab_d + A.o_G;
-    if (UNI || A.guni) reduce(G + (UNI ? s * A.nd * K2 * K2 : 0));
-    else reduce(G + s * A.nd * K2 * K2);
+    const int go = A.guni ? 0 : s * A.nd * K2 * K2;
+    if (!UNI && A.glds) reduce(gl + go);
+    else reduce(A.tab_d + A.o_G + go);
     PT spk = tb + M * (2 * K + 1);
 #pragma unroll
     for (int j = 0; j < M; ++j) {
@@ -183,13 +185,45 @@ __device__ __forceinline__ void ovl_solve(const ApplyArgs &A, double (&d)[M], PT
 // contiguous index leaves no lane idle (A.nb == 1 in the launch then, and
 // A.lgn == 1 says that pencils are numbered through).
 // ---------------------------------------------------------------------------
-template <int K, int M> __device__ __forceinline__ void stage_tables(const ApplyArgs &A, double *tb)
-{
-    // types 0, 1, 2 (or 3 alone)
-    constexpr int TW = type_words<K, M>();
-    const double *src = A.tab_d + A.o_fac + (A.P == 1 ? 3 : 0) * TW;
-    for (int i = threadIdx.x; i < (A.P == 1 ? 1 : 3) * TW; i += blockDim.x) tb[i] = src[i];
-}
+// Tables a workgroup reads from LDS: the coupling rows (A.glds words) and, with
+// LT, types 0, 1, 2 (or 3 alone).  Loaded to registers here, ahead of the field
+// loads, so that one round trip to memory serves both; stage_write puts them
+// in place.  Reading them where they are needed costs a dependent miss each.
+constexpr int STAGE = 8;
+template <int K, int M, bool LT> struct Staged {
+    double v[STAGE];
+    const double *src, *tab;
+    int ng, nw;
+    __device__ __forceinline__ double at(int i) const { return i < ng ? src[i] : tab[i - ng]; }
+    __device__ __forceinline__ Staged(const ApplyArgs &A)
+    {
+        constexpr int TW = type_words<K, M>();
+        src = A.tab_d + A.o_G;
+        tab = A.tab_d + A.o_fac + (A.P == 1 ? 3 : 0) * TW;
+        ng = A.glds;
+        nw = ng + (LT ? (A.P == 1 ? 1 : 3) * TW : 0);
+#pragma unroll
+        for (int i = 0; i < STAGE; ++i) {
+            const int e = threadIdx.x + i * blockDim.x;
+            v[i] = e < nw ? at(e) : 0.0;
+        }
+    }
+    __device__ __forceinline__ void write(double *lds) const
+    {
+#pragma unroll
+        for (int i = 0; i < STAGE; ++i) {
+            const int e = threadIdx.x + i * blockDim.x;
+            if (e < nw) lds[e] = v[i];
+        }
+        for (int e = threadIdx.x + STAGE * blockDim.x; e < nw; e += blockDim.x) lds[e] = at(e);
+    }
+};
+
+// scalar rows (UNI) read their tables through the scalar cache
+struct NotStaged {
+    __device__ __forceinline__ NotStaged(const ApplyArgs &) {}
+    __device__ __forceinline__ void write(double *) const {}
+};
 
 template <int FAM, typename TS, int M, int NPW, bool LT>
 __global__ void __launch_bounds__(1024) k_ovl_strided(ApplyArgs A)
@@ -207,37 +241,63 @@ __global__ void __launch_bounds__(1024) k_ovl_strided(ApplyArgs A)
     const int ty = A.periodic ? 1 : (P == 1 ? 3 : (s == 0 ? 0 : (s == P - 1 ? 2 : 1)));
     const Seg g = segment<K>(A, s, M);
     const int r0 = g.r0, own = g.own;
+    std::conditional_t<UNI, NotStaged, Staged<K, M, LT>> stage(A);
     const unsigned vi = (a + b * (unsigned)A.sb_in) * (unsigned)sizeof(TS);
     const char *fb = (const char *)A.f + (size_t)blockIdx.y * A.sb_in * sizeof(TS);
     TS win[W];
+    const __amdgpu_buffer_rsrc_t rs = field_rsrc(A.f);
+    const unsigned ss = (unsigned)A.se_in * (unsigned)sizeof(TS);
+    // offset of row r0 - R (modulo 2^32), and how far the wrapped rows are off
+    const unsigned vl = vi + (unsigned)(r0 - R) * ss;
+    const unsigned turn = (unsigned)(A.periodic ? A.n_sys : A.n_in) * ss;
+    const int end = A.periodic ? A.n_read : A.n_in;
 #pragma unroll
     for (int w = 0; w < W; ++w) {
-        const int r = wrap_row(A, r0 - R + w, A.periodic);
-        win[w] = *(const TS *)(fb + (size_t)r * A.se_in * sizeof(TS) + vi);
+        if constexpr (UNI) {
+            const int r = wrap_row(A, r0 - R + w, A.periodic);
+            win[w] = *(const TS *)(fb + (size_t)r * A.se_in * sizeof(TS) + vi);
+        } else {
+            // the whole offset in the lane's 32 bits, where a row before the
+            // pencil's start wraps back into range
+            const int r = r0 - R + w;
+            const unsigned vo = vl + (unsigned)w * ss;
+            win[w] = buf_ld<TS>(rs, r < 0 ? vo + turn : (r >= end ? vo - turn : vo), 0u);
+        }
     }
     double d[M];
 #pragma unroll
     for (int j = 0; j < M; ++j) d[j] = stencil_row<FAM, double>(win, j, A.c);
     if (!A.periodic) {
-        auto ld = [&](int r) { return (double)*(const TS *)(fb + (size_t)r * A.se_in * sizeof(TS) + vi); };
+        auto ld = [&](int r) {
+            return UNI ? (double)*(const TS *)(fb + (size_t)r * A.se_in * sizeof(TS) + vi)
+                       : (double)buf_ld<TS>(rs, vi, (unsigned)r * ss);
+        };
         if (!UNI || s == 0) end_rows<M>(A, d, true, s == 0, ld);
         if (!UNI || s == P - 1) end_rows<M>(A, d, false, s == P - 1, ld);
     }
     extern __shared__ double lds[];
+    double *gl = lds + P * 2 * K * NPW, *tb = gl + A.glds;
+    stage.write(gl);
     if constexpr (LT) {
-        double *tb = lds + P * 2 * K * NPW;
-        stage_tables<K, M>(A, tb);
         __syncthreads();
-        ovl_solve<K, M, UNI, 2>(A, d, tb + (P == 1 ? 0 : ty) * type_words<K, M>(), lds, NPW, s, pl, g);
+        ovl_solve<K, M, UNI, 2>(A, d, tb + (P == 1 ? 0 : ty) * type_words<K, M>(), lds, gl, NPW, s, pl, g);
     } else {
-        ovl_solve<K, M, UNI, 8>(A, d, A.tab_d + A.o_fac + (UNI ? ty : 1) * type_words<K, M>(), lds, NPW, s, pl, g);
+        ovl_solve<K, M, UNI, 8>(A, d, A.tab_d + A.o_fac + (UNI ? ty : 1) * type_words<K, M>(), lds, gl, NPW, s, pl, g);
     }
     if (!act) return;
     const unsigned vo = (a + b * (unsigned)A.sb_out) * (unsigned)sizeof(TS);
     char *ob = (char *)A.out + (size_t)blockIdx.y * A.sb_out * sizeof(TS);
+    if constexpr (UNI) {
 #pragma unroll
-    for (int j = 0; j < M; ++j)
-        if (j < own) *(TS *)(ob + (size_t)(r0 + j) * A.se_out * sizeof(TS) + vo) = (TS)d[j];
+        for (int j = 0; j < M; ++j)
+            if (j < own) *(TS *)(ob + (size_t)(r0 + j) * A.se_out * sizeof(TS) + vo) = (TS)d[j];
+    } else {
+        const __amdgpu_buffer_rsrc_t ro = field_rsrc(A.out);
+        const unsigned so = (unsigned)A.se_out * (unsigned)sizeof(TS), vr = vo + (unsigned)r0 * so;
+#pragma unroll
+        for (int j = 0; j < M; ++j)
+            if (j < own) buf_st((TS)d[j], ro, vr, (unsigned)j * so);
+    }
     // periodic edge layouts repeat row 0 at row n_sys
     if (A.n_out > A.n_sys && s == 0) *(TS *)(ob + (size_t)A.n_sys * A.se_out * sizeof(TS) + vo) = (TS)d[0];
 }
@@ -255,20 +315,24 @@ __global__ void __launch_bounds__(512) k_ovl_x(ApplyArgs A, int TP, int LD, unsi
     constexpr int K = F::K, R = F::R, W = M + 2 * R;
     const int P = A.P, n = A.n_sys, nt = TP * P;
     extern __shared__ double lds[];
-    double *red = lds, *tb = red + P * 2 * K * TP;
+    double *red = lds, *gl = red + P * 2 * K * TP, *tb = gl + A.glds;
+    const Staged<K, M, LT> stage(A);
     TS *tile = (TS *)(tb + (LT ? (P == 1 ? 1 : 3) * type_words<K, M>() : 0));
     const int p = threadIdx.x % TP, s = threadIdx.x / TP;
     const long pen0 = (long)blockIdx.x * TP, left = A.na * A.nb - pen0;
     const int total = (int)(left < TP ? left : TP) * n;
     const TS *__restrict__ f = (const TS *)A.f + pen0 * n;
     // element e is row e % n of pencil e / n; e n < 2^32 makes the quotient by
-    // the rounded-up reciprocal exact
+    // the rounded-up reciprocal exact.  (Holding all n / P loads of a thread in
+    // flight takes 225 instead of 124 registers and halves the waves of large
+    // fields: 331 against 213-240 us for 384 x 320 x 640, 1 us gained on small ones.)
+    const int pad = LD - n;  // 0 or 1
 #pragma unroll 8
     for (int e = threadIdx.x; e < total; e += nt) {
         const int q = (int)__umulhi((unsigned)e, magic);
-        tile[q * LD + (e - q * n)] = f[e];
+        tile[e + (q & -pad)] = f[e];
     }
-    if constexpr (LT) stage_tables<K, M>(A, tb);
+    stage.write(gl);
     __syncthreads();
     const int ty = A.periodic ? 1 : (P == 1 ? 3 : (s == 0 ? 0 : (s == P - 1 ? 2 : 1)));
     const Seg g = segment<K>(A, s, M);
@@ -286,9 +350,9 @@ __global__ void __launch_bounds__(512) k_ovl_x(ApplyArgs A, int TP, int LD, unsi
         auto ld = [&](int r) { return (double)line[r]; };
         end_rows<M>(A, d, true, s == 0, ld);
         end_rows<M>(A, d, false, s == P - 1, ld);
-        ovl_solve<K, M, false, 2>(A, d, tb + (P == 1 ? 0 : ty) * type_words<K, M>(), red, TP, s, p, g);
+        ovl_solve<K, M, false, 2>(A, d, tb + (P == 1 ? 0 : ty) * type_words<K, M>(), red, gl, TP, s, p, g);
     } else {
-        ovl_solve<K, M, false, 8>(A, d, A.tab_d + A.o_fac + type_words<K, M>(), red, TP, s, p, g);
+        ovl_solve<K, M, false, 8>(A, d, A.tab_d + A.o_fac + type_words<K, M>(), red, gl, TP, s, p, g);
     }
     // the exchange's barrier came after every read of the tile
 #pragma unroll
@@ -299,13 +363,21 @@ __global__ void __launch_bounds__(512) k_ovl_x(ApplyArgs A, int TP, int LD, unsi
 #pragma unroll 8
     for (int e = threadIdx.x; e < total; e += nt) {
         const int q = (int)__umulhi((unsigned)e, magic);
-        out[e] = tile[q * LD + (e - q * n)];
+        out[e] = tile[e + (q & -pad)];
     }
+}
+
+// coupling rows staged in LDS up to 24 KiB
+template <int K> int staged_words(const ApplyArgs &A)
+{
+    const int words = (A.guni ? 1 : A.P) * A.nd * 4 * K * K;
+    return words <= 3072 ? words : 0;
 }
 
 template <int FAM, typename TS, int M> hipError_t strided_m(ApplyArgs A, hipStream_t st)
 {
     constexpr int K = Fam<FAM>::K;
+    A.glds = A.P > PMAX ? staged_words<K>(A) : 0;
     // pencils numbered through where 32-bit offsets reach the whole field
     const size_t nmax = (size_t)(A.n_in > A.n_out ? A.n_in : A.n_out);
     const size_t bytes = (size_t)A.na * A.nb * nmax * sizeof(TS);
@@ -319,8 +391,9 @@ template <int FAM, typename TS, int M> hipError_t strided_m(ApplyArgs A, hipStre
         return hipGetLastError();
     }
     if constexpr (M == MAXM && Fam<FAM>::SHIFT == 0) {
-        const dim3 grid((unsigned)((pen + 31) / 32), A.lgn ? 1u : (unsigned)A.nb);
-        const size_t red = (size_t)A.P * 2 * K * 32 * sizeof(double);
+        if (!A.lgn) return hipErrorInvalidValue;
+        const dim3 grid((unsigned)((pen + 31) / 32));
+        const size_t red = ((size_t)A.P * 2 * K * 32 + A.glds) * sizeof(double);
         if (A.periodic)
             hipLaunchKernelGGL((k_ovl_strided<FAM, TS, M, 32, false>), grid, dim3(32 * A.P), red, st, A);
         else
@@ -331,11 +404,12 @@ template <int FAM, typename TS, int M> hipError_t strided_m(ApplyArgs A, hipStre
     return hipErrorInvalidValue;
 }
 
-template <int FAM, typename TS, int M> hipError_t x_m(const ApplyArgs &A, hipStream_t st)
+template <int FAM, typename TS, int M> hipError_t x_m(ApplyArgs A, hipStream_t st)
 {
     constexpr int K = Fam<FAM>::K;
+    A.glds = staged_words<K>(A);
     const int n = A.n_sys, LD = n | 1;
-    const size_t tabs = A.periodic ? 0 : (size_t)(A.P == 1 ? 1 : 3) * type_words<K, M>() * sizeof(double);
+    const size_t tabs = ((A.periodic ? 0 : (A.P == 1 ? 1 : 3) * type_words<K, M>()) + (size_t)A.glds) * sizeof(double);
     auto lds = [&](int tp) { return (size_t)tp * (LD * sizeof(TS) + A.P * 2 * K * sizeof(double)) + tabs; };
     // two workgroups on a CU (80 KiB each), at most 512 threads
     int TP = 32;
