@@ -54,8 +54,10 @@ hipError_t run_filter2(const PoissonPlanDev &pl, int mode, const void *in, void 
 hipError_t run_ifft2(const PoissonPlanDev &pl, int mode, const void *in, void *work, void *out, int nplanes,
                      int oddball, hipStream_t st);
 // z transform, multiply by m, inverse z transform of an unpadded
-// (nx/2+1, ny, nz) spectrum (in may equal out).
-hipError_t run_zmul(const PoissonPlanDev &pl, int mode, const void *in, void *out, const SpecMul &m, hipStream_t st);
+// (nx/2+1, ny, nz) spectrum (in may equal out); lines > 0: of its first
+// `lines` kx only.
+hipError_t run_zmul(const PoissonPlanDev &pl, int mode, const void *in, void *out, const SpecMul &m, hipStream_t st,
+                    int lines = 0);
 // tables of the PadePoisson solve with walls (device, FP64): ax (nx/2+1),
 // ay (ny), az (2 nz) the squared wavenumbers, kcm and kcp (2 nz complex,
 // interleaved) k3' exp(-+ i k3 dz / 2)
@@ -67,6 +69,43 @@ struct PadeWallTables {
 // is; the plan's transforms have length 2 nz (its nz)
 hipError_t run_pp_walls(const PoissonPlanDev &pl, int mode, void *f, void *w, const PadeWallTables &t, bool upd,
                         hipStream_t st);
+
+// Transforms of several fields in few launches (pdo_fft_multi.hip).  All
+// fields share the plan's nx, ny; planes may differ.
+constexpr int MULTI_TASKS = 12;  // fields of one launch
+// src (nx/2+1, ny, planes) -> f = its inverse 2D transform, fx and fy (null:
+// not wanted) those of i kx src and i ky src.  A, and B with fy, are spectra
+// of work; A may be src.
+struct InvTask {
+    const void *src;
+    void *A, *B, *f, *fx, *fy;
+    int planes;
+};
+// spec = the forward 2D transform of (a1 - b1) c1 + (a2 - b2) c2; b1 null: of
+// a1, a2 null: of the first product
+struct FwdTask {
+    const void *a1, *b1, *c1, *a2, *b2, *c2;
+    void *spec;
+    int planes;
+};
+struct InvBatch {
+    InvTask t[MULTI_TASKS];
+    unsigned end[MULTI_TASKS];
+    int count;
+};
+struct FwdBatch {
+    FwdTask t[MULTI_TASKS];
+    unsigned end[MULTI_TASKS];
+    int count;
+};
+// modes of dealiased spectra that may differ from zero: kx < kxc, and of ky
+// index j those with j < kyc or j > ny - kyc
+struct BandLimit {
+    int kxc, kyc;
+};
+hipError_t run_inv_multi(const PoissonPlanDev &pl, int mode, const InvTask *t, int count, const BandLimit &bl,
+                         const double *kx, const double *ky, hipStream_t st);
+hipError_t run_fwd_multi(const PoissonPlanDev &pl, int mode, const FwdTask *t, int count, hipStream_t st);
 
 // Fourier-collocation derivative along dir of real f (n along dir; x:
 // (nx, na, nb), y: (na, ny, nb), z: (na, nb, nz)): the spectrum is multiplied

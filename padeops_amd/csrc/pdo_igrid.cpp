@@ -166,6 +166,65 @@ int pdo_igrid_interp_primitive(pdo_duidxj h, int prec, const pdo_interp_fields *
 
 }  // extern "C"
 
+namespace pdo {
+
+int igrid_fields(pdo_duidxj h, int prec, const pdo_interp_fields &I, const pdo_duidxj_fields &D, void *u, void *v,
+                 void *w, const BandLimit &bl, hipStream_t st)
+{
+    SpectralObject &C = *h->spC;
+    const int mode = fft_mode(prec), nxh = C.nxh, ny = C.ny, nz = C.nz, nx = C.nx;
+    const size_t W = mode == 0 ? 8 : 4;
+    const size_t rC = (size_t)nx * ny * nz * W, rE = (size_t)nx * ny * (nz + 1) * W;
+    const size_t cC = (size_t)nxh * ny * nz * 2 * W, cE = (size_t)nxh * ny * (nz + 1) * 2 * W;
+    // components 1 dudx 2 dudy 3 dudz 4 dvdx 5 dvdy 6 dvdz 7 dwdx 8 dwdy 9 dwdz
+    auto at = [](void *base, size_t bytes, int k) { return (void *)((char *)base + bytes * (k - 1)); };
+    auto RC = [&](int k) { return at(D.duidxjC, rC, k); };
+    auto RE = [&](int k) { return at(D.duidxjE, rE, k); };
+    auto HC = [&](int k) { return at(D.duidxjChat, cC, k); };
+    auto HE = [&](int k) { return at(D.duidxjEhat, cE, k); };
+    const int *bc = h->bc;
+    auto z = [&](int kind, int b, int t, const void *in, void *out) {
+        return pdo_pade6stagg_apply(h->dz, kind, b, t, prec, in, out, nxh, ny, 1, (void *)st);
+    };
+    int r;
+#define PDO_TRY(x)               \
+    do {                         \
+        if ((r = (x))) return r; \
+    } while (0)
+    // igrid.F90:1423-1463 and :2621-2679 in spectral space
+    PDO_TRY(z(14, bc[4], bc[5], I.what, I.whatC));
+    PDO_TRY(z(15, bc[0], bc[1], I.uhat, I.uEhat));
+    PDO_TRY(z(15, bc[2], bc[3], I.vhat, I.vEhat));
+    PDO_TRY(z(10, bc[4], bc[5], I.what, HC(9)));
+    PDO_TRY(z(15, bc[10], bc[11], HC(9), HE(9)));
+    if (!h->inviscid) PDO_TRY(z(13, bc[4], bc[5], I.what, D.d2wdz2hatE));
+    const void *uv[2] = {I.uhat, I.vhat};
+    void *d2[2] = {D.d2udz2hatC, D.d2vdz2hatC};
+    for (int q = 0; q < 2; q++) {
+        const int b = bc[2 * q], t = bc[2 * q + 1], db = bc[6 + 2 * q], dt = bc[7 + 2 * q], k = 3 + 3 * q;
+        PDO_TRY(z(11, b, t, uv[q], HE(k)));
+        if (!h->inviscid) {
+            // a one-sided boundary takes the second derivative as E2C(C2E(.))
+            if (t == 0 || b == 0) PDO_TRY(z(10, db, dt, HE(k), d2[q]));
+            else PDO_TRY(z(12, b, t, uv[q], d2[q]));
+        }
+        PDO_TRY(z(14, db, dt, HE(k), HC(k)));
+    }
+#undef PDO_TRY
+    const InvTask task[12] = {
+        {I.uhat, HC(1), HC(2), u, RC(1), RC(2), nz},      {I.vhat, HC(4), HC(5), v, RC(4), RC(5), nz},
+        {I.whatC, HC(7), HC(8), I.wC, RC(7), RC(8), nz},  {I.uEhat, HE(1), HE(2), I.uE, RE(1), RE(2), nz + 1},
+        {I.vEhat, HE(4), HE(5), I.vE, RE(4), RE(5), nz + 1}, {I.what, HE(7), HE(8), w, RE(7), RE(8), nz + 1},
+        {HC(3), HC(3), nullptr, RC(3), nullptr, nullptr, nz}, {HC(6), HC(6), nullptr, RC(6), nullptr, nullptr, nz},
+        {HC(9), HC(9), nullptr, RC(9), nullptr, nullptr, nz}, {HE(3), HE(3), nullptr, RE(3), nullptr, nullptr, nz + 1},
+        {HE(6), HE(6), nullptr, RE(6), nullptr, nullptr, nz + 1},
+        {HE(9), HE(9), nullptr, RE(9), nullptr, nullptr, nz + 1}};
+    const hipError_t e = run_inv_multi(C.plan, mode, task, 12, bl, C.d_k1, C.d_k2, st);
+    return e == hipSuccess ? 0 : hip_fail(e, "prepared fields");
+}
+
+}  // namespace pdo
+
 // ---------------------------------------------------------------------------
 // sgs_igrid%getRHS_SGS (sgsmod_igrid.F90:204-266) with getTauSGS (:156-201)
 // for the eddy-viscosity models
@@ -180,8 +239,10 @@ struct SgsRhsObject {
     size_t nC = 0, nE = 0, sC = 0, sE = 0;     // points (cells, edges), spectral values (cells, edges)
     int wprec = -1;                            // precision the work buffers are sized for
     std::vector<void *> bufs;
-    void *SC = nullptr, *SE = nullptr, *nuC = nullptr, *nuE = nullptr, *tauC = nullptr, *tauE = nullptr;
-    void *cb1 = nullptr, *cb2 = nullptr;
+    void *nuC = nullptr, *nuE = nullptr, *tauC = nullptr, *tauE = nullptr;
+    // spectra of tau11, 12, 22, 33 (cells), 13, 23 (edges) and the z
+    // derivatives of 13, 23 (cells), 33 (edges)
+    void *hC[4] = {}, *hE[2] = {}, *zC[2] = {}, *zE = nullptr;
     // learned closure (pdo_sgsrhs_set_closure): its stress replaces the
     // eddy-viscosity stress, which stays where the closure's dissipation is
     // negative when `fallback` is set
@@ -209,9 +270,10 @@ struct SgsRhsObject {
         if (wprec == prec) return 0;
         free_bufs();
         const size_t W = prec == PDO_F64 ? 8 : 4;
-        const size_t sizes[8] = {6 * nC * W, 6 * nE * W, nC * W, nE * W, 4 * nC * W, 2 * nE * W, 2 * sC * W, 2 * sE * W};
-        void **dst[8] = {&SC, &SE, &nuC, &nuE, &tauC, &tauE, &cb1, &cb2};
-        for (int i = 0; i < 8; i++) {
+        const size_t c = 2 * sC * W, e2 = 2 * sE * W;
+        const size_t sizes[13] = {nC * W, nE * W, 4 * nC * W, 2 * nE * W, c, c, c, c, e2, e2, c, c, e2};
+        void **dst[13] = {&nuC, &nuE, &tauC, &tauE, &hC[0], &hC[1], &hC[2], &hC[3], &hE[0], &hE[1], &zC[0], &zC[1], &zE};
+        for (int i = 0; i < 13; i++) {
             hipError_t e = hipMalloc(dst[i], sizes[i]);
             if (e != hipSuccess) return hip_fail(e, "hipMalloc(sgs work)");
             bufs.push_back(*dst[i]);
@@ -294,7 +356,7 @@ static int sgsrhs_compute(pdo_sgsrhs h, int prec, const void *duidxjC, const voi
         return PDO_ERR_ARG;
     }
     hipStream_t st = (hipStream_t)stream;
-    SpectralObject &C = *h->spC, &E = *h->spE;
+    SpectralObject &C = *h->spC;
     const int nx = C.nx, ny = C.ny, nz = C.nz, nxh = C.nxh;
     const long nxy = (long)nx * ny;
     const pdo_sgs_params &p = h->p;
@@ -308,29 +370,25 @@ static int sgsrhs_compute(pdo_sgsrhs h, int prec, const void *duidxjC, const voi
         hipError_t ee = (x);                                    \
         if (ee != hipSuccess) return hip_fail(ee, what);        \
     } while (0)
-    // Step 0/1: S_ij and the model kernel on cells; on edges S_ij and, with
-    // explicitCalcEdgeEddyViscosity, the kernel too
-    const bool edge_kernel = p.explicit_edge && !lambda;
-    PDO_TRY(pdo_sgs_kernel(prec, p.model, duidxjC, h->SC, h->nuC, (long)h->nC, p.camd_x, p.camd_y, p.camd_z, stream));
-    PDO_TRY(pdo_sgs_kernel(prec, p.model, duidxjE, h->SE, edge_kernel ? h->nuE : nullptr, (long)h->nE, p.camd_x,
-                           p.camd_y, p.camd_z, stream));
-    // Step 3: multiply_by_model_constant (eddyViscosity.F90:74-103)
-    if (lambda) {
-        // the dynamic procedure's planar coefficient, then C2E interpolation
-        PDO_TRY(pdo_sgs_scale(prec, h->nuC, nxy, nz, lambda, 0.0, stream));
-        PDO_TRY(pdo_pade6stagg_apply(h->dz, 15, 0, 0, prec, h->nuC, h->nuE, nx, ny, 0, stream));
+    // Steps 0-3 of getTauSGS: the model kernel times its constant
+    // (multiply_by_model_constant, eddyViscosity.F90:74-103; the dynamic
+    // procedure's planar coefficient) and tau_ij = -2 nu S_ij, on cells; on
+    // edges the viscosity interpolated, or with explicitCalcEdgeEddyViscosity
+    // from the edge gradients
+    const double camd[3] = {p.camd_x, p.camd_y, p.camd_z};
+    PDO_HIP(launch_sgs_tau(mode, false, duidxjC, h->nuC, h->tauC, (long)h->nC, nxy, p.model, camd,
+                           lambda ? lambda : h->d_cC, p.cglobal, st),
+            "subgrid stress");
+    if (p.explicit_edge && !lambda) {
+        PDO_HIP(launch_sgs_tau(mode, true, duidxjE, h->nuE, h->tauE, (long)h->nE, nxy, p.model, camd, h->d_cE,
+                               p.cglobal, st),
+                "subgrid stress");
     } else {
-        PDO_TRY(pdo_sgs_scale(prec, h->nuC, nxy, nz, h->d_cC, p.cglobal, stream));
-        if (p.explicit_edge) {
-            PDO_TRY(pdo_sgs_scale(prec, h->nuE, nxy, nz + 1, h->d_cE, p.cglobal, stream));
-        } else {
-            // interpolate_eddy_viscosity(checknegative = .true.)
-            PDO_TRY(pdo_pade6stagg_apply(h->dz, 15, 0, 0, prec, h->nuC, h->nuE, nx, ny, 0, stream));
-            PDO_HIP(launch_clip_negative(mode, h->nuE, (long)h->nE, st), "clip");
-        }
+        // interpolate_eddy_viscosity (checknegative = .true. without the
+        // dynamic procedure)
+        PDO_TRY(pdo_pade6stagg_apply(h->dz, 15, 0, 0, prec, h->nuC, h->nuE, nx, ny, 0, stream));
+        PDO_HIP(launch_edge_tau(mode, !lambda, duidxjE, h->nuE, h->tauE, (long)h->nE, st), "subgrid stress");
     }
-    // tau_ij = -2 nu S_ij
-    PDO_HIP(launch_tau(mode, h->nuC, h->SC, h->nuE, h->SE, h->tauC, h->tauE, (long)h->nC, (long)h->nE, st), "tau");
     if (h->closure) {
         // the learned stress on cells (scale from the cell gradients) and on
         // edges (the same scale)
@@ -348,27 +406,20 @@ static int sgsrhs_compute(pdo_sgsrhs h, int prec, const void *duidxjC, const voi
     const size_t W = prec == PDO_F64 ? 8 : 4;
     auto tc = [&](int q) { return (const void *)((const char *)h->tauC + (size_t)q * h->nC * W); };
     auto te = [&](int q) { return (const void *)((const char *)h->tauE + (size_t)q * h->nE * W); };
-    const long nsC = (long)h->sC, nsE = (long)h->sE;
-    // ddx(tau11) -> urhs; ddy(tau22) -> vrhs
-    PDO_TRY(pdo_spectral_fft(h->spC, prec, tc(0), h->cb1, stream));
-    PDO_HIP(launch_sub(mode, urhs, h->cb1, C.d_k1, nxh, ny, nsC, 1, st), "rhs");
-    PDO_TRY(pdo_spectral_fft(h->spC, prec, tc(2), h->cb1, stream));
-    PDO_HIP(launch_sub(mode, vrhs, h->cb1, C.d_k2, nxh, ny, nsC, 2, st), "rhs");
-    // ddz(tau33) -> wrhs (ddz_C2E with (0, 0) ends)
-    PDO_TRY(pdo_spectral_fft(h->spC, prec, tc(3), h->cb1, stream));
-    PDO_TRY(pdo_pade6stagg_apply(h->dz, 11, 0, 0, prec, h->cb1, h->cb2, nxh, ny, 1, stream));
-    PDO_HIP(launch_sub(mode, wrhs, h->cb2, nullptr, nxh, ny, nsE, 0, st), "rhs");
-    // ddx(tau12) -> vrhs, ddy(tau12) -> urhs
-    PDO_TRY(pdo_spectral_fft(h->spC, prec, tc(1), h->cb1, stream));
-    PDO_HIP(launch_sub(mode, vrhs, h->cb1, C.d_k1, nxh, ny, nsC, 1, st), "rhs");
-    PDO_HIP(launch_sub(mode, urhs, h->cb1, C.d_k2, nxh, ny, nsC, 2, st), "rhs");
-    // ddz(tau13) -> urhs, ddx(tau13) -> wrhs; ddz(tau23) -> vrhs, ddy(tau23) -> wrhs
-    for (int q = 0; q < 2; q++) {
-        PDO_TRY(pdo_spectral_fft(h->spE, prec, te(q), h->cb2, stream));
-        PDO_TRY(pdo_pade6stagg_apply(h->dz, 10, 0, 0, prec, h->cb2, h->cb1, nxh, ny, 1, stream));
-        PDO_HIP(launch_sub(mode, q == 0 ? urhs : vrhs, h->cb1, nullptr, nxh, ny, nsC, 0, st), "rhs");
-        PDO_HIP(launch_sub(mode, wrhs, h->cb2, q == 0 ? E.d_k1 : E.d_k2, nxh, ny, nsE, q + 1, st), "rhs");
+    // the six stresses transformed, the z derivatives of 13, 23 (E2C) and 33
+    // (C2E, (0, 0) ends), then all terms of the divergence at once
+    FwdTask task[6] = {};
+    for (int q = 0; q < 6; q++) {
+        task[q].a1 = q < 4 ? tc(q) : te(q - 4);
+        task[q].spec = q < 4 ? h->hC[q] : h->hE[q - 4];
+        task[q].planes = q < 4 ? nz : nz + 1;
     }
+    PDO_HIP(run_fwd_multi(C.plan, mode, task, 6, st), "stress transforms");
+    for (int q = 0; q < 2; q++)
+        PDO_TRY(pdo_pade6stagg_apply(h->dz, 10, 0, 0, prec, h->hE[q], h->zC[q], nxh, ny, 1, stream));
+    PDO_TRY(pdo_pade6stagg_apply(h->dz, 11, 0, 0, prec, h->hC[3], h->zE, nxh, ny, 1, stream));
+    const StressSpectra S{h->hC[0], h->hC[1], h->hC[2], h->zC[0], h->zC[1], h->zE, h->hE[0], h->hE[1]};
+    PDO_HIP(launch_stress_div(mode, urhs, vrhs, wrhs, S, C.d_k1, C.d_k2, nxh, ny, (long)h->sC, (long)h->sE, st), "rhs");
 #undef PDO_TRY
 #undef PDO_HIP
     return 0;

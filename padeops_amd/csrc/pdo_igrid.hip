@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include "pdo_igrid.hpp"
+#include "pdo_sgs_dev.hpp"
 
 namespace pdo {
 
@@ -32,119 +33,156 @@ __global__ void __launch_bounds__(256) k_surface_plane(TS *f, long nplane, doubl
     PDO_GRID_STRIDE(t, nplane) z[t] = V{(TS)(t == 0 ? v : 0.0), (TS)0};
 }
 
-// tau_ij = -2 nu S_ij: cells 11, 12, 22, 33 from (nuC, SC), edges 13, 23
-// from (nuE, SE); S holds (11, 12, 13, 22, 23, 33) as in get_Sij_from_duidxj
-template <typename TS, typename TC>
-__global__ void __launch_bounds__(256) k_tau(const TS *nuC, const TS *SC, const TS *nuE, const TS *SE, TS *tauC,
-                                           TS *tauE, long nC, long nE)
+// 32-bit index arithmetic of (i, j) of a complex value: fields of a plane
+// count below 2^31 values
+__device__ __forceinline__ void line_of(unsigned t, unsigned nxh, unsigned ny, unsigned &i, unsigned &j)
 {
-    PDO_GRID_STRIDE(t, nC)
-    {
-        const TC m = (TC)-2 * (TC)nuC[t];
-        tauC[t] = (TS)(m * (TC)SC[t]);
-        tauC[t + nC] = (TS)(m * (TC)SC[t + nC]);
-        tauC[t + 2 * nC] = (TS)(m * (TC)SC[t + 3 * nC]);
-        tauC[t + 3 * nC] = (TS)(m * (TC)SC[t + 5 * nC]);
-    }
-    PDO_GRID_STRIDE(t, nE)
-    {
-        const TC m = (TC)-2 * (TC)nuE[t];
-        tauE[t] = (TS)(m * (TC)SE[t + 2 * nE]);
-        tauE[t + nE] = (TS)(m * (TC)SE[t + 4 * nE]);
-    }
+    const unsigned q = t / nxh;
+    i = t - q * nxh;
+    j = q % ny;
 }
 
-template <typename TS>
-__global__ void __launch_bounds__(256) k_clip_negative(TS *a, long n)
-{
-    PDO_GRID_STRIDE(t, n) if (a[t] < (TS)0) a[t] = (TS)0;
-}
-
-// rhs -= i k f (k = kv[index along dim]) or, kv == NULL, rhs -= f; complex
-// arrays of (nxh, ny, planes)
-template <typename TS, typename TC>
-__global__ void __launch_bounds__(256) k_sub(TS *rhs, const TS *f, const double *__restrict__ kv, int nxh, int ny,
-                                           long n, int dim)
-{
-    using V = typename C2<TS>::V;
-    V *r = (V *)rhs;
-    const V *s = (const V *)f;
-    PDO_GRID_STRIDE(t, n)
-    {
-        const V a = s[t];
-        V o = r[t];
-        if (kv) {
-            const long ij = dim == 1 ? t % nxh : (t / nxh) % ny;
-            const TC k = (TC)kv[ij];
-            // i k (a.x + i a.y) = -k a.y + i k a.x
-            o.x = (TS)((TC)o.x - (-k * (TC)a.y));
-            o.y = (TS)((TC)o.y - k * (TC)a.x);
-        } else {
-            o.x = (TS)((TC)o.x - (TC)a.x);
-            o.y = (TS)((TC)o.y - (TC)a.y);
-        }
-        r[t] = o;
-    }
-}
-
-// out = (a1 - b1) c1 [+ (a2 - b2) c2]: the rotational-form products of
-// AddNonLinearTerm_Rot (igrid.F90:1497-1566)
-template <typename TS, typename TC>
-__global__ void __launch_bounds__(256) k_cross(const TS *a1, const TS *b1, const TS *c1, const TS *a2, const TS *b2,
-                                             const TS *c2, TS *out, long n)
+// subgrid viscosity and stress in one pass over the gradients: the strain
+// stays in registers (it was a field of six components, written, and read
+// again by the stress kernel: 36 words per cell and 24 per edge, now 14 and
+// 8).  nu is the model kernel times its constant.
+template <typename TS, typename TC, bool EDGES>
+__global__ void __launch_bounds__(256) k_sgs_tau(const TS *__restrict__ g, TS *__restrict__ nu, TS *__restrict__ tau,
+                                                long n, long nxy, int model, TC cx, TC cy, TC cz,
+                                                const double *__restrict__ cplane, double cglobal)
 {
     PDO_GRID_STRIDE(t, n)
     {
-        TC v = ((TC)a1[t] - (TC)b1[t]) * (TC)c1[t];
-        if (a2) v += ((TC)a2[t] - (TC)b2[t]) * (TC)c2[t];
-        out[t] = (TS)v;
-    }
-}
-
-// r += s (real words)
-template <typename TS, typename TC>
-__global__ void __launch_bounds__(256) k_add(TS *r, const TS *s, long n)
-{
-    PDO_GRID_STRIDE(t, n) r[t] = (TS)((TC)r[t] + (TC)s[t]);
-}
-
-// addViscousTerm (igrid.F90:1914-1959): rhs += (1/Re) (-(k1^2 + k2^2) f + d2f)
-template <typename TS, typename TC>
-__global__ void __launch_bounds__(256) k_visc(TS *rhs, const TS *f, const TS *d2, const double *__restrict__ k1,
-                                            const double *__restrict__ k2, int nxh, int ny, long n, double invRe)
-{
-    using V = typename C2<TS>::V;
-    V *r = (V *)rhs;
-    const V *a = (const V *)f;
-    const V *b = (const V *)d2;
-    PDO_GRID_STRIDE(t, n)
-    {
-        const long i = t % nxh, j = (t / nxh) % ny;
-        const TC ks = (TC)(k1[i] * k1[i] + k2[j] * k2[j]);
-        const V x = a[t], y = b[t];
-        V o = r[t];
-        o.x = (TS)((TC)o.x + (TC)invRe * (-ks * (TC)x.x + (TC)y.x));
-        o.y = (TS)((TC)o.y + (TC)invRe * (-ks * (TC)x.y + (TC)y.y));
-        r[t] = o;
-    }
-}
-
-// out = sum_q c[q] x[q], terms added left to right (real words); NULL
-// operands end the list
-struct LinComb {
-    const void *x[5];
-    double c[5];
-};
-template <typename TS, typename TC>
-__global__ void __launch_bounds__(256) k_lincomb(TS *out, LinComb L, long n)
-{
-    PDO_GRID_STRIDE(t, n)
-    {
-        TC v = (TC)L.c[0] * (TC)((const TS *)L.x[0])[t];
+        TC d[9], s[6];
 #pragma unroll
-        for (int q = 1; q < 5; ++q)
-            if (L.x[q]) v += (TC)L.c[q] * (TC)((const TS *)L.x[q])[t];
-        out[t] = (TS)v;
+        for (int c = 0; c < 9; ++c) d[c] = (TC)g[t + c * n];
+        strain<TC>(d, s);
+        const TS v = (TS)((double)(TS)sgs_viscosity<TC>(d, s, model, cx, cy, cz) * (cplane ? cplane[t / nxy] : cglobal));
+        nu[t] = v;
+        const TC m = (TC)-2 * (TC)v;
+        if constexpr (EDGES) {
+            tau[t] = (TS)(m * s[2]);
+            tau[t + n] = (TS)(m * s[4]);
+        } else {
+            tau[t] = (TS)(m * s[0]);
+            tau[t + n] = (TS)(m * s[1]);
+            tau[t + 2 * n] = (TS)(m * s[3]);
+            tau[t + 3 * n] = (TS)(m * s[5]);
+        }
+    }
+}
+
+// edge stresses 13, 23 from an interpolated viscosity
+template <typename TS, typename TC>
+__global__ void __launch_bounds__(256) k_edge_tau(const TS *__restrict__ g, TS *nu, TS *__restrict__ tau, long n,
+                                                 bool clip)
+{
+    PDO_GRID_STRIDE(t, n)
+    {
+        TS v = nu[t];
+        if (clip && v < (TS)0) {
+            v = (TS)0;
+            nu[t] = v;
+        }
+        const TC m = (TC)-2 * (TC)v;
+        const TC s13 = (TC)0.5 * ((TC)g[t + 2 * n] + (TC)g[t + 6 * n]);
+        const TC s23 = (TC)0.5 * ((TC)g[t + 5 * n] + (TC)g[t + 7 * n]);
+        tau[t] = (TS)(m * s13);
+        tau[t + n] = (TS)(m * s23);
+    }
+}
+
+// the stress divergence of the three components in one pass (it was a
+// read-modify-write of the right-hand side per term: 27 words, now 15)
+template <typename TS, typename TC>
+__global__ void __launch_bounds__(256) k_stress_div(TS *u, TS *v, TS *w, StressSpectra S,
+                                                   const double *__restrict__ k1, const double *__restrict__ k2,
+                                                   unsigned nxh, unsigned ny, long ncell, long nedge)
+{
+    using V = typename C2<TS>::V;
+    auto at = [](const void *p, long t) { return ((const V *)p)[t]; };
+    // r -= i (a p + b q) + z
+    auto term = [](V *r, long t, TC a, V p, TC b, V q, V z) {
+        const V o = r[t];
+        r[t] = V{(TS)((TC)o.x + a * (TC)p.y + b * (TC)q.y - (TC)z.x), (TS)((TC)o.y - a * (TC)p.x - b * (TC)q.x - (TC)z.y)};
+    };
+    PDO_GRID_STRIDE(t, nedge)
+    {
+        unsigned i, j;
+        line_of((unsigned)t, nxh, ny, i, j);
+        const TC a = (TC)k1[i], b = (TC)k2[j];
+        if (t < ncell) {
+            const V t12 = at(S.t12, t);
+            term((V *)u, t, a, at(S.t11, t), b, t12, at(S.z13, t));
+            term((V *)v, t, a, t12, b, at(S.t22, t), at(S.z23, t));
+        }
+        term((V *)w, t, a, at(S.t13, t), b, at(S.t23, t), at(S.z33, t));
+    }
+}
+
+// the nonlinear term's cell part and addViscousTerm (igrid.F90:1914-1959)
+template <typename TS, typename TC>
+__global__ void __launch_bounds__(256) k_rhs_terms(RhsTerms T, const double *__restrict__ k1,
+                                                  const double *__restrict__ k2, unsigned nxh, unsigned ny, long ncell,
+                                                  long nedge, TC invRe)
+{
+    using V = typename C2<TS>::V;
+    PDO_GRID_STRIDE(t, nedge)
+    {
+        unsigned i, j;
+        line_of((unsigned)t, nxh, ny, i, j);
+        const TC ks = (TC)(k1[i] * k1[i] + k2[j] * k2[j]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            if (c < 2 && t >= ncell) continue;
+            if (!T.s[c] && invRe == (TC)0) continue;
+            V *r = (V *)T.rhs[c];
+            V o = r[t];
+            if (T.s[c]) {
+                const V x = ((const V *)T.s[c])[t];
+                o.x = (TS)((TC)o.x + (TC)x.x);
+                o.y = (TS)((TC)o.y + (TC)x.y);
+            }
+            if (invRe != (TC)0) {
+                const V x = ((const V *)T.f[c])[t], y = ((const V *)T.d2[c])[t];
+                o.x = (TS)((TC)o.x + invRe * (-ks * (TC)x.x + (TC)y.x));
+                o.y = (TS)((TC)o.y + invRe * (-ks * (TC)x.y + (TC)y.y));
+            }
+            r[t] = o;
+        }
+    }
+}
+
+// a Runge-Kutta stage of the three components with the x-y dealiasing mask
+template <typename TS, typename TC>
+__global__ void __launch_bounds__(256) k_stage(StageTerms T, const double *__restrict__ g1,
+                                              const double *__restrict__ g2, unsigned nxh, unsigned ny, long ncell,
+                                              long nedge)
+{
+    using V = typename C2<TS>::V;
+    PDO_GRID_STRIDE(t, nedge)
+    {
+        unsigned i, j;
+        line_of((unsigned)t, nxh, ny, i, j);
+        const bool keep = g1[i] * g2[j] != 0.0;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            if (c < 2 && t >= ncell) continue;
+            V o{(TS)0, (TS)0};
+            if (keep) {
+                const V x0 = ((const V *)T.x[0][c])[t];
+                TC re = (TC)T.coef[0] * (TC)x0.x, im = (TC)T.coef[0] * (TC)x0.y;
+#pragma unroll
+                for (int q = 1; q < 5; ++q)
+                    if (q < T.nterms) {
+                        const V x = ((const V *)T.x[q][c])[t];
+                        re += (TC)T.coef[q] * (TC)x.x;
+                        im += (TC)T.coef[q] * (TC)x.y;
+                    }
+                o = V{(TS)re, (TS)im};
+            }
+            ((V *)T.out[c])[t] = o;
+        }
     }
 }
 
@@ -300,26 +338,6 @@ hipError_t launch_surface_plane(int mode, void *f, long nplane, double v, hipStr
     return surface_t<float, float>(f, nplane, v, st);
 }
 
-hipError_t launch_tau(int mode, const void *nuC, const void *SC, const void *nuE, const void *SE, void *tauC,
-                      void *tauE, long nC, long nE, hipStream_t st)
-{
-    const dim3 g(blocks_for(nC > nE ? nC : nE)), b(256);
-    switch (mode) {
-    case 0:
-        hipLaunchKernelGGL((k_tau<double, double>), g, b, 0, st, (const double *)nuC, (const double *)SC,
-                           (const double *)nuE, (const double *)SE, (double *)tauC, (double *)tauE, nC, nE);
-        break;
-    case 1:
-        hipLaunchKernelGGL((k_tau<float, float>), g, b, 0, st, (const float *)nuC, (const float *)SC,
-                           (const float *)nuE, (const float *)SE, (float *)tauC, (float *)tauE, nC, nE);
-        break;
-    default:
-        hipLaunchKernelGGL((k_tau<float, double>), g, b, 0, st, (const float *)nuC, (const float *)SC,
-                           (const float *)nuE, (const float *)SE, (float *)tauC, (float *)tauE, nC, nE);
-    }
-    return hipGetLastError();
-}
-
 // ---------------------------------------------------------------------------
 // Moeng wall model: first-plane sums, the surface quantities, the embedded
 // wall stresses
@@ -432,99 +450,68 @@ hipError_t launch_mean_add(int mode, void *f, long nplane, int nz, double v, hip
     return hipGetLastError();
 }
 
-hipError_t launch_clip_negative(int mode, void *a, long n, hipStream_t st)
-{
-    if (mode == 0)
-        hipLaunchKernelGGL((k_clip_negative<double>), dim3(blocks_for(n)), dim3(256), 0, st, (double *)a, n);
-    else
-        hipLaunchKernelGGL((k_clip_negative<float>), dim3(blocks_for(n)), dim3(256), 0, st, (float *)a, n);
+// calls F<TS, TC> of the mode
+#define PDO_MODES(CALL)                        \
+    switch (mode) {                            \
+    case 0: { CALL(double, double); break; }   \
+    case 1: { CALL(float, float); break; }     \
+    default: { CALL(float, double); }          \
+    }                                          \
     return hipGetLastError();
+
+hipError_t launch_sgs_tau(int mode, bool edges, const void *g, void *nu, void *tau, long n, long nxy, int model,
+                          const double (&camd)[3], const double *cplane, double cglobal, hipStream_t st)
+{
+    const dim3 gr(blocks_for(n)), b(256);
+#define PDO_CALL(TS, TC)                                                                                          \
+    if (edges)                                                                                                    \
+        hipLaunchKernelGGL((k_sgs_tau<TS, TC, true>), gr, b, 0, st, (const TS *)g, (TS *)nu, (TS *)tau, n, nxy,   \
+                           model, (TC)camd[0], (TC)camd[1], (TC)camd[2], cplane, cglobal);                        \
+    else                                                                                                          \
+        hipLaunchKernelGGL((k_sgs_tau<TS, TC, false>), gr, b, 0, st, (const TS *)g, (TS *)nu, (TS *)tau, n, nxy,  \
+                           model, (TC)camd[0], (TC)camd[1], (TC)camd[2], cplane, cglobal);
+    PDO_MODES(PDO_CALL)
+#undef PDO_CALL
 }
 
-hipError_t launch_sub(int mode, void *rhs, const void *f, const double *kv, int nxh, int ny, long n, int dim,
-                      hipStream_t st)
+hipError_t launch_edge_tau(int mode, bool clip, const void *g, void *nu, void *tau, long n, hipStream_t st)
 {
-    const dim3 g(blocks_for(n)), b(256);
-    switch (mode) {
-    case 0:
-        hipLaunchKernelGGL((k_sub<double, double>), g, b, 0, st, (double *)rhs, (const double *)f, kv, nxh, ny, n,
-                           dim);
-        break;
-    case 1:
-        hipLaunchKernelGGL((k_sub<float, float>), g, b, 0, st, (float *)rhs, (const float *)f, kv, nxh, ny, n, dim);
-        break;
-    default:
-        hipLaunchKernelGGL((k_sub<float, double>), g, b, 0, st, (float *)rhs, (const float *)f, kv, nxh, ny, n, dim);
-    }
-    return hipGetLastError();
+#define PDO_CALL(TS, TC)                                                                                           \
+    hipLaunchKernelGGL((k_edge_tau<TS, TC>), dim3(blocks_for(n)), dim3(256), 0, st, (const TS *)g, (TS *)nu,       \
+                       (TS *)tau, n, clip)
+    PDO_MODES(PDO_CALL)
+#undef PDO_CALL
 }
 
-hipError_t launch_cross(int mode, const void *a1, const void *b1, const void *c1, const void *a2, const void *b2,
-                        const void *c2, void *out, long n, hipStream_t st)
+hipError_t launch_stress_div(int mode, void *u, void *v, void *w, const StressSpectra &S, const double *k1,
+                             const double *k2, int nxh, int ny, long ncell, long nedge, hipStream_t st)
 {
-    const dim3 g(blocks_for(n)), b(256);
-    switch (mode) {
-    case 0:
-        hipLaunchKernelGGL((k_cross<double, double>), g, b, 0, st, (const double *)a1, (const double *)b1,
-                           (const double *)c1, (const double *)a2, (const double *)b2, (const double *)c2,
-                           (double *)out, n);
-        break;
-    case 1:
-        hipLaunchKernelGGL((k_cross<float, float>), g, b, 0, st, (const float *)a1, (const float *)b1,
-                           (const float *)c1, (const float *)a2, (const float *)b2, (const float *)c2, (float *)out,
-                           n);
-        break;
-    default:
-        hipLaunchKernelGGL((k_cross<float, double>), g, b, 0, st, (const float *)a1, (const float *)b1,
-                           (const float *)c1, (const float *)a2, (const float *)b2, (const float *)c2, (float *)out,
-                           n);
-    }
-    return hipGetLastError();
+#define PDO_CALL(TS, TC)                                                                                         \
+    hipLaunchKernelGGL((k_stress_div<TS, TC>), dim3(blocks_for(nedge)), dim3(256), 0, st, (TS *)u, (TS *)v,      \
+                       (TS *)w, S, k1, k2, (unsigned)nxh, (unsigned)ny, ncell, nedge)
+    PDO_MODES(PDO_CALL)
+#undef PDO_CALL
 }
 
-hipError_t launch_add(int mode, void *r, const void *s, long n, hipStream_t st)
+hipError_t launch_rhs_terms(int mode, const RhsTerms &T, const double *k1, const double *k2, int nxh, int ny,
+                            long ncell, long nedge, double invRe, hipStream_t st)
 {
-    const dim3 g(blocks_for(n)), b(256);
-    if (mode == 0)
-        hipLaunchKernelGGL((k_add<double, double>), g, b, 0, st, (double *)r, (const double *)s, n);
-    else
-        hipLaunchKernelGGL((k_add<float, float>), g, b, 0, st, (float *)r, (const float *)s, n);
-    return hipGetLastError();
+#define PDO_CALL(TS, TC)                                                                                           \
+    hipLaunchKernelGGL((k_rhs_terms<TS, TC>), dim3(blocks_for(nedge)), dim3(256), 0, st, T, k1, k2, (unsigned)nxh, \
+                       (unsigned)ny, ncell, nedge, (TC)invRe)
+    PDO_MODES(PDO_CALL)
+#undef PDO_CALL
 }
 
-hipError_t launch_visc(int mode, void *rhs, const void *f, const void *d2, const double *k1, const double *k2, int nxh,
-                       int ny, long n, double invRe, hipStream_t st)
+hipError_t launch_stage(int mode, const StageTerms &T, const double *g1, const double *g2, int nxh, int ny, long ncell,
+                        long nedge, hipStream_t st)
 {
-    const dim3 g(blocks_for(n)), b(256);
-    switch (mode) {
-    case 0:
-        hipLaunchKernelGGL((k_visc<double, double>), g, b, 0, st, (double *)rhs, (const double *)f,
-                           (const double *)d2, k1, k2, nxh, ny, n, invRe);
-        break;
-    case 1:
-        hipLaunchKernelGGL((k_visc<float, float>), g, b, 0, st, (float *)rhs, (const float *)f, (const float *)d2, k1,
-                           k2, nxh, ny, n, invRe);
-        break;
-    default:
-        hipLaunchKernelGGL((k_visc<float, double>), g, b, 0, st, (float *)rhs, (const float *)f, (const float *)d2, k1,
-                           k2, nxh, ny, n, invRe);
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_lincomb(int mode, void *out, const void *const *x, const double *c, int nterms, long n,
-                          hipStream_t st)
-{
-    if (nterms < 1 || nterms > 5) return hipErrorInvalidValue;
-    LinComb L{};
-    for (int q = 0; q < nterms; ++q) { L.x[q] = x[q]; L.c[q] = c[q]; }
-    const dim3 g(blocks_for(n)), b(256);
-    switch (mode) {
-    case 0: hipLaunchKernelGGL((k_lincomb<double, double>), g, b, 0, st, (double *)out, L, n); break;
-    case 1: hipLaunchKernelGGL((k_lincomb<float, float>), g, b, 0, st, (float *)out, L, n); break;
-    default: hipLaunchKernelGGL((k_lincomb<float, double>), g, b, 0, st, (float *)out, L, n);
-    }
-    return hipGetLastError();
+    if (T.nterms < 1 || T.nterms > 5) return hipErrorInvalidValue;
+#define PDO_CALL(TS, TC)                                                                                       \
+    hipLaunchKernelGGL((k_stage<TS, TC>), dim3(blocks_for(nedge)), dim3(256), 0, st, T, g1, g2, (unsigned)nxh, \
+                       (unsigned)ny, ncell, nedge)
+    PDO_MODES(PDO_CALL)
+#undef PDO_CALL
 }
 
 hipError_t launch_cfl(int mode, const void *u, const void *v, const void *w, long n, double idx, double idy,

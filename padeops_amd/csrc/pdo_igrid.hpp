@@ -11,29 +11,43 @@ namespace pdo {
 // plane 0 of a spectrum of nplane complex values per plane: zero, except the
 // mean mode, which is set to v
 hipError_t launch_surface_plane(int mode, void *f, long nplane, double v, hipStream_t st);
-// tau = -2 nu S: cells (nC points) 11, 12, 22, 33; edges (nE points) 13, 23
-hipError_t launch_tau(int mode, const void *nuC, const void *SC, const void *nuE, const void *SE, void *tauC,
-                      void *tauE, long nC, long nE, hipStream_t st);
 // f[k nplane] += v (the real part of the mean mode of each of nz planes of
 // a spectrum with nplane complex values per plane)
 hipError_t launch_mean_add(int mode, void *f, long nplane, int nz, double v, hipStream_t st);
-// a = max(a, 0) (real)
-hipError_t launch_clip_negative(int mode, void *a, long n, hipStream_t st);
-// rhs -= i k f (kv per index along dim 1 or 2) or rhs -= f (kv NULL); complex
-hipError_t launch_sub(int mode, void *rhs, const void *f, const double *kv, int nxh, int ny, long n, int dim,
-                      hipStream_t st);
+// subgrid terms of one set of points: nu from the gradients g (9 components n
+// apart) and the model constant (cplane per plane of nxy points, or cglobal),
+// and tau = -2 nu S: on cells 11, 12, 22, 33; on edges 13, 23
+hipError_t launch_sgs_tau(int mode, bool edges, const void *g, void *nu, void *tau, long n, long nxy, int model,
+                          const double (&camd)[3], const double *cplane, double cglobal, hipStream_t st);
+// edges, nu given: nu = max(nu, 0) with clip, and tau
+hipError_t launch_edge_tau(int mode, bool clip, const void *g, void *nu, void *tau, long n, hipStream_t st);
+// divergence of the stress from its spectra: u -= i k1 t11 + i k2 t12 + z13,
+// v -= i k1 t12 + i k2 t22 + z23 (cells), w -= z33 + i k1 t13 + i k2 t23
+// (edges); complex, cells ncell values, edges nedge
+struct StressSpectra {
+    const void *t11, *t12, *t22, *z13, *z23, *z33, *t13, *t23;
+};
+hipError_t launch_stress_div(int mode, void *u, void *v, void *w, const StressSpectra &S, const double *k1,
+                             const double *k2, int nxh, int ny, long ncell, long nedge, hipStream_t st);
 
-// out = (a1 - b1) c1 + (a2 - b2) c2 (second term when a2 != NULL), real
-hipError_t launch_cross(int mode, const void *a1, const void *b1, const void *c1, const void *a2, const void *b2,
-                        const void *c2, void *out, long n, hipStream_t st);
-// r += s (n real words)
-hipError_t launch_add(int mode, void *r, const void *s, long n, hipStream_t st);
-// rhs += invRe (-(k1^2 + k2^2) f + d2) on complex (nxh, ny, planes)
-hipError_t launch_visc(int mode, void *rhs, const void *f, const void *d2, const double *k1, const double *k2, int nxh,
-                       int ny, long n, double invRe, hipStream_t st);
-// out = c[0] x[0] + ... + c[nterms-1] x[nterms-1] (n real words, left to right)
-hipError_t launch_lincomb(int mode, void *out, const void *const *x, const double *c, int nterms, long n,
-                          hipStream_t st);
+// rhs[c] += s[c] (c = 0, 1; null: nothing) + invRe (-(k1^2 + k2^2) f[c] + d2[c])
+// (invRe 0: nothing), c = 0, 1 on cells, 2 on edges; complex
+struct RhsTerms {
+    void *rhs[3];
+    const void *s[3], *f[3], *d2[3];
+};
+hipError_t launch_rhs_terms(int mode, const RhsTerms &T, const double *k1, const double *k2, int nxh, int ny,
+                            long ncell, long nedge, double invRe, hipStream_t st);
+// out[c] = (coef[0] x[0][c] + ... + coef[nterms-1] x[nterms-1][c], left to
+// right) g1[kx] g2[ky], components c = 0, 1 on cells, 2 on edges; complex
+struct StageTerms {
+    void *out[3];
+    const void *x[5][3];
+    double coef[5];
+    int nterms;
+};
+hipError_t launch_stage(int mode, const StageTerms &T, const double *g1, const double *g2, int nxh, int ny, long ncell,
+                        long nedge, hipStream_t st);
 // partial[b] = max over block b of |u|/dx + |v|/dy + |w|/dz (nblocks blocks)
 hipError_t launch_cfl(int mode, const void *u, const void *v, const void *w, long n, double idx, double idy,
                       double idz, double *partial, int nblocks, hipStream_t st);
@@ -49,6 +63,14 @@ hipError_t launch_wall_model(int mode, const void *u, const void *v, void *tauE,
                              int nb, double kappa, double lg, double *wm, hipStream_t st);
 // whether a Pade6stagg object is periodic (pdo_pade6.cpp)
 bool pade6stagg_periodic(pdo_pade6stagg h);
+
+struct BandLimit;
+// interp_PrimitiveVars and compute_duidxj of dealiased spectra in one go: the
+// physical fields, their gradients and the second derivatives; I.uE etc. as
+// in those, with u, v, w the physical velocity too.  The gradient spectra
+// (duidxjChat, duidxjEhat) are work here and do not come back.
+int igrid_fields(pdo_duidxj h, int prec, const pdo_interp_fields &I, const pdo_duidxj_fields &D, void *u, void *v,
+                 void *w, const BandLimit &bl, hipStream_t st);
 
 struct HitForcingArgs {
     int nxh, ny, nz, nwaves;

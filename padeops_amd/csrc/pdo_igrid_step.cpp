@@ -57,7 +57,7 @@ struct IgridObject {
     void *whC = nullptr, *uEh = nullptr, *vEh = nullptr;
     void *gC = nullptr, *gE = nullptr, *gCh = nullptr, *gEh = nullptr;
     void *d2w = nullptr, *d2u = nullptr, *d2v = nullptr;
-    void *tC1 = nullptr, *tE1 = nullptr, *fC1 = nullptr, *fE1 = nullptr;  // nonlinear-term work
+    BandLimit band{};  // modes the dealiasing leaves
     double *k3 = nullptr;
     double *partial = nullptr;
     int nblocks = 1024;
@@ -107,33 +107,56 @@ namespace {
         if (e_ != hipSuccess) return hip_fail(e_, what); \
     } while (0)
 
-// project_and_prep (igrid.F90:1961-1992) for the spectra (uh, vh, wh)
-int project_and_prep(pdo_igrid h, void *uh, void *vh, void *wh, hipStream_t st)
+// the modes left by the x-y mask g1[kx] g2[ky]
+BandLimit band_of(const SpectralObject &s)
+{
+    BandLimit b{0, 0};
+    while (b.kxc < s.nxh && s.g1[b.kxc] != 0.0) b.kxc++;
+    while (b.kyc < s.ny && s.g2[b.kyc] != 0.0) b.kyc++;
+    bool plain = b.kxc > 0;
+    for (int i = b.kxc; i < s.nxh; i++) plain = plain && s.g1[i] == 0.0;
+    for (int j = b.kyc; j < s.ny; j++) plain = plain && (s.g2[j] == 0.0) == (j <= s.ny - b.kyc);
+    return plain ? b : BandLimit{s.nxh, s.ny};
+}
+
+// dealiasFields (igrid.F90:1020-1037): periodic in z the 3D mask on cells,
+// the edge variant on w; with walls the x-y mask of each object.  masked: the
+// x-y mask is applied already, and its zero lines need no z transform.
+int dealias_fields(pdo_igrid h, void *uh, void *vh, void *wh, bool masked, hipStream_t st)
 {
     void *s = (void *)st;
-    // Step 1: dealiasFields (:1020-1037; periodic in z: the 3D mask on cells,
-    // the edge variant on w; with walls the x-y mask of each object)
-    PDO_TRY(pdo_spectral_dealias(h->spC, h->prec, uh, s));
-    PDO_TRY(pdo_spectral_dealias(h->spC, h->prec, vh, s));
-    if (h->p.walls) PDO_TRY(pdo_spectral_dealias(h->spE, h->prec, wh, s));
-    else PDO_TRY(pdo_spectral_dealias_edge(h->spC, h->prec, wh, s));
+    if (!masked) {
+        PDO_TRY(pdo_spectral_dealias(h->spC, h->prec, uh, s));
+        PDO_TRY(pdo_spectral_dealias(h->spC, h->prec, vh, s));
+        return h->p.walls ? pdo_spectral_dealias(h->spE, h->prec, wh, s)
+                          : pdo_spectral_dealias_edge(h->spC, h->prec, wh, s);
+    }
+    if (h->p.walls) return 0;
+    const SpectralObject &C = *h->spC;
+    const SpecMul m{C.d_g1, C.d_g2, C.d_g3, 2, 1.0 / h->nz};
+    for (void *f : {uh, vh, wh}) PDO_HIP(run_zmul(C.plan, h->mode, f, f, m, st, h->band.kxc), "dealias");
+    // edge nz + 1 repeats edge 1
+    const size_t plane = (size_t)h->nxh * h->ny * 2 * h->W;
+    PDO_HIP(hipMemcpyAsync((char *)wh + plane * h->nz, wh, plane, hipMemcpyDeviceToDevice, st), "dealias");
+    return 0;
+}
+
+// project_and_prep (igrid.F90:1961-1992) for the spectra (uh, vh, wh)
+int project_and_prep(pdo_igrid h, void *uh, void *vh, void *wh, bool masked, hipStream_t st)
+{
+    // Step 1: dealiasFields
+    PDO_TRY(dealias_fields(h, uh, vh, wh, masked, st));
     // Step 2: pressure projection
-    PDO_TRY(pdo_padepoisson_projection(h->pp, h->prec, uh, vh, wh, s));
-    // Step 3: physical fields
-    PDO_TRY(pdo_spectral_ifft(h->spC, h->prec, uh, h->u, 0, s));
-    PDO_TRY(pdo_spectral_ifft(h->spC, h->prec, vh, h->v, 0, s));
-    PDO_TRY(pdo_spectral_ifft(h->spE, h->prec, wh, h->w, 0, s));
-    // Step 4: interp_PrimitiveVars
+    PDO_TRY(pdo_padepoisson_projection(h->pp, h->prec, uh, vh, wh, (void *)st));
+    // Steps 3-5: the physical fields, interp_PrimitiveVars and compute_duidxj
     pdo_interp_fields I{};
     I.uhat = uh; I.vhat = vh; I.what = wh;
     I.whatC = h->whC; I.wC = h->wC; I.uEhat = h->uEh; I.uE = h->uE; I.vEhat = h->vEh; I.vE = h->vE;
-    PDO_TRY(pdo_igrid_interp_primitive(h->dj, h->prec, &I, s));
-    // Step 5: compute_duidxj
     pdo_duidxj_fields D{};
     D.uhat = uh; D.vhat = vh; D.whatC = h->whC; D.what = wh; D.uEhat = h->uEh; D.vEhat = h->vEh;
     D.duidxjC = h->gC; D.duidxjE = h->gE; D.duidxjChat = h->gCh; D.duidxjEhat = h->gEh;
     D.d2wdz2hatE = h->d2w; D.d2udz2hatC = h->d2u; D.d2vdz2hatC = h->d2v;
-    PDO_TRY(pdo_duidxj_compute(h->dj, h->prec, &D, s));
+    PDO_TRY(igrid_fields(h->dj, h->prec, I, D, h->u, h->v, h->w, h->band, st));
     h->cur_u = uh; h->cur_v = vh; h->cur_w = wh;
     return 0;
 }
@@ -144,43 +167,29 @@ int populate_rhs(pdo_igrid h, void *ur, void *vr, void *wr, hipStream_t st)
     void *s = (void *)st;
     const int mode = h->mode;
     const size_t W = h->W;
-    auto g = [&](void *base, size_t n, int slot) { return (const void *)((const char *)base + (slot - 1) * n * W); };
-    const size_t nC = h->nC, nE = h->nE;
-    const long nsC = (long)(h->sC / 2), nsE = (long)(h->sE / 2);
+    auto slot = [&](void *base, size_t n, int k) { return (void *)((char *)base + (k - 1) * n * W); };
+    auto gC = [&](int k) { return (const void *)slot(h->gC, h->nC, k); };
+    auto gE = [&](int k) { return (const void *)slot(h->gE, h->nE, k); };
+    const size_t nC = h->nC;
     // Step 1: AddNonLinearTerm_Rot (:1497-1566)
     //   u: T1C = (dvdx - dudy) v, T2E = (dwdx - dudz) w; urhs = E2C(fft T2E) + fft T1C
-    PDO_HIP(launch_cross(mode, g(h->gC, nC, 4), g(h->gC, nC, 2), h->v, nullptr, nullptr, nullptr, h->tC1, (long)nC, st),
-            "nonlinear");
-    PDO_TRY(pdo_spectral_fft(h->spC, h->prec, h->tC1, h->fC1, s));
-    PDO_HIP(launch_cross(mode, g(h->gE, nE, 7), g(h->gE, nE, 3), h->w, nullptr, nullptr, nullptr, h->tE1, (long)nE, st),
-            "nonlinear");
-    PDO_TRY(pdo_spectral_fft(h->spE, h->prec, h->tE1, h->fE1, s));
-    PDO_TRY(pdo_pade6stagg_apply(h->d6, 14, 0, 0, h->prec, h->fE1, ur, h->nxh, h->ny, 1, s));
-    PDO_HIP(launch_add(mode, ur, h->fC1, (long)h->sC, st), "nonlinear");
     //   v: T1C = (dudy - dvdx) u, T2E = (dwdy - dvdz) w
-    PDO_HIP(launch_cross(mode, g(h->gC, nC, 2), g(h->gC, nC, 4), h->u, nullptr, nullptr, nullptr, h->tC1, (long)nC, st),
-            "nonlinear");
-    PDO_TRY(pdo_spectral_fft(h->spC, h->prec, h->tC1, h->fC1, s));
-    PDO_HIP(launch_cross(mode, g(h->gE, nE, 8), g(h->gE, nE, 6), h->w, nullptr, nullptr, nullptr, h->tE1, (long)nE, st),
-            "nonlinear");
-    PDO_TRY(pdo_spectral_fft(h->spE, h->prec, h->tE1, h->fE1, s));
-    PDO_TRY(pdo_pade6stagg_apply(h->d6, 14, 0, 0, h->prec, h->fE1, vr, h->nxh, h->ny, 1, s));
-    PDO_HIP(launch_add(mode, vr, h->fC1, (long)h->sC, st), "nonlinear");
     //   w: T1E = (dudz - dwdx) uE + (dvdz - dwdy) vE; wrhs = fft T1E
-    PDO_HIP(launch_cross(mode, g(h->gE, nE, 3), g(h->gE, nE, 7), h->uE, g(h->gE, nE, 6), g(h->gE, nE, 8), h->vE, h->tE1,
-                         (long)nE, st),
-            "nonlinear");
-    PDO_TRY(pdo_spectral_fft(h->spE, h->prec, h->tE1, wr, s));
-    // Step 5: addViscousTerm (:1914-1959)
-    if (h->p.Re > 0) {
-        const double invRe = 1.0 / h->p.Re;
-        PDO_HIP(launch_visc(mode, ur, h->cur_u, h->d2u, h->spC->d_k1, h->spC->d_k2, h->nxh, h->ny, nsC, invRe, st),
-                "viscous");
-        PDO_HIP(launch_visc(mode, vr, h->cur_v, h->d2v, h->spC->d_k1, h->spC->d_k2, h->nxh, h->ny, nsC, invRe, st),
-                "viscous");
-        PDO_HIP(launch_visc(mode, wr, h->cur_w, h->d2w, h->spE->d_k1, h->spE->d_k2, h->nxh, h->ny, nsE, invRe, st),
-                "viscous");
-    }
+    // (the gradients' spectra are free between two preparations)
+    void *fC[2] = {slot(h->gCh, h->sC, 1), slot(h->gCh, h->sC, 2)}, *fE[2] = {slot(h->gEh, h->sE, 1), slot(h->gEh, h->sE, 2)};
+    const FwdTask task[5] = {{gC(4), gC(2), h->v, nullptr, nullptr, nullptr, fC[0], h->nz},
+                             {gC(2), gC(4), h->u, nullptr, nullptr, nullptr, fC[1], h->nz},
+                             {gE(7), gE(3), h->w, nullptr, nullptr, nullptr, fE[0], h->nz + 1},
+                             {gE(8), gE(6), h->w, nullptr, nullptr, nullptr, fE[1], h->nz + 1},
+                             {gE(3), gE(7), h->uE, gE(6), gE(8), h->vE, wr, h->nz + 1}};
+    PDO_HIP(run_fwd_multi(h->spC->plan, mode, task, 5, st), "nonlinear");
+    PDO_TRY(pdo_pade6stagg_apply(h->d6, 14, 0, 0, h->prec, fE[0], ur, h->nxh, h->ny, 1, s));
+    PDO_TRY(pdo_pade6stagg_apply(h->d6, 14, 0, 0, h->prec, fE[1], vr, h->nxh, h->ny, 1, s));
+    // ... and Step 5: addViscousTerm (:1914-1959)
+    const RhsTerms T{{ur, vr, wr}, {fC[0], fC[1], nullptr}, {h->cur_u, h->cur_v, h->cur_w}, {h->d2u, h->d2v, h->d2w}};
+    PDO_HIP(launch_rhs_terms(mode, T, h->spC->d_k1, h->spC->d_k2, h->nxh, h->ny, (long)(h->sC / 2), (long)(h->sE / 2),
+                             h->p.Re > 0 ? 1.0 / h->p.Re : 0.0, st),
+            "nonlinear and viscous terms");
     // Step 6: SGS stress divergence (with the dynamic procedure's planar
     // coefficient of this stage for closure kinds 1 and 2)
     if (h->sgs) {
@@ -238,17 +247,20 @@ int compute_dt(pdo_igrid h, hipStream_t st)
     return 0;
 }
 
-// one linear combination per velocity component; x[q] and c[q] of the
-// cell components, the edge component's operands follow the same pattern
+// a Runge-Kutta stage: one linear combination per velocity component, with
+// the x-y part of the dealiasing that follows it
 int combine(pdo_igrid h, void *const out[3], const std::vector<void *const *> &terms, const std::vector<double> &c,
             hipStream_t st)
 {
+    StageTerms T{};
+    T.nterms = (int)terms.size();
     for (int comp = 0; comp < 3; comp++) {
-        const void *x[5];
-        for (size_t q = 0; q < terms.size(); q++) x[q] = terms[q][comp];
-        const long n = (long)(comp == 2 ? h->sE : h->sC);
-        PDO_HIP(launch_lincomb(h->mode, out[comp], x, c.data(), (int)terms.size(), n, st), "stage update");
+        T.out[comp] = out[comp];
+        for (size_t q = 0; q < terms.size(); q++) T.x[q][comp] = terms[q][comp];
     }
+    for (size_t q = 0; q < c.size(); q++) T.coef[q] = c[q];
+    PDO_HIP(launch_stage(h->mode, T, h->spC->d_g1, h->spC->d_g2, h->nxh, h->ny, (long)(h->sC / 2), (long)(h->sE / 2), st),
+            "stage update");
     return 0;
 }
 
@@ -270,23 +282,23 @@ int ssp_rk45(pdo_igrid h, hipStream_t st)
     PDO_TRY(populate_rhs(h, h->ur, h->vr, h->wr, st));
     h->newTimeStep = false;
     PDO_TRY(combine(h, S1, {S0, R}, {1.0, b01 * dt}, st));
-    PDO_TRY(project_and_prep(h, S1[0], S1[1], S1[2], st));
+    PDO_TRY(project_and_prep(h, S1[0], S1[1], S1[2], true, st));
     // stage 2
     PDO_TRY(populate_rhs(h, h->ur, h->vr, h->wr, st));
     PDO_TRY(combine(h, S2, {S0, S1, R}, {a20, a21, b12 * dt}, st));
-    PDO_TRY(project_and_prep(h, S2[0], S2[1], S2[2], st));
+    PDO_TRY(project_and_prep(h, S2[0], S2[1], S2[2], true, st));
     // stage 3
     PDO_TRY(populate_rhs(h, h->ur, h->vr, h->wr, st));
     PDO_TRY(combine(h, S3, {S0, S2, R}, {a30, a32, b23 * dt}, st));
-    PDO_TRY(project_and_prep(h, S3[0], S3[1], S3[2], st));
+    PDO_TRY(project_and_prep(h, S3[0], S3[1], S3[2], true, st));
     // stage 4 (u4 overwrites the state in place)
     PDO_TRY(populate_rhs(h, h->ur, h->vr, h->wr, st));
     PDO_TRY(combine(h, S0, {S0, S3, R}, {a40, a43, b34 * dt}, st));
-    PDO_TRY(project_and_prep(h, S0[0], S0[1], S0[2], st));
+    PDO_TRY(project_and_prep(h, S0[0], S0[1], S0[2], true, st));
     // stage 5: rhs of u4 into the spare buffers; R still holds L(u3)
     PDO_TRY(populate_rhs(h, h->ur5, h->vr5, h->wr5, st));
     PDO_TRY(combine(h, S0, {S2, S3, R, S0, R5}, {a52, a53, b35 * dt, a54, b45 * dt}, st));
-    PDO_TRY(project_and_prep(h, S0[0], S0[1], S0[2], st));
+    PDO_TRY(project_and_prep(h, S0[0], S0[1], S0[2], true, st));
     return 0;
 }
 
@@ -299,13 +311,13 @@ int tvd_rk3(pdo_igrid h, hipStream_t st)
     PDO_TRY(populate_rhs(h, h->ur, h->vr, h->wr, st));
     h->newTimeStep = false;
     PDO_TRY(combine(h, S1, {S0, R}, {1.0, dt}, st));
-    PDO_TRY(project_and_prep(h, S1[0], S1[1], S1[2], st));
+    PDO_TRY(project_and_prep(h, S1[0], S1[1], S1[2], true, st));
     PDO_TRY(populate_rhs(h, h->ur, h->vr, h->wr, st));
     PDO_TRY(combine(h, S1, {S0, S1, R}, {3.0 / 4.0, 1.0 / 4.0, (1.0 / 4.0) * dt}, st));
-    PDO_TRY(project_and_prep(h, S1[0], S1[1], S1[2], st));
+    PDO_TRY(project_and_prep(h, S1[0], S1[1], S1[2], true, st));
     PDO_TRY(populate_rhs(h, h->ur, h->vr, h->wr, st));
     PDO_TRY(combine(h, S0, {S0, S1, R}, {1.0 / 3.0, 2.0 / 3.0, (2.0 / 3.0) * dt}, st));
-    PDO_TRY(project_and_prep(h, S0[0], S0[1], S0[2], st));
+    PDO_TRY(project_and_prep(h, S0[0], S0[1], S0[2], true, st));
     return 0;
 }
 
@@ -383,6 +395,7 @@ int pdo_igrid_init(pdo_igrid *out, const pdo_igrid_params *p, int prec)
     }
     if (!st && p->use_sgs) st = pdo_sgsrhs_init(&h->sgs, h->spC, h->spE, h->d6, &p->sgs, prec);
     if (st) { delete h; return st; }
+    h->band = band_of(*h->spC);
     const size_t W = h->W;
     h->nC = (size_t)h->nx * h->ny * h->nz;
     h->nE = (size_t)h->nx * h->ny * (h->nz + 1);
@@ -393,16 +406,16 @@ int pdo_igrid_init(pdo_igrid *out, const pdo_igrid_params *p, int prec)
         if (!st) st = h->alloc(&h->vh[i], h->sC * W);
         if (!st) st = h->alloc(&h->wh[i], h->sE * W);
     }
-    void **cbufs[] = {&h->ur, &h->vr, &h->ur5, &h->vr5, &h->whC, &h->d2u, &h->d2v, &h->fC1};
+    void **cbufs[] = {&h->ur, &h->vr, &h->ur5, &h->vr5, &h->whC, &h->d2u, &h->d2v};
     for (void **b : cbufs)
         if (!st) st = h->alloc(b, h->sC * W);
-    void **ebufs[] = {&h->wr, &h->wr5, &h->uEh, &h->vEh, &h->d2w, &h->fE1};
+    void **ebufs[] = {&h->wr, &h->wr5, &h->uEh, &h->vEh, &h->d2w};
     for (void **b : ebufs)
         if (!st) st = h->alloc(b, h->sE * W);
-    void **rC[] = {&h->u, &h->v, &h->wC, &h->tC1};
+    void **rC[] = {&h->u, &h->v, &h->wC};
     for (void **b : rC)
         if (!st) st = h->alloc(b, h->nC * W);
-    void **rE[] = {&h->w, &h->uE, &h->vE, &h->tE1};
+    void **rE[] = {&h->w, &h->uE, &h->vE};
     for (void **b : rE)
         if (!st) st = h->alloc(b, h->nE * W);
     if (!st) st = h->alloc(&h->gC, 9 * h->nC * W);
@@ -433,7 +446,7 @@ int pdo_igrid_set_velocity(pdo_igrid h, const void *u, const void *v, const void
     PDO_TRY(pdo_spectral_fft(h->spC, h->prec, u, h->uh[0], stream));
     PDO_TRY(pdo_spectral_fft(h->spC, h->prec, v, h->vh[0], stream));
     PDO_TRY(pdo_spectral_fft(h->spE, h->prec, w, h->wh[0], stream));
-    PDO_TRY(project_and_prep(h, h->uh[0], h->vh[0], h->wh[0], st));
+    PDO_TRY(project_and_prep(h, h->uh[0], h->vh[0], h->wh[0], false, st));
     h->tsim = 0; h->step = 0; h->newTimeStep = true; h->draws = 0;
     return 0;
 }
