@@ -888,7 +888,10 @@ template <int FAM, int MODE>
 static hipError_t launch_strided_t(const ApplyArgs &A, hipStream_t st)
 {
     if (!A.periodic) {
-        if (A.epi) return hipErrorInvalidValue;
+        // refined non-periodic passes run on overlapping segments
+        if (A.epi || MODE == MODE_F32R) return hipErrorInvalidValue;
+    }
+    if constexpr (MODE != MODE_F32R) if (!A.periodic) {
         if (A.xr) {
             if constexpr (has_extra_row<FAM>()) {
                 if (A.P <= 8) return launch_strided_k<FAM, MODE, 64, false, false, 1, 512>(A, st);

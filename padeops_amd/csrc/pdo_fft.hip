@@ -655,7 +655,7 @@ template <int L, size_t CE> constexpr int pp_walls_lines()
 {
     int tx = 512 / (L / 8);
     if (tx < 1) tx = 1;
-    while (tx > 1 && (2 * (size_t)tx + 1) * L * CE > 64 * 1024) tx >>= 1;
+    while (tx > 1 && (2 * (size_t)tx + 1) * L * CE > 80 * 1024) tx >>= 1;
     return tx;
 }
 
@@ -664,7 +664,8 @@ static void launch_pp_walls(TS *f, TS *w, long na, long sb, long se, const TC *t
                             bool upd, hipStream_t st)
 {
     constexpr size_t ce = 2 * sizeof(TC);
-    // two line tiles and the twiddles: at most 64 KiB
+    // two line tiles and the twiddles: at most 80 KiB, two workgroups to a CU
+    // (8 instead of 4 lines of 512 FP32 points: rows of 64 bytes)
     constexpr int TX = pp_walls_lines<L, ce>();
     const size_t lds = (2 * (size_t)TX + 1) * L * ce;
     dim3 grid((unsigned)((na + TX - 1) / TX), (unsigned)nb);
@@ -678,11 +679,11 @@ static void launch_pp_walls(TS *f, TS *w, long na, long sb, long se, const TC *t
 
 template <typename TS, typename TC>
 static hipError_t run_pp_walls_t(const PoissonPlanDev &pl, TS *f, TS *w, const PadeWallTables &t, bool upd,
-                                 hipStream_t st)
+                                 hipStream_t st, int lines)
 {
     const int ny = pl.ny, L = pl.nz, nxh = pl.nx / 2 + 1;
     const Tw<TC> tw(pl);
-    const long na = nxh, sb = nxh, se = (long)nxh * ny;
+    const long na = lines > 0 ? lines : nxh, sb = nxh, se = (long)nxh * ny;
     switch (L) {
     case 8: launch_pp_walls<TS, TC, 8>(f, w, na, sb, se, tw.z, t, ny, upd, st); break;
     case 16: launch_pp_walls<TS, TC, 16>(f, w, na, sb, se, tw.z, t, ny, upd, st); break;
@@ -698,12 +699,12 @@ static hipError_t run_pp_walls_t(const PoissonPlanDev &pl, TS *f, TS *w, const P
 }
 
 hipError_t run_pp_walls(const PoissonPlanDev &pl, int mode, void *f, void *w, const PadeWallTables &t, bool upd,
-                        hipStream_t st)
+                        hipStream_t st, int lines)
 {
     switch (mode) {
-    case 0: return run_pp_walls_t<double, double>(pl, (double *)f, (double *)w, t, upd, st);
-    case 1: return run_pp_walls_t<float, float>(pl, (float *)f, (float *)w, t, upd, st);
-    case 2: return run_pp_walls_t<float, double>(pl, (float *)f, (float *)w, t, upd, st);
+    case 0: return run_pp_walls_t<double, double>(pl, (double *)f, (double *)w, t, upd, st, lines);
+    case 1: return run_pp_walls_t<float, float>(pl, (float *)f, (float *)w, t, upd, st, lines);
+    case 2: return run_pp_walls_t<float, double>(pl, (float *)f, (float *)w, t, upd, st, lines);
     }
     return hipErrorInvalidValue;
 }

@@ -66,9 +66,10 @@ struct PadeWallTables {
 };
 // the extended solve and (upd) w update of PadePoisson with walls, in place
 // on f (nx/2+1, ny, nz) and w (nx/2+1, ny, nz+1); upd false leaves w as it
-// is; the plan's transforms have length 2 nz (its nz)
+// is; the plan's transforms have length 2 nz (its nz); lines > 0: the first
+// `lines` kx only
 hipError_t run_pp_walls(const PoissonPlanDev &pl, int mode, void *f, void *w, const PadeWallTables &t, bool upd,
-                        hipStream_t st);
+                        hipStream_t st, int lines = 0);
 
 // Transforms of several fields in few launches (pdo_fft_multi.hip).  All
 // fields share the plan's nx, ny; planes may differ.

@@ -396,6 +396,7 @@ int pdo_igrid_init(pdo_igrid *out, const pdo_igrid_params *p, int prec)
     if (!st && p->use_sgs) st = pdo_sgsrhs_init(&h->sgs, h->spC, h->spE, h->d6, &p->sgs, prec);
     if (st) { delete h; return st; }
     h->band = band_of(*h->spC);
+    h->pp->lines = h->band.kxc;
     const size_t W = h->W;
     h->nC = (size_t)h->nx * h->ny * h->nz;
     h->nE = (size_t)h->nx * h->ny * (h->nz + 1);

@@ -173,7 +173,7 @@ static bool overlap_fits(const Variant &v, int dir, long na, long nb, size_t wor
         if (f.shift != 0 || s.n_in != s.n_sys || s.n_out != s.n_sys) return false;
         // at least 8 pencils fit a workgroup's LDS, with the exchange values and tables
         const size_t pen = (size_t)(s.n_sys | 1) * word + (size_t)o.P * 2 * o.K * 8;
-        return 8 * pen + (s.periodic ? 0 : 3 * (size_t)o.m * 9 * 8) + 24 * 1024 <= 160 * 1024 &&
+        return 8 * pen + (s.periodic ? 0 : 3 * (size_t)o.m * 9 * 8) + 4 * 1024 <= 160 * 1024 &&
                (size_t)na * nb < ((size_t)1 << 31);
     }
     if (o.P > PMAX && (f.shift != 0 || o.m != MAXM)) return false;
@@ -242,6 +242,15 @@ static int prepare(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, 
     scratch_elems = (shape == SHAPE_GENERAL) ? (size_t)s.n_sys * (size_t)(na * nb) : 0;
     if (shape == SHAPE_GENERAL && force_shape != SHAPE_GENERAL && !epi && overlap_fits(*v, dir, na, nb, word))
         shape = dir == 1 ? SHAPE_OVL_X : SHAPE_OVL_STRIDED;
+    // FP32 + refinement without periodicity: the refined kernels carry two
+    // solves and closure rows in up to 149 registers and scratch, the
+    // overlapping segments one FP64 solve (512 x 512 x 256 FP32, along z: cd10
+    // 287 -> 160 us, cf90 298 -> 163, 257-row staggered systems 231 -> 174,
+    // cd06 131 -> 134; 512^3: cd06 317 -> 258).  FP64 passes stay (cd10 216
+    // against 257 us), and so do periodic ones (cd10 150 against 166).
+    if (shape == SHAPE_STRIDED && !s.periodic && mode == MODE_F32R && v->ovl.P <= PMAX &&
+        overlap_fits(*v, dir, na, nb, word))
+        shape = SHAPE_OVL_STRIDED;
     TabSet *ts = &v->fast;
     if (shape == SHAPE_GENERAL && !v->fast.tab.general) {
         // built with the variant

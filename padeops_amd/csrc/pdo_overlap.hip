@@ -367,11 +367,12 @@ __global__ void __launch_bounds__(512) k_ovl_x(ApplyArgs A, int TP, int LD, unsi
     }
 }
 
-// coupling rows staged in LDS up to 24 KiB
+// coupling rows staged in LDS up to 4 KiB: the ones of long pencils would
+// cost a workgroup per CU (they come through the cache then)
 template <int K> int staged_words(const ApplyArgs &A)
 {
     const int words = (A.guni ? 1 : A.P) * A.nd * 4 * K * K;
-    return words <= 3072 ? words : 0;
+    return words <= 512 ? words : 0;
 }
 
 template <int FAM, typename TS, int M> hipError_t strided_m(ApplyArgs A, hipStream_t st)

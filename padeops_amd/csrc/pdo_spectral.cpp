@@ -420,7 +420,7 @@ static int walls_solve(pdo_padepoisson h, int mode, void *uhat, void *vhat, void
         return hip_fail(e, "Stokes pressure");
     if ((e = launch_div_spec(mode, uhat, vhat, nullptr, h->f, k1, k2, s->nxh, s->ny, ncell, str)) != hipSuccess)
         return hip_fail(e, "projection divergence");
-    if ((e = run_pp_walls(h->zplan2, mode, h->f, what, h->wt, upd, str)) != hipSuccess)
+    if ((e = run_pp_walls(h->zplan2, mode, h->f, what, h->wt, upd, str, h->lines)) != hipSuccess)
         return hip_fail(e, "projection solve");
     if (upd && (e = launch_proj_update(mode, uhat, vhat, what, h->f, nullptr, k1, k2, s->nxh, s->ny, ncell, ncell,
                                        str)) != hipSuccess)
@@ -451,7 +451,7 @@ static int periodic_solve(pdo_padepoisson h, int mode, int prec, void *uhat, voi
     hipError_t e = launch_div_spec(mode, uhat, vhat, h->f, h->f, s->d_k1, s->d_k2, s->nxh, s->ny, ncell, str);
     if (e != hipSuccess) return hip_fail(e, "projection divergence");
     const SpecMul m{h->d_ax, h->d_ay, h->d_az, 1, 1.0 / h->nz};
-    if ((e = run_zmul(h->zplan, mode, h->f, h->f, m, str)) != hipSuccess) return hip_fail(e, "projection solve");
+    if ((e = run_zmul(h->zplan, mode, h->f, h->f, m, str, h->lines)) != hipSuccess) return hip_fail(e, "projection solve");
     if (!upd) return 0;
     if ((st = apply(h->derz, KIND_STG_D1_C2E, 0, 0, 3, prec, h->f, h->dp, 2L * s->nxh, s->ny, str))) return st;
     e = launch_proj_update(mode, uhat, vhat, what, h->f, h->dp, s->d_k1, s->d_k2, s->nxh, s->ny, ncell, nedge, str);

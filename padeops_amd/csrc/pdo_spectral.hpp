@@ -66,6 +66,7 @@ struct PadePoissonObject {
     size_t f_bytes = 0, dp_bytes = 0;
     // walls in z (init_nonperiodic): transforms of the 2 nz-point
     // extensions and their tables; the odd-ended cd06stagg of DivergenceCheck
+    int lines = 0;  // > 0: u, v, w vanish from this kx on (dealiased by the caller)
     bool periodic = true;
     pdo_op_s *dz_odd = nullptr;
     PoissonPlanDev zplan2{};
