@@ -887,9 +887,14 @@ template <int FAM> constexpr bool has_epilogue() { return FAM == 0; }
 template <int FAM, int MODE>
 static hipError_t launch_strided_t(const ApplyArgs &A, hipStream_t st)
 {
-    if (!A.periodic) {
-        // refined non-periodic passes run on overlapping segments
-        if (A.epi || MODE == MODE_F32R) return hipErrorInvalidValue;
+    if (!A.periodic && A.epi) return hipErrorInvalidValue;
+    if constexpr (MODE == MODE_F32R) if (!A.periodic) {
+        // refined non-periodic passes run on overlapping segments, but for
+        // the 513 rows (32 x 16 + 1) of the tridiagonal families: one segment
+        // more than those take
+        if constexpr (has_extra_row<FAM>())
+            if (A.xr && A.P > 8) return launch_strided_k<FAM, MODE, 64, false, false, 1, 1024>(A, st);
+        return hipErrorInvalidValue;
     }
     if constexpr (MODE != MODE_F32R) if (!A.periodic) {
         if (A.xr) {
