@@ -21,18 +21,21 @@ enum {
     F_PRIM = 0,            // rho u v w e p T
     F_G = F_PRIM + 7,      // du_i/dx_j at 3 i + j
     F_MU = F_G + 9,        // mu, bulk, kap (physical + artificial)
-    F_STAR = F_MU + 3,     // mustar, bulkstar, kapstar
-    F_TAU = F_STAR + 3,    // xx xy xz yy yz zz
+    F_TAU = F_MU + 3,      // xx xy xz yy yz zz
     F_Q = F_TAU + 6,       // qx qy qz
-    F_FUNC = F_Q + 3,
-    F_T1 = F_FUNC + 1,
-    F_D4 = F_T1 + 1,       // fourth derivatives along x, y, z
-    F_R = F_D4 + 3,        // gradient of rho or e
-    F_FIL = F_R + 3,       // two filter buffers
-    F_FLUX = F_FIL + 2,    // five fluxes
-    F_DFLUX = F_FLUX + 5,  // their derivatives
-    F_COUNT = F_DFLUX + 5
+    F_STAR = F_Q + 3,      // mustar, bulkstar, kapstar
+    F_DE = F_STAR + 3,     // gradient of e
+    // of the artificial coefficients alone: the fluxes overlie them
+    F_T1 = F_DE + 3,       // a second derivative per coefficient
+    F_D4 = F_T1 + 3,       // fourth derivatives along x, y, z of each
+    F_FIL = F_D4 + 9,      // two filter buffers for each
+    F_DRHO = F_FIL + 6,    // gradient of rho
+    F_FUNC = F_DRHO + 3,   // strain-rate magnitude
+    F_DIL = F_FUNC + 1,    // dilatation
+    F_COUNT = F_DIL + 1,
+    F_FLUX = F_T1          // momentum and energy fluxes per direction
 };
+static_assert(F_COUNT - F_FLUX >= 12, "the fluxes overlie 12 work fields");
 
 struct CgridObject {
     pdo_cgrid_params p{};
@@ -100,54 +103,64 @@ int gradient(pdo_cgrid h, const void *f, void *out3, int flipdir, hipStream_t st
     return 0;
 }
 
-// the fourth derivative along each direction (two second-derivative passes)
-// into F_D4 + d
-int fourth(pdo_cgrid h, const void *f, hipStream_t st)
+// the fourth derivatives along each direction (two second-derivative passes)
+// of the functions of the coefficients [k0, k1) into F_D4 + 3 k + d
+int fourth(pdo_cgrid h, const void *const f[3], int k0, int k1, hipStream_t st)
 {
     for (int d = 0; d < 3; d++) {
         const int *b = bc_of(h, d);
-        PDO_TRY(d2(h, d, f, h->f(F_T1), b[0], b[1], st));
-        PDO_TRY(d2(h, d, h->f(F_T1), h->f(F_D4 + d), b[0], b[1], st));
+        for (int k = k0; k < k1; k++) PDO_TRY(d2(h, d, f[k], h->f(F_T1 + k), b[0], b[1], st));
+        for (int k = k0; k < k1; k++) PDO_TRY(d2(h, d, h->f(F_T1 + k), h->f(F_D4 + 3 * k + d), b[0], b[1], st));
     }
     return 0;
 }
 
 // filter (cgrid.F90:1259-1336): numtimes passes along y, then x, then z, in
-// place on arr, through the two filter buffers
-int filter3(pdo_cgrid h, pdo_filters fl, void *arr, int numtimes, hipStream_t st)
+// place on each of arr[0 .. count), through two buffers each.  Two
+// applications along a direction go together where the filter can.
+int filter3(pdo_cgrid h, pdo_filters fl, void *const *arr, int count, int numtimes, hipStream_t st)
 {
     void *s = (void *)st;
-    void *bufs[2] = {h->f(F_FIL), h->f(F_FIL + 1)};
     const int order[3] = {1, 0, 2};
-    const int total = 3 * numtimes;
-    void *cur = arr;
-    int k = 0, pass = 0;
-    for (int q = 0; q < 3; q++) {
-        const int d = order[q];
+    int total = 0;
+    for (int d : order) total += filters_twice(fl, d, h->prec) ? (numtimes + 1) / 2 : numtimes;
+    void *cur[3];
+    for (int k = 0; k < count; k++) cur[k] = arr[k];
+    int pass = 0, buf = 0;
+    for (int d : order) {
         const int *b = bc_of(h, d);
-        for (int r = 0; r < numtimes; r++, pass++) {
+        const bool two = filters_twice(fl, d, h->prec);
+        for (int left = numtimes; left > 0; pass++) {
+            const int times = two && left > 1 ? 2 : 1;
             // out of place: the last pass writes arr unless it also reads it
-            void *dst = (pass == total - 1 && cur != arr) ? arr : bufs[k];
-            const int e = d == 0 ? pdo_filters_filterx(fl, h->prec, cur, dst, b[0], b[1], s)
-                        : d == 1 ? pdo_filters_filtery(fl, h->prec, cur, dst, b[0], b[1], s)
-                                 : pdo_filters_filterz(fl, h->prec, cur, dst, b[0], b[1], s);
-            if (e) return e;
-            if (dst != arr) k ^= 1;
-            cur = dst;
+            const bool home = pass == total - 1 && cur[0] != arr[0];
+            for (int k = 0; k < count; k++) {
+                void *dst = home ? arr[k] : h->f(F_FIL + 2 * k + buf);
+                const int e = times == 2 ? filters_apply_twice(fl, d, h->prec, cur[k], dst, b[0], b[1], st)
+                            : d == 0     ? pdo_filters_filterx(fl, h->prec, cur[k], dst, b[0], b[1], s)
+                            : d == 1     ? pdo_filters_filtery(fl, h->prec, cur[k], dst, b[0], b[1], s)
+                                         : pdo_filters_filterz(fl, h->prec, cur[k], dst, b[0], b[1], s);
+                if (e) return e;
+                cur[k] = dst;
+            }
+            buf ^= 1;
+            left -= times;
         }
     }
-    if (cur != arr) {
+    for (int k = 0; k < count; k++) {
+        if (cur[k] == arr[k]) continue;
         CgArgs a;
-        a.in[0] = cur;
-        a.out[0] = arr;
+        a.in[0] = cur[k];
+        a.out[0] = arr[k];
         a.n = h->n;
         PDO_TRY(cg(h, CG_COPY, a, st));
     }
     return 0;
 }
 
-// getLAD (cgrid.F90:1058-1257), one species: adds the filtered artificial
-// shear and bulk viscosity and conductivity to mu, bulk, kap
+// getLAD (cgrid.F90:1058-1257), one species: the filtered artificial shear
+// and bulk viscosity and conductivity into F_STAR.  Gradients of rho and e
+// precede it.
 int lad(pdo_cgrid h, hipStream_t st)
 {
     const pdo_cgrid_params &p = h->p;
@@ -155,82 +168,50 @@ int lad(pdo_cgrid h, hipStream_t st)
     const double dx2 = dx * dx, dy2 = dy * dy, dz2 = dz * dz;
     const double dx4 = dx2 * dx2, dy4 = dy2 * dy2, dz4 = dz2 * dz2;
     const long n = h->n;
-    // artificial shear viscosity
-    {
-        CgArgs a;
-        a.in[0] = h->f(F_G);
-        a.out[0] = h->f(F_FUNC);
-        a.n = n;
-        PDO_TRY(cg(h, CG_SHEAR, a, st));
-    }
-    PDO_TRY(fourth(h, h->f(F_FUNC), st));
-    {
-        CgArgs a;
-        a.in[0] = h->f(F_D4);
-        a.in[1] = h->f(F_D4 + 1);
-        a.in[2] = h->f(F_D4 + 2);
-        a.in[3] = h->f(F_PRIM);
-        a.out[0] = h->f(F_STAR);
-        a.n = n;
-        a.c[0] = p.Cmu;
-        a.c[1] = dx4 * dx2;
-        a.c[2] = dy4 * dy2;
-        a.c[3] = dz4 * dz2;
-        PDO_TRY(cg(h, CG_MUSTAR, a, st));
-    }
-    PDO_TRY(filter3(h, h->gfil, h->f(F_STAR), 2, st));
-    // artificial bulk viscosity
-    {
-        CgArgs a;
-        a.in[0] = h->f(F_G);
-        a.out[0] = h->f(F_FUNC);
-        a.n = n;
-        PDO_TRY(cg(h, CG_DILATATION, a, st));
-    }
-    PDO_TRY(gradient(h, h->f(F_PRIM), h->f(F_R), -1, st));
-    PDO_TRY(fourth(h, h->f(F_FUNC), st));
-    {
-        CgArgs a;
-        a.in[0] = h->f(F_D4);
-        a.in[1] = h->f(F_D4 + 1);
-        a.in[2] = h->f(F_D4 + 2);
-        a.in[3] = h->f(F_R);
-        a.in[4] = h->f(F_G);
-        a.in[5] = h->f(F_FUNC);
-        a.in[6] = h->f(F_PRIM);
-        a.out[0] = h->f(F_STAR + 1);
-        a.n = n;
-        const double c[7] = {p.Cbeta, dx, dy, dz, dx4, dy4, dz4};
-        for (int i = 0; i < 7; i++) a.c[i] = c[i];
-        PDO_TRY(cg(h, CG_BULKSTAR, a, st));
-    }
-    PDO_TRY(filter3(h, h->gfil, h->f(F_STAR + 1), 2, st));
-    // artificial conductivity
-    PDO_TRY(gradient(h, h->f(F_PRIM + 4), h->f(F_R), -1, st));
-    PDO_TRY(fourth(h, h->f(F_PRIM + 4), st));
-    {
-        CgArgs a;
-        a.in[0] = h->f(F_D4);
-        a.in[1] = h->f(F_D4 + 1);
-        a.in[2] = h->f(F_D4 + 2);
-        a.in[3] = h->f(F_R);
-        a.in[4] = h->f(F_PRIM);
-        a.out[0] = h->f(F_STAR + 2);
-        a.n = n;
-        const double c[8] = {p.Ckap, p.gam, dx, dy, dz, dx4, dy4, dz4};
-        for (int i = 0; i < 8; i++) a.c[i] = c[i];
-        PDO_TRY(cg(h, CG_KAPSTAR, a, st));
-    }
-    PDO_TRY(filter3(h, h->gfil, h->f(F_STAR + 2), 2, st));
     CgArgs a;
-    a.out[0] = h->f(F_MU);
-    a.out[1] = h->f(F_MU + 1);
-    a.out[2] = h->f(F_MU + 2);
-    a.in[0] = h->f(F_STAR);
-    a.in[1] = h->f(F_STAR + 1);
-    a.in[2] = h->f(F_STAR + 2);
+    a.in[0] = h->f(F_G);
+    a.out[0] = h->f(F_FUNC);
+    a.out[1] = h->f(F_DIL);
     a.n = n;
-    return cg(h, CG_ADD3, a, st);
+    PDO_TRY(cg(h, CG_STRAIN, a, st));
+    PDO_TRY(gradient(h, h->f(F_PRIM), h->f(F_DRHO), -1, st));
+    PDO_TRY(gradient(h, h->f(F_PRIM + 4), h->f(F_DE), -1, st));
+    const void *const func[3] = {h->f(F_FUNC), h->f(F_DIL), h->f(F_PRIM + 4)};
+    auto star = [&](int k) -> int {
+        CgArgs c;
+        for (int d = 0; d < 3; d++) c.in[d] = h->f(F_D4 + 3 * k + d);
+        c.out[0] = h->f(F_STAR + k);
+        c.n = n;
+        if (k == 0) {
+            c.in[3] = h->f(F_PRIM);
+            const double v[4] = {p.Cmu, dx4 * dx2, dy4 * dy2, dz4 * dz2};
+            for (int i = 0; i < 4; i++) c.c[i] = v[i];
+            return cg(h, CG_MUSTAR, c, st);
+        }
+        if (k == 1) {
+            c.in[3] = h->f(F_DRHO);
+            c.in[4] = h->f(F_G);
+            c.in[5] = h->f(F_DIL);
+            c.in[6] = h->f(F_PRIM);
+            const double v[7] = {p.Cbeta, dx, dy, dz, dx4, dy4, dz4};
+            for (int i = 0; i < 7; i++) c.c[i] = v[i];
+            return cg(h, CG_BULKSTAR, c, st);
+        }
+        c.in[3] = h->f(F_DE);
+        c.in[4] = h->f(F_PRIM);
+        const double v[8] = {p.Ckap, p.gam, dx, dy, dz, dx4, dy4, dz4};
+        for (int i = 0; i < 8; i++) c.c[i] = v[i];
+        return cg(h, CG_KAPSTAR, c, st);
+    };
+    // one coefficient after the other: a pass finds what the last one wrote
+    // in the Infinity Cache
+    for (int k = 0; k < 3; k++) {
+        PDO_TRY(fourth(h, func, k, k + 1, st));
+        PDO_TRY(star(k));
+        void *s = h->f(F_STAR + k);
+        PDO_TRY(filter3(h, h->gfil, &s, 1, 2, st));
+    }
+    return 0;
 }
 
 }  // namespace
@@ -285,13 +266,19 @@ int pdo_cgrid_rhs(pdo_cgrid h, int prec, const void *Wc, void *rhs, void *stream
     }
     // velocity gradients: u with -x_bc, v with -y_bc, w with -z_bc
     for (int c = 0; c < 3; c++) PDO_TRY(gradient(h, h->f(F_PRIM + 1 + c), h->f(F_G + 3 * c), c, st));
-    // transport properties, then the artificial ones
+    PDO_TRY(lad(h, st));
+    // transport properties, tau, q and the fluxes along every direction
     {
         CgArgs a;
-        a.in[0] = h->f(F_PRIM + 6);
+        a.in[0] = Wc;
+        a.in[1] = h->f(F_PRIM);
+        a.in[2] = h->f(F_G);
+        a.in[3] = h->f(F_STAR);
+        a.in[4] = h->f(F_DE);
         a.out[0] = h->f(F_MU);
-        a.out[1] = h->f(F_MU + 1);
-        a.out[2] = h->f(F_MU + 2);
+        a.out[1] = h->f(F_TAU);
+        a.out[2] = h->f(F_Q);
+        a.out[3] = h->f(F_FLUX);
         a.n = n;
         a.i0 = p.inviscid;
         a.c[0] = p.mu_ref;
@@ -299,52 +286,21 @@ int pdo_cgrid_rhs(pdo_cgrid h, int prec, const void *Wc, void *rhs, void *stream
         a.c[2] = p.visc_n;
         a.c[3] = p.gam * p.Rgas * (1.0 / (p.gam - 1.0));
         a.c[4] = p.Pr;
-        PDO_TRY(cg(h, CG_TRANSPORT, a, st));
-    }
-    PDO_TRY(lad(h, st));
-    // tau and q
-    {
-        CgArgs a;
-        a.in[0] = h->f(F_G);
-        a.in[1] = h->f(F_MU);
-        a.in[2] = h->f(F_MU + 1);
-        a.out[0] = h->f(F_TAU);
-        a.n = n;
-        PDO_TRY(cg(h, CG_TAU, a, st));
-    }
-    for (int d = 0; d < 3; d++) {
-        const int *b = bc_of(h, d);
-        PDO_TRY(dd(h, d, h->f(F_PRIM + 6), h->f(F_T1), b[0], b[1], st));
-        CgArgs a;
-        a.in[0] = h->f(F_MU + 2);
-        a.in[1] = h->f(F_T1);
-        a.out[0] = h->f(F_Q + d);
-        a.n = n;
-        PDO_TRY(cg(h, CG_NEGMUL, a, st));
+        a.c[5] = (p.gam - 1.0) * (1.0 / p.Rgas);
+        PDO_TRY(cg(h, CG_FLUXES, a, st));
     }
     // rhs = -sum_d d/dx_d (fluxes along d): symmetric ends for the momentum
     // along d, antisymmetric for the others
     for (int d = 0; d < 3; d++) {
-        CgArgs a;
-        a.in[0] = Wc;
-        a.in[1] = h->f(F_PRIM);
-        a.in[2] = h->f(F_TAU);
-        a.in[3] = h->f(F_Q);
-        a.out[0] = h->f(F_FLUX);
-        a.n = n;
-        a.i0 = d;
-        PDO_TRY(cg(h, CG_FLUXES, a, st));
         const int *b = bc_of(h, d);
         for (int c = 0; c < 5; c++) {
             const int sg = c == 1 + d ? 1 : -1;
-            PDO_TRY(dd(h, d, h->f(F_FLUX + c), h->f(F_DFLUX + c), sg * b[0], sg * b[1], st));
+            void *r = (char *)rhs + (size_t)c * n * h->W;
+            // the mass flux is the momentum
+            const void *f = c == 0 ? (const char *)Wc + (size_t)(1 + d) * n * h->W : h->f(F_FLUX + 4 * d + c - 1);
+            PDO_TRY(derivatives_subtract(h->der, d, h->prec, f, r, d == 0, sg * b[0], sg * b[1],
+                                         h->f(F_STAR), st));
         }
-        CgArgs s;
-        s.in[0] = h->f(F_DFLUX);
-        s.out[0] = rhs;
-        s.n = n;
-        s.i0 = d == 0;
-        PDO_TRY(cg(h, CG_SUB5, s, st));
     }
     return 0;
 }
@@ -353,7 +309,7 @@ int pdo_cgrid_filter(pdo_cgrid h, int prec, void *arr, int numtimes, int gaussia
 {
     if (!h || !arr || numtimes < 1) { set_error("invalid argument"); return PDO_ERR_ARG; }
     if (prec != h->prec) { set_error("cgrid: the object's work buffers were sized for another precision"); return PDO_ERR_ARG; }
-    return filter3(h, gaussian ? h->gfil : h->fil, arr, numtimes, (hipStream_t)stream);
+    return filter3(h, gaussian ? h->gfil : h->fil, &arr, 1, numtimes, (hipStream_t)stream);
 }
 
 int pdo_cgrid_field(pdo_cgrid h, int which, const void **ptr)

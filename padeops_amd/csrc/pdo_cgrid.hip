@@ -40,30 +40,10 @@ __global__ void __launch_bounds__(256) k_primitive(const TS *W, TS *prim, long n
     }
 }
 
-// get_transport_properties, one species (MixtureEOS.F90:175-203) with the
-// power law (PowerLawViscosity.F90:46-76): mu, bulk = 0, kappa = Cp mu / Pr;
-// all zero when inviscid
+// getLAD (cgrid.F90:1081-1084, 1116): the strain-rate magnitude and the
+// dilatation of the gradients g (9 fields n apart, du_i/dx_j at 3 i + j)
 template <typename TS>
-__global__ void __launch_bounds__(256) k_transport(const TS *T, TS *mu, TS *bulk, TS *kap, long n, int inviscid,
-                                                  double mu_ref, double T_ref, double vn, double Cp, double Pr)
-{
-    PDO_CG_LOOP(n)
-    {
-        double m = 0, k = 0;
-        if (!inviscid) {
-            m = mu_ref * pow(ld(T, t) / T_ref, vn);
-            k = Cp * m / Pr;
-        }
-        mu[t] = (TS)m;
-        bulk[t] = (TS)0;
-        kap[t] = (TS)k;
-    }
-}
-
-// getLAD (cgrid.F90:1081-1084): the strain-rate magnitude of the gradients g
-// (9 fields n apart, du_i/dx_j at 3 i + j)
-template <typename TS>
-__global__ void __launch_bounds__(256) k_shear_func(const TS *g, TS *func, long n)
+__global__ void __launch_bounds__(256) k_strain(const TS *g, TS *func, TS *dil, long n)
 {
     PDO_CG_LOOP(n)
     {
@@ -72,14 +52,8 @@ __global__ void __launch_bounds__(256) k_shear_func(const TS *g, TS *func, long 
         for (int c = 0; c < 9; ++c) d[c] = ld(g, t + c * n);
         const double a = d[3] + d[1], b = d[6] + d[2], c = d[7] + d[5];
         func[t] = (TS)sqrt(d[0] * d[0] + 0.5 * a * a + 0.5 * b * b + d[4] * d[4] + 0.5 * c * c + d[8] * d[8]);
+        dil[t] = (TS)(d[0] + d[4] + d[8]);
     }
-}
-
-// dilatation dudx + dvdy + dwdz (:1116)
-template <typename TS>
-__global__ void __launch_bounds__(256) k_dilatation(const TS *g, TS *func, long n)
-{
-    PDO_CG_LOOP(n) func[t] = (TS)(ld(g, t) + ld(g, t + 4 * n) + ld(g, t + 8 * n));
 }
 
 // mustar = Cmu rho |X dx^6 + Z dz^6 + Y dy^6| (:1086-1110), X, Y, Z the
@@ -148,83 +122,70 @@ __global__ void __launch_bounds__(256) k_kapstar(const TS *X, const TS *Y, const
     }
 }
 
-// mu += mustar, bulk += bulkstar, kap += kapstar (:1251-1255)
+// Everything between the artificial coefficients and the flux derivatives in
+// one pass: get_transport_properties (MixtureEOS.F90:175-203 with the power
+// law, PowerLawViscosity.F90:46-76; mu = 0 = kappa when inviscid, Cp mu / Pr
+// otherwise) plus the artificial coefficients (cgrid.F90:1251-1255), get_tau
+// (:1360-1404; xx, xy, xz, yy, yz, zz), get_q (:1406-1452; dT = dTde de, T
+// being proportional to e) and the fluxes along each direction d
+// (getRHS_x/y/z :896-1056):
+//   momentum rho u_d u_i + p delta_id - tau_id;
+//   energy (TE + p - tau_dd) u_d - sum_{i != d} u_i tau_id + q_d
+// (that of mass is the momentum itself).  Bound by HBM: 25 words read and 24
+// written per point, where the steps one by one moved 88.
+// flux may overlie anything but the inputs.
 template <typename TS>
-__global__ void __launch_bounds__(256) k_add3(TS *mu, TS *bulk, TS *kap, const TS *ms, const TS *bs, const TS *ks,
-                                             long n)
+__global__ void __launch_bounds__(256) k_fluxes(const TS *W, const TS *prim, const TS *g, const TS *star, const TS *de,
+                                               TS *coef, TS *tau, TS *q, TS *flux, long n, int inviscid, double mu_ref,
+                                               double T_ref, double vn, double Cp, double Pr, double dTde)
 {
-    PDO_CG_LOOP(n)
-    {
-        mu[t] = (TS)(ld(mu, t) + ld(ms, t));
-        bulk[t] = (TS)(ld(bulk, t) + ld(bs, t));
-        kap[t] = (TS)(ld(kap, t) + ld(ks, t));
-    }
-}
-
-// get_tau (:1360-1404): tau = (xx, xy, xz, yy, yz, zz), n apart
-template <typename TS>
-__global__ void __launch_bounds__(256) k_tau(const TS *g, const TS *mu, const TS *bulk, TS *tau, long n)
-{
+    constexpr int TI[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
     PDO_CG_LOOP(n)
     {
         double d[9];
 #pragma unroll
         for (int c = 0; c < 9; ++c) d[c] = ld(g, t + c * n);
-        const double m = ld(mu, t), bk = ld(bulk, t);
-        const double bambda = (4.0 / 3.0) * m + bk, lam = bk - (2.0 / 3.0) * m;
-        tau[t] = (TS)(bambda * d[0] + lam * (d[4] + d[8]));
-        tau[t + n] = (TS)(m * (d[1] + d[3]));
-        tau[t + 2 * n] = (TS)(m * (d[2] + d[6]));
-        tau[t + 3 * n] = (TS)(bambda * d[4] + lam * (d[0] + d[8]));
-        tau[t + 4 * n] = (TS)(m * (d[5] + d[7]));
-        tau[t + 5 * n] = (TS)(bambda * d[8] + lam * (d[0] + d[4]));
-    }
-}
-
-// q = -kappa dT (get_q :1428-1444)
-template <typename TS>
-__global__ void __launch_bounds__(256) k_neg_mul(const TS *a, const TS *b, TS *out, long n)
-{
-    PDO_CG_LOOP(n) out[t] = (TS)(-ld(a, t) * ld(b, t));
-}
-
-// the five fluxes along direction dir (getRHS_x/y/z :896-1056):
-//   mass rho u_d; momentum rho u_d u_i + p delta_id - tau_id;
-//   energy (TE + p - tau_dd) u_d - sum_{i != d} u_i tau_id + q_d
-template <typename TS>
-__global__ void __launch_bounds__(256) k_fluxes(const TS *W, const TS *prim, const TS *tau, const TS *q, TS *flux,
-                                               long n, int dir)
-{
-    // tau component of (i, d), components xx xy xz yy yz zz
-    constexpr int TI[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
-    PDO_CG_LOOP(n)
-    {
-        const double m = ld(W, t + (1 + dir) * n);  // rho u_d
+        const double mom[3] = {ld(W, t + n), ld(W, t + 2 * n), ld(W, t + 3 * n)}, TE = ld(W, t + 4 * n);
         const double vel[3] = {ld(prim, t + n), ld(prim, t + 2 * n), ld(prim, t + 3 * n)};
-        const double p = ld(prim, t + 5 * n);
-        double ti[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) ti[i] = ld(tau, t + TI[i][dir] * n);
-        flux[t] = (TS)m;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            double f = m * vel[i];
-            if (i == dir) f = f + p;
-            flux[t + (1 + i) * n] = (TS)(f - ti[i]);
+        const double p = ld(prim, t + 5 * n), T = ld(prim, t + 6 * n);
+        const double ms = ld(star, t), bs = ld(star, t + n), ks = ld(star, t + 2 * n);
+        const double dT[3] = {dTde * ld(de, t), dTde * ld(de, t + n), dTde * ld(de, t + 2 * n)};
+        double mu = 0, kap = 0;
+        if (!inviscid) {
+            mu = mu_ref * pow(T / T_ref, vn);
+            kap = Cp * mu / Pr;
         }
-        double E = (ld(W, t + 4 * n) + p - ti[dir]) * vel[dir];
+        mu += ms;
+        kap += ks;
+        coef[t] = (TS)mu;
+        coef[t + n] = (TS)bs;
+        coef[t + 2 * n] = (TS)kap;
+        const double bambda = (4.0 / 3.0) * mu + bs, lam = bs - (2.0 / 3.0) * mu;
+        double ts[6];
+        ts[0] = bambda * d[0] + lam * (d[4] + d[8]);
+        ts[1] = mu * (d[1] + d[3]);
+        ts[2] = mu * (d[2] + d[6]);
+        ts[3] = bambda * d[4] + lam * (d[0] + d[8]);
+        ts[4] = mu * (d[5] + d[7]);
+        ts[5] = bambda * d[8] + lam * (d[0] + d[4]);
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
-            if (i != dir) E = E - vel[i] * ti[i];
-        flux[t + 4 * n] = (TS)(E + ld(q, t + dir * n));
+        for (int c = 0; c < 6; ++c) tau[t + c * n] = (TS)ts[c];
+#pragma unroll
+        for (int dir = 0; dir < 3; ++dir) {
+            const double qd = -kap * dT[dir];
+            q[t + dir * n] = (TS)qd;
+            TS *F = flux + 4 * dir * n;
+            double E = (TE + p - ts[TI[dir][dir]]) * vel[dir];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                double f = mom[dir] * vel[i];
+                if (i == dir) f = f + p;
+                else E = E - vel[i] * ts[TI[i][dir]];
+                F[t + i * n] = (TS)(f - ts[TI[i][dir]]);
+            }
+            F[t + 3 * n] = (TS)(E + qd);
+        }
     }
-}
-
-// rhs -= d (five fields n apart), or rhs = -d when first
-template <typename TS>
-__global__ void __launch_bounds__(256) k_sub5(TS *rhs, const TS *d, long n5, int first)
-{
-    PDO_CG_LOOP(n5) rhs[t] = (TS)((first ? 0.0 : ld(rhs, t)) - ld(d, t));
 }
 
 template <typename TS>
@@ -241,20 +202,13 @@ template <typename TS> const TS *C(const void *p) { return (const TS *)p; }
 template <typename TS>
 hipError_t pointwise_t(CgOp op, const CgArgs &a, hipStream_t st)
 {
-    const dim3 g(grid_of(op == CG_SUB5 ? 5 * a.n : a.n)), b(256);
+    const dim3 g(grid_of(a.n)), b(256);
     switch (op) {
     case CG_PRIMITIVE:
         hipLaunchKernelGGL((k_primitive<TS>), g, b, 0, st, C<TS>(a.in[0]), P<TS>(a.out[0]), a.n, a.c[0], a.c[1]);
         break;
-    case CG_TRANSPORT:
-        hipLaunchKernelGGL((k_transport<TS>), g, b, 0, st, C<TS>(a.in[0]), P<TS>(a.out[0]), P<TS>(a.out[1]),
-                           P<TS>(a.out[2]), a.n, a.i0, a.c[0], a.c[1], a.c[2], a.c[3], a.c[4]);
-        break;
-    case CG_SHEAR:
-        hipLaunchKernelGGL((k_shear_func<TS>), g, b, 0, st, C<TS>(a.in[0]), P<TS>(a.out[0]), a.n);
-        break;
-    case CG_DILATATION:
-        hipLaunchKernelGGL((k_dilatation<TS>), g, b, 0, st, C<TS>(a.in[0]), P<TS>(a.out[0]), a.n);
+    case CG_STRAIN:
+        hipLaunchKernelGGL((k_strain<TS>), g, b, 0, st, C<TS>(a.in[0]), P<TS>(a.out[0]), P<TS>(a.out[1]), a.n);
         break;
     case CG_MUSTAR:
         hipLaunchKernelGGL((k_mustar<TS>), g, b, 0, st, C<TS>(a.in[0]), C<TS>(a.in[1]), C<TS>(a.in[2]),
@@ -270,23 +224,10 @@ hipError_t pointwise_t(CgOp op, const CgArgs &a, hipStream_t st)
                            C<TS>(a.in[3]), C<TS>(a.in[4]), P<TS>(a.out[0]), a.n, a.c[0], a.c[1], a.c[2], a.c[3],
                            a.c[4], a.c[5], a.c[6], a.c[7]);
         break;
-    case CG_ADD3:
-        hipLaunchKernelGGL((k_add3<TS>), g, b, 0, st, P<TS>(a.out[0]), P<TS>(a.out[1]), P<TS>(a.out[2]),
-                           C<TS>(a.in[0]), C<TS>(a.in[1]), C<TS>(a.in[2]), a.n);
-        break;
-    case CG_TAU:
-        hipLaunchKernelGGL((k_tau<TS>), g, b, 0, st, C<TS>(a.in[0]), C<TS>(a.in[1]), C<TS>(a.in[2]),
-                           P<TS>(a.out[0]), a.n);
-        break;
-    case CG_NEGMUL:
-        hipLaunchKernelGGL((k_neg_mul<TS>), g, b, 0, st, C<TS>(a.in[0]), C<TS>(a.in[1]), P<TS>(a.out[0]), a.n);
-        break;
     case CG_FLUXES:
         hipLaunchKernelGGL((k_fluxes<TS>), g, b, 0, st, C<TS>(a.in[0]), C<TS>(a.in[1]), C<TS>(a.in[2]),
-                           C<TS>(a.in[3]), P<TS>(a.out[0]), a.n, a.i0);
-        break;
-    case CG_SUB5:
-        hipLaunchKernelGGL((k_sub5<TS>), g, b, 0, st, P<TS>(a.out[0]), C<TS>(a.in[0]), 5 * a.n, a.i0);
+                           C<TS>(a.in[3]), C<TS>(a.in[4]), P<TS>(a.out[0]), P<TS>(a.out[1]), P<TS>(a.out[2]),
+                           P<TS>(a.out[3]), a.n, a.i0, a.c[0], a.c[1], a.c[2], a.c[3], a.c[4], a.c[5]);
         break;
     case CG_COPY:
         hipLaunchKernelGGL((k_copy<TS>), g, b, 0, st, C<TS>(a.in[0]), P<TS>(a.out[0]), a.n);

@@ -4,32 +4,35 @@
 
 #include <hip/hip_runtime.h>
 
+#include "../../include/padeops_hip.h"
+
 namespace pdo {
 
 enum CgOp {
     CG_PRIMITIVE,   // in W; out prim (7 fields); c: gam - 1, 1 / Rgas
-    CG_TRANSPORT,   // in T; out mu, bulk, kap; i0 inviscid; c: mu_ref, T_ref, n, Cp, Pr
-    CG_SHEAR,       // in g (9 fields); out func
-    CG_DILATATION,  // in g; out func
+    CG_STRAIN,      // in g (9 fields); out strain-rate magnitude, dilatation
     CG_MUSTAR,      // in X, Y, Z, rho; out; c: Cmu, dx^6, dy^6, dz^6
     CG_BULKSTAR,    // in X, Y, Z, grad rho (3), g, dil, rho; out; c: Cbeta, dx, dy, dz, dx^4, dy^4, dz^4
     CG_KAPSTAR,     // in X, Y, Z, grad e (3), prim; out; c: Ckap, gam, dx, dy, dz, dx^4, dy^4, dz^4
-    CG_ADD3,        // out mu, bulk, kap += in mustar, bulkstar, kapstar
-    CG_TAU,         // in g, mu, bulk; out tau (6 fields)
-    CG_NEGMUL,      // out = -in0 in1
-    CG_FLUXES,      // in W, prim, tau, q (3 fields); out 5 fluxes; i0 direction
-    CG_SUB5,        // out (5 fields) -= in (5 fields); i0: first (out = -in)
+    CG_FLUXES,      // in W, prim, g, star (3), grad e (3); out mu/bulk/kap (3), tau (6), q (3), fluxes (12: 4
+                    // per direction); i0 inviscid; c: mu_ref, T_ref, n, Cp, Pr, dT/de
     CG_COPY,        // out = in
 };
 
 struct CgArgs {
     const void *in[8] = {};
-    void *out[3] = {};
+    void *out[4] = {};
     long n = 0;  // points per field
     int i0 = 0;
     double c[8] = {};
 };
 
 hipError_t launch_cgrid(bool dbl, CgOp op, const CgArgs &a, hipStream_t st);
+
+// of the derivatives and filters objects (pdo_dispatch.cpp)
+int derivatives_subtract(pdo_derivatives h, int d, int prec, const void *f, void *out, bool first, int bc1, int bcn,
+                         void *work, hipStream_t st);
+bool filters_twice(pdo_filters h, int d, int prec);
+int filters_apply_twice(pdo_filters h, int d, int prec, const void *f, void *ff, int bc1, int bcn, hipStream_t st);
 
 }  // namespace pdo

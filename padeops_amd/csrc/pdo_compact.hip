@@ -396,7 +396,10 @@ __device__ __forceinline__ void strided_store(const ApplyArgs &A, const typename
 #pragma unroll
         for (int j0 = 0; j0 < MM; j0 += CH) {
             TS av[CH];
-            if (far) {
+            if (A.epi == 3) {
+#pragma unroll
+                for (int j = 0; j < CH; ++j) av[j] = TS(0);
+            } else if (far) {
 #pragma unroll
                 for (int j = 0; j < CH; ++j) av[j] = buf_ld<TS>(ra, vo + (unsigned)(j0 + j) * ss, 0u);
             } else {
@@ -426,7 +429,7 @@ __device__ __forceinline__ void strided_store(const ApplyArgs &A, const typename
         const unsigned off = (unsigned)A.n_sys * ss;
         TC v = d[0];
         if (EPI) {
-            const TC av = (TC)buf_ld<TS>(ra, vo, off);
+            const TC av = A.epi == 3 ? TC(0) : (TC)buf_ld<TS>(ra, vo, off);
             v = A.epi == 1 ? av + v : av - v;
         }
         buf_st((TS)v, ro, vo, off);
@@ -678,7 +681,8 @@ __device__ __forceinline__ void xdir_store(const ApplyArgs &A, typename Mode<MOD
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int v = tid + i * 256;
-            if (v < nvec) ops[i] = reinterpret_cast<const V *>(aux)[v];
+            if (A.epi == 3) ops[i] = V{};
+            else if (v < nvec) ops[i] = reinterpret_cast<const V *>(aux)[v];
         }
     }
 #pragma unroll
@@ -829,6 +833,7 @@ __global__ void __launch_bounds__(256) k_general(ApplyArgs A, double *scratch)
         const long idx = po + (long)i * A.se_out;
         if (A.epi == 1) v = (double)aux[idx] + v;
         else if (A.epi == 2) v = (double)aux[idx] - v;
+        else if (A.epi == 3) v = -v;
         out[idx] = (TS)v;
     }
     if (A.n_out > n) {
@@ -836,6 +841,7 @@ __global__ void __launch_bounds__(256) k_general(ApplyArgs A, double *scratch)
         double v = first;
         if (A.epi == 1) v = (double)aux[idx] + v;
         else if (A.epi == 2) v = (double)aux[idx] - v;
+        else if (A.epi == 3) v = -v;
         out[idx] = (TS)v;
     }
 }
@@ -874,9 +880,10 @@ static hipError_t launch_strided_k(const ApplyArgs &A, hipStream_t st)
 // staggered operators (tridiagonal families)
 template <int FAM> constexpr bool has_extra_row() { return Fam<FAM>::K == 1; }
 
-// epilogue operands (divergence accumulation, projection subtraction) are
-// only used with the periodic cd06 first derivative
-template <int FAM> constexpr bool has_epilogue() { return FAM == 0; }
+// epilogue operands (divergence accumulation, projection subtraction, the sum
+// of flux derivatives) are only used with the periodic first derivatives of
+// cd06 and cd10
+template <int FAM> constexpr bool has_epilogue() { return FAM == 0 || FAM == 2; }
 
 // pencils per workgroup of the periodic strided kernel: 32 (two segments per
 // wave) or 64 (one); tuning constant

@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "../../include/padeops_hip.h"
+#include "pdo_cgrid.hpp"
 #include "pdo_explicit.hpp"
 #include "pdo_fft.hpp"
 #include "pdo_kernels.hpp"
@@ -229,6 +230,45 @@ struct pdo_derivatives_s : public pdo::DerivativesObject {};
 struct pdo_filters_s : public pdo::FiltersObject {};
 
 using namespace pdo;
+
+namespace pdo {
+
+// out -= df/dx_d (first: out = -df/dx_d); work holds one field
+int derivatives_subtract(pdo_derivatives h, int d, int prec, const void *f, void *out, bool first, int bc1, int bcn,
+                         void *work, hipStream_t st)
+{
+    int na, nb, r;
+    h->pencils(d, na, nb);
+    if (h->n_of(d) > 1 && (h->method[d] == METHOD_CD10 || h->method[d] == METHOD_CD06)) {
+        if (h->method[d] == METHOD_CD06) bc1 = bcn = 0;
+        return apply(h->op[d], KIND_D1, bc1, bcn, d + 1, prec, f, out, na, nb, st, first ? 3 : 2, out);
+    }
+    const long N = (long)h->nx * h->ny * h->nz;
+    const bool dbl = prec == PDO_F64;
+    if (first) {
+        const hipError_t e = launch_zero_words(out, N * (dbl ? 2 : 1), st);
+        if (e != hipSuccess) return hip_fail(e, "zero fill");
+    }
+    if (h->n_of(d) == 1) return 0;
+    if ((r = h->apply(d, 1, prec, f, work, bc1, bcn, st))) return r;
+    const hipError_t e = launch_axpy(dbl, out, out, work, -1.0, N, st);
+    return e == hipSuccess ? 0 : hip_fail(e, "derivative sum");
+}
+
+// whether one pass along d can apply the filter twice, and that pass
+bool filters_twice(pdo_filters h, int d, int prec)
+{
+    if (h->method[d] == FIL_CF90 || prec_mode(prec) < 0) return false;
+    return xfilter_can_twice(h->xf[d], d + 1);
+}
+int filters_apply_twice(pdo_filters h, int d, int prec, const void *f, void *ff, int bc1, int bcn, hipStream_t st)
+{
+    int na, nb;
+    h->pencils(d, na, nb);
+    return xfilter_twice(h->xf[d], d + 1, prec, f, ff, na, nb, bc1, bcn, st);
+}
+
+}  // namespace pdo
 
 static size_t word_of(int prec) { return prec == PDO_F64 ? 8 : 4; }
 

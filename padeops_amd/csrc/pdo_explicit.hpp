@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "../../include/padeops_hip.h"
+
 namespace pdo {
 
 constexpr int EXPL_R = 4;   // stencil half-width
@@ -18,7 +20,14 @@ struct ExplicitArgs {
     double right[EXPL_NB * EXPL_WB];      // rows n-4..n-1 against points n-8..n-1
 };
 
-hipError_t launch_explicit(bool dbl, const ExplicitArgs &E, const void *f, void *out, hipStream_t st);
+// the filter applied `times` (1, or 2 where explicit_twice) times
+hipError_t launch_explicit(bool dbl, const ExplicitArgs &E, const void *f, void *out, hipStream_t st, int times = 1);
+bool explicit_twice(const ExplicitArgs &E);
+// two applications of an explicit filter along dir in one pass, where
+// xfilter_can_twice
+bool xfilter_can_twice(pdo_xfilter h, int dir);
+int xfilter_twice(pdo_xfilter h, int dir, int prec, const void *f, void *fil, long na, long nb, int bc1, int bcn,
+                  hipStream_t st);
 // out = a + s b, elementwise over n values (FP64 arithmetic)
 hipError_t launch_axpy(bool dbl, void *out, const void *a, const void *b, double s, long n, hipStream_t st);
 

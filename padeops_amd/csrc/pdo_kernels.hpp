@@ -19,7 +19,7 @@ constexpr int OVL_PMAX = 32;  // most overlapping segments per pencil (n <= 1024
 struct ApplyArgs {
     const void *f;
     void *out;
-    const void *aux;   // epilogue operand (epi 1: out = aux + y, 2: out = aux - y)
+    const void *aux;   // epilogue operand (epi 1: out = aux + y, 2: out = aux - y, 3: out = -y)
     int epi;
     int periodic;
     long na, nb;

@@ -199,7 +199,7 @@ static int prepare(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, 
     }
     mode = prec_mode(prec);
     if (mode < 0) { set_error("unknown precision mode"); return PDO_ERR_ARG; }
-    if (epi && !aux) { set_error("epilogue without operand"); return PDO_ERR_ARG; }
+    if ((epi == 1 || epi == 2) && !aux) { set_error("epilogue without operand"); return PDO_ERR_ARG; }
     if (na == 0 || nb == 0) { *empty = true; return 0; }
     Variant *v = nullptr;
     int st = 0;
@@ -240,7 +240,8 @@ static int prepare(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, 
     // segments, where they fit (n >= 16, at most 512 rows, 1024 of the
     // collocated operators), else one lane per pencil
     scratch_elems = (shape == SHAPE_GENERAL) ? (size_t)s.n_sys * (size_t)(na * nb) : 0;
-    if (shape == SHAPE_GENERAL && force_shape != SHAPE_GENERAL && !epi && overlap_fits(*v, dir, na, nb, word))
+    if (shape == SHAPE_GENERAL && force_shape != SHAPE_GENERAL && (!epi || s.n_out == s.n_sys) &&
+        overlap_fits(*v, dir, na, nb, word))
         shape = dir == 1 ? SHAPE_OVL_X : SHAPE_OVL_STRIDED;
     // FP32 + refinement without periodicity: the refined kernels carry two
     // solves and closure rows in up to 149 registers and scratch, the

@@ -57,7 +57,7 @@ struct OpObject {
 
 // Apply one variant along dir (1 x, 2 y, 3 z) of a field whose pencil count
 // is na*nb, optionally fused with an epilogue: epi 1 out = aux + y,
-// epi 2 out = aux - y.
+// epi 2 out = aux - y, epi 3 out = -y.
 int apply(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, const void *f, void *out, long na, long nb,
           hipStream_t stream, int epi = 0, const void *aux = nullptr, int force_shape = -1);
 

@@ -287,6 +287,24 @@ __global__ void __launch_bounds__(1024) k_ovl_strided(ApplyArgs A)
     if (!act) return;
     const unsigned vo = (a + b * (unsigned)A.sb_out) * (unsigned)sizeof(TS);
     char *ob = (char *)A.out + (size_t)blockIdx.y * A.sb_out * sizeof(TS);
+    if (A.epi) {
+        // the operand's rows in chunks, read before the chunk's rows are
+        // written (it may be the output)
+        const char *xb = (const char *)A.aux + (size_t)blockIdx.y * A.sb_out * sizeof(TS);
+        constexpr int CH = 8;
+#pragma unroll
+        for (int j0 = 0; j0 < M; j0 += CH) {
+            double x[CH];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                x[j] = 0.0;
+                if (A.epi != 3 && j0 + j < own)
+                    x[j] = (double)*(const TS *)(xb + (size_t)(r0 + j0 + j) * A.se_out * sizeof(TS) + vo);
+            }
+#pragma unroll
+            for (int j = 0; j < CH; ++j) d[j0 + j] = A.epi == 1 ? x[j] + d[j0 + j] : x[j] - d[j0 + j];
+        }
+    }
     if constexpr (UNI) {
 #pragma unroll
         for (int j = 0; j < M; ++j)
@@ -359,11 +377,15 @@ __global__ void __launch_bounds__(512) k_ovl_x(ApplyArgs A, int TP, int LD, unsi
     for (int j = 0; j < M; ++j)
         if (j < own) line[r0 + j] = (TS)d[j];
     __syncthreads();
-    TS *__restrict__ out = (TS *)A.out + pen0 * n;
+    TS *out = (TS *)A.out + pen0 * n;
+    const TS *aux = (const TS *)A.aux + (A.epi == 1 || A.epi == 2 ? pen0 * n : 0);  // may be out
 #pragma unroll 8
     for (int e = threadIdx.x; e < total; e += nt) {
         const int q = (int)__umulhi((unsigned)e, magic);
-        out[e] = tile[e + (q & -pad)];
+        const TS y = tile[e + (q & -pad)];
+        out[e] = A.epi == 0 ? y
+                            : (A.epi == 1 ? (TS)((double)aux[e] + (double)y)
+                                          : (TS)((A.epi == 2 ? (double)aux[e] : 0.0) - (double)y));
     }
 }
 

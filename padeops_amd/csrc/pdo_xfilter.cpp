@@ -103,7 +103,7 @@ static void fill_args(const XFilterObject *h, int bc1, int bcn, ExplicitArgs &E)
 }
 
 static int xfilter_apply(pdo_xfilter h, int dir, int prec, const void *f, void *fil, long na, long nb, int bc1,
-                         int bcn, void *stream)
+                         int bcn, void *stream, int times = 1)
 {
     if (!h || !f || !fil || na < 0 || nb < 0) { set_error("invalid argument"); return PDO_ERR_ARG; }
     const int mode = prec_mode(prec);
@@ -131,9 +131,25 @@ static int xfilter_apply(pdo_xfilter h, int dir, int prec, const void *f, void *
     E.na = (int)na;
     E.nb = (int)nb;
     E.dir = dir;
-    hipError_t e = launch_explicit(dbl, E, f, fil, st);
+    hipError_t e = launch_explicit(dbl, E, f, fil, st, times);
     return e == hipSuccess ? 0 : hip_fail(e, "explicit filter launch");
 }
+
+namespace pdo {
+bool xfilter_can_twice(pdo_xfilter h, int dir)
+{
+    if (h->n == 1) return true;
+    ExplicitArgs E;
+    fill_args(h, 0, 0, E);
+    E.dir = dir;
+    return explicit_twice(E);
+}
+int xfilter_twice(pdo_xfilter h, int dir, int prec, const void *f, void *fil, long na, long nb, int bc1, int bcn,
+                  hipStream_t st)
+{
+    return xfilter_apply(h, dir, prec, f, fil, na, nb, bc1, bcn, (void *)st, 2);
+}
+}  // namespace pdo
 
 extern "C" {
 

@@ -1,0 +1,104 @@
+"""GPU: cgrid at the sizes where its kernels change over, against the oracle.
+
+Filters: the strided kernel gives a lane 16 rows of a pencil and shares the
+rows out evenly, the x kernel holds whole lines, and either applies the
+filter once or twice in a pass; other sizes take the general kernel, once per
+pass.  Right-hand side: flux derivatives are summed in the passes of the
+register, the overlapping-segment and the general kernels."""
+import numpy as np
+import pytest
+
+import oracle.explicit as X
+import padeops_amd as P
+from fields import from_dev, random_field, rel_l2, to_dev
+from oracle.cgrid import Cgrid
+
+pytestmark = pytest.mark.gpu
+
+D = (0.1, 0.13, 0.17)
+
+
+@pytest.mark.parametrize("periodic,bc", [(True, (0, 0)), (False, (0, 0)), (False, (1, -1)), (False, (-1, 1))])
+@pytest.mark.parametrize("n", [8, 9, 15, 16, 17, 23, 24, 25, 32, 33, 49, 100])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_filter_once_and_twice(cuda, axis, n, periodic, bc):
+    import torch
+    shape = [11, 9, 10]
+    shape[axis] = n
+    shape = tuple(shape)
+    per, bcs = [True] * 3, [(0, 0)] * 3
+    per[axis], bcs[axis] = periodic, bc
+    f = random_field(shape, seed=n + axis)
+    for kind in ("gaussian", "lstsq"):
+        cg = P.cgrid()
+        assert cg.init(shape, D, prec="f64", periodic=tuple(per), bc=tuple(bcs), filter=(kind,) * 3) == 0
+        for times in (1, 2, 3, 4):
+            ref = f
+            for ax in (1, 0, 2):
+                for _ in range(times):
+                    ref = X.filter_axis(ref, ax, kind, per[ax], *bcs[ax])
+            fd = to_dev(f, torch.float64, cuda)
+            assert cg.filter(fd, numtimes=times, gaussian=kind == "gaussian") == 0
+            torch.cuda.synchronize()
+            # 9-point sums with weights of at most 1 in magnitude, FP64
+            assert rel_l2(from_dev(fd, shape), ref) <= 1e-14 * 3 * times, (kind, times)
+
+
+@pytest.mark.parametrize("n", [4095, 4096, 4097, 6000])
+@pytest.mark.parametrize("prec", ["f64", "f32_refine"])
+def test_filter_long_lines(cuda, n, prec):
+    import torch
+    dt = torch.float64 if prec == "f64" else torch.float32
+    shape = (n, 3, 2)
+    for periodic in (True, False):
+        o = P.gaussian()
+        o.init(n, periodic)
+        ft = to_dev(random_field(shape, seed=n), dt, cuda)
+        out = torch.full_like(ft, float("nan"))
+        o.filter1(ft, out, 3, 2, *((0, 0) if periodic else (1, -1)), prec=prec)
+        torch.cuda.synchronize()
+        ref = X.filter_axis(from_dev(ft, shape), 0, "gaussian", periodic, *((0, 0) if periodic else (1, -1)))
+        assert rel_l2(from_dev(out, shape), ref) <= (1e-14 if prec == "f64" else 1e-7)
+
+
+def _state(shape):
+    """phases of no symmetry: no point has a zero density gradient, whose
+    direction the artificial bulk viscosity takes"""
+    x = list(np.meshgrid(*[2 * np.pi * (np.arange(s) + 0.37) / s for s in shape], indexing="ij"))
+    x[0] = x[0] + 0.3 * np.sin(x[1] + 0.7)
+    rho = 1.0 + 0.1 * np.sin(x[0] + 0.2) * np.cos(x[1] + 0.9) + 0.05 * np.cos(x[2] + 2 * x[1])
+    u, v, w = 0.3 * np.cos(x[1] + x[2] + 0.4), 0.2 * np.sin(x[0] - x[2]), 0.25 * np.sin(x[0] + 1) * np.cos(x[1])
+    p = 1.0 + 0.1 * np.cos(x[0] + x[1] + 0.6)
+    e = p / (0.4 * rho)
+    return np.stack([rho, rho * u, rho * v, rho * w, rho * (e + 0.5 * (u * u + v * v + w * w))], axis=-1)
+
+
+@pytest.mark.parametrize("periodic", [(True, True, True), (False, True, False), (False, False, False)])
+@pytest.mark.parametrize("shape", [(32, 64, 32), (33, 17, 20), (16, 40, 49), (12, 10, 14), (32, 36, 1)])
+def test_rhs(cuda, shape, periodic):
+    import torch
+    bc = tuple((0, 0) if q else (1, -1) for q in periodic)
+    kw = dict(periodic=periodic, bc=bc, inviscid=False, mu_ref=0.02, T_ref=0.9, visc_n=0.7, Pr=0.72)
+    W = _state(shape).astype(np.float32).astype(np.float64)
+    ref, parts = Cgrid(shape, D, **kw).rhs(W, parts=True)
+    for prec in ("f64", "f32_refine"):
+        dt = torch.float64 if prec == "f64" else torch.float32
+        cg = P.cgrid()
+        assert cg.init(shape, D, prec=prec, **kw) == 0
+        wd = to_dev(W, dt, cuda)
+        rhs = torch.full_like(wd, float("nan"))
+        for _ in range(2):  # the second call starts from the first one's sums
+            assert cg.getRHS(wd, rhs) == 0
+        torch.cuda.synchronize()
+        got = from_dev(rhs, shape + (5,))
+        for c in range(5):
+            err = np.sqrt(np.mean((got[..., c] - ref[..., c]) ** 2))
+            if prec == "f64":
+                assert err <= 1e-12 * np.sqrt(np.mean(ref[..., c] ** 2)), c
+            else:
+                # the fluxes, at most 1.5 and the stresses (large where a wall
+                # cuts the state), are stored to 2^-24 and a derivative lifts
+                # what is rounded by at most 2.6 / dx inside, up to 4 / dx in
+                # one-sided closure rows
+                top = 1.5 + np.abs(parts["tau"]).max() + np.abs(parts["q"]).max()
+                assert err <= 2.0 ** -24 * top * np.sqrt(sum((4.0 / d) ** 2 for d in D)), c
