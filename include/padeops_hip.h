@@ -590,7 +590,7 @@ int pdo_mlp_destroy(pdo_mlp h);
  * pdo_closure_loss: the training loss sum_b sum_c w_c (p_c - T_c)^2 / (9 B)
  *   of p = sum_n G_n T_n(A9) against T (B, 6), w = (1 2 2 1 2 1), and dL/dG
  *   (B, 6); loss (host) may be NULL (no synchronisation).
- * FP64 arithmetic per point; buffers X, G sized for max_points. */
+ * FP64 arithmetic per point. */
 int pdo_closure_create(pdo_closure *h, pdo_mlp net, long max_points);
 int pdo_closure_features(pdo_closure h, int prec, const void *duidxj, long npts, double dratio, float *X, float *A9,
                          void *stream);

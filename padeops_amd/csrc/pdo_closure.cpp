@@ -1,11 +1,11 @@
-// Learned SGS closure object behind the C ABI: the network (pdo_mlp), the
-// feature and output buffers of one field, and the reductions; kernels in
-// pdo_closure.hip.
+// Learned SGS closure object behind the C ABI: the network (pdo_mlp) and the
+// reductions' buffers; kernels in pdo_closure.hip.
 #include <cmath>
 #include <vector>
 
 #include "../../include/padeops_hip.h"
 #include "pdo_closure.hpp"
+#include "pdo_mlp.hpp"
 #include "pdo_ops.hpp"
 
 namespace pdo {
@@ -13,7 +13,6 @@ namespace pdo {
 struct ClosureObject {
     pdo_mlp net = nullptr;
     long max_points = 0;
-    float *X = nullptr, *G = nullptr;
     double *partial = nullptr, *sumsq = nullptr, *loss = nullptr;
     unsigned *nfall = nullptr;
     long nnorm = 0;       // points behind the current scale (sumsq)
@@ -54,8 +53,6 @@ int pdo_closure_create(pdo_closure *h, pdo_mlp net, long max_points)
     o->net = net;
     o->max_points = max_points;
     int st = 0;
-    if (!st) st = o->alloc(&o->X, (size_t)max_points * 10);
-    if (!st) st = o->alloc(&o->G, (size_t)max_points * 6);
     if (!st) st = o->alloc(&o->partial, 8192);
     if (!st) st = o->alloc(&o->sumsq, 1);
     if (!st) st = o->alloc(&o->loss, 1);
@@ -94,13 +91,11 @@ int pdo_closure_stress(pdo_closure h, int prec, const void *duidxj, long npts, d
         if ((rc = ok(launch_grad_sumsq(dbl, duidxj, npts, npts, h->partial, h->sumsq, st), "closure scale"))) return rc;
         h->nnorm = npts;
     }
-    if ((rc = ok(launch_closure_features(dbl, duidxj, npts, npts, h->sumsq, h->nnorm, dratio, h->X, nullptr, st),
-                 "closure features")))
-        return rc;
-    if ((rc = pdo_mlp_forward(h->net, h->X, h->G, npts, stream))) return rc;
-    h->fall_blocks = closure_blocks(npts);
-    return ok(launch_closure_stress(dbl, duidxj, npts, npts, h->sumsq, h->nnorm, delta * delta, h->G, which, fallback,
-                                    tau, npts, h->nfall, st),
+    const unsigned short *Wb;
+    const float *P;
+    mlp_params(h->net, &Wb, &P);
+    return ok(launch_closure_stress(dbl, duidxj, npts, npts, h->sumsq, h->nnorm, delta * delta, dratio, Wb, P, which,
+                                    fallback, tau, npts, h->nfall, &h->fall_blocks, st),
               "closure stress");
 }
 

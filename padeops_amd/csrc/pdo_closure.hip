@@ -20,7 +20,10 @@
 // FP32 roots and principal-strain trigonometry of the features.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "pdo_closure.hpp"
+#include "pdo_mlp_dev.hpp"
 
 namespace pdo {
 
@@ -71,14 +74,89 @@ __device__ __forceinline__ void strain_rotation(const TS *g, long t, long stride
         }
 }
 
+// strain s (11 12 13 22 23 33) and rotation w (r12, r13, r23) of a normalised
+// gradient
+struct Split {
+    double s[6], w[3];
+};
+__device__ __forceinline__ Split split_of(const double (&A)[9])
+{
+    const double t3 = (A[0] + A[4] + A[8]) / 3.0;
+    return {{A[0] - t3, 0.5 * (A[1] + A[3]), 0.5 * (A[2] + A[6]), A[4] - t3, 0.5 * (A[5] + A[7]), A[8] - t3},
+            {0.5 * (A[1] - A[3]), 0.5 * (A[2] - A[6]), 0.5 * (A[5] - A[7])}};
+}
+
+// trace of the product of two symmetric tensors
+__device__ __forceinline__ double tr2(const double (&x)[6], const double (&y)[6])
+{
+    return x[0] * y[0] + x[3] * y[3] + x[5] * y[5] + 2.0 * (x[1] * y[1] + x[2] * y[2] + x[4] * y[4]);
+}
+__device__ __forceinline__ void squares(const Split &q, double (&s2)[6], double (&r2)[6])
+{
+    const double(&s)[6] = q.s;
+    s2[0] = s[0] * s[0] + s[1] * s[1] + s[2] * s[2];
+    s2[1] = s[0] * s[1] + s[1] * s[3] + s[2] * s[4];
+    s2[2] = s[0] * s[2] + s[1] * s[4] + s[2] * s[5];
+    s2[3] = s[1] * s[1] + s[3] * s[3] + s[4] * s[4];
+    s2[4] = s[1] * s[2] + s[3] * s[4] + s[4] * s[5];
+    s2[5] = s[2] * s[2] + s[4] * s[4] + s[5] * s[5];
+    const double a = q.w[0], b = q.w[1], c = q.w[2];
+    r2[0] = -(a * a + b * b);
+    r2[1] = -(b * c);
+    r2[2] = a * c;
+    r2[3] = -(a * a + c * c);
+    r2[4] = -(a * b);
+    r2[5] = -(b * b + c * c);
+}
+// z = x y for symmetric x, y / x r for any x
+__device__ __forceinline__ void mul_ss(const double (&x)[6], const double (&y)[6], double (&z)[9])
+{
+    constexpr int I[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            z[3 * i + j] = x[I[i][0]] * y[I[0][j]] + x[I[i][1]] * y[I[1][j]] + x[I[i][2]] * y[I[2][j]];
+}
+template <class F> __device__ __forceinline__ void mul_r(F x, const double (&w)[3], double (&z)[9])
+{
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        z[3 * i] = -(x(i, 1) * w[0] + x(i, 2) * w[1]);
+        z[3 * i + 1] = x(i, 0) * w[0] - x(i, 2) * w[2];
+        z[3 * i + 2] = x(i, 0) * w[1] + x(i, 1) * w[2];
+    }
+}
+__device__ __forceinline__ double sym_at(const double (&x)[6], int i, int j)
+{
+    constexpr int I[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
+    return x[I[i][j]];
+}
+
+// sine and cosine on [0, pi/3] by their Taylor polynomials (terms to x^13 and
+// x^12: below 1e-9)
+__device__ __forceinline__ void sincos_third(float x, float &sn, float &cs)
+{
+    const float z = x * x;
+    sn = x * (1.0f + z * (-1.0f / 6 + z * (1.0f / 120 + z * (-1.0f / 5040 + z * (1.0f / 362880 - z * (1.0f / 39916800))))));
+    cs = 1.0f + z * (-0.5f + z * (1.0f / 24 + z * (-1.0f / 720 + z * (1.0f / 40320 - z * (1.0f / 3628800 - z * (1.0f / 479001600))))));
+}
+
 // The invariants (traces, where cancellation lives) are FP64; their roots and
 // the principal-strain trigonometry are FP32, whose ~1e-7 relative error is
 // far below the BF16 rounding the network applies to its inputs.
-__device__ void features_of(const M3 &s, const M3 &r, double dratio, float *x)
+__device__ __forceinline__ void features_of(const Split &d, double dratio, float (&x)[10])
 {
-    const M3 s2 = mul(s, s), r2 = mul(r, r);
-    const double i1 = tr(s2), i2 = -tr(r2), i3 = tr(mul(s2, s)), i4 = tr(mul(r2, s)), i5 = tr(mul(r2, s2));
-    const double i6 = tr(mul(mul(r2, s), mul(r, s2)));
+    double s2[6], r2[6], r2s[9], s2r[9];
+    squares(d, s2, r2);
+    const double i1 = s2[0] + s2[3] + s2[5], i2 = -(r2[0] + r2[3] + r2[5]);
+    const double i3 = tr2(s2, d.s), i4 = tr2(r2, d.s), i5 = tr2(r2, s2);
+    // tr(r^2 s r s^2), r s^2 = -(s^2 r)^T
+    mul_ss(r2, d.s, r2s);
+    mul_r([&](int i, int j) { return sym_at(s2, i, j); }, d.w, s2r);
+    double i6 = 0;
+#pragma unroll
+    for (int c = 0; c < 9; ++c) i6 -= r2s[c] * s2r[c];
     x[0] = sqrtf(i1 > 0 ? (float)i1 : 0.0f);
     x[1] = sqrtf(i2 > 0 ? (float)i2 : 0.0f);
     x[2] = cbrtf((float)i3);
@@ -91,16 +169,45 @@ __device__ void features_of(const M3 &s, const M3 &r, double dratio, float *x)
     if (p > 1e-300) {
         double c = 1.5 * q / p * sqrt(3.0 / p);
         c = c > 1.0 ? 1.0 : (c < -1.0 ? -1.0 : c);
-        const float ph = acosf((float)c) / 3.0f, m = 2.0f * sqrtf((float)(p / 3.0));
-        l0 = m * cosf(ph);
-        l1 = m * cosf(ph - 2.0943951023931955f);   // 2 pi / 3
-        l2 = m * cosf(ph - 4.1887902047863905f);   // 4 pi / 3
+        const float ph = acosf((float)c) / 3.0f, m = sqrtf((float)(p / 3.0));
+        float sn, cs;
+        sincos_third(ph, sn, cs);
+        // 2 m cos(ph - 2 pi k / 3)
+        l0 = 2.0f * m * cs;
+        l1 = m * (1.7320508075688772f * sn - cs);
+        l2 = -m * (1.7320508075688772f * sn + cs);
     }
     // descending order: l0 >= l1 >= l2 for ph in [0, pi/3]
     x[6] = l0;
     x[7] = l1;
     x[8] = l2;
     x[9] = (float)dratio;
+}
+
+// sum_n G_n T_n, components (11 12 13 22 23 33).  T2 = s r + (s r)^T,
+// T5 = -(s^2 r + (s^2 r)^T) and T6 = s r r + (s r r)^T up to its trace, so
+// the three are N r + (N r)^T with N = G2 s - G5 s^2 + G6 s r.
+__device__ __forceinline__ void stress_of(const Split &d, const float (&G)[6], double (&t)[6])
+{
+    double s2[6], r2[6], sr[9], N[9], Nr[9];
+    squares(d, s2, r2);
+    mul_r([&](int i, int j) { return sym_at(d.s, i, j); }, d.w, sr);
+    const double g2 = G[1], g5 = G[4], g6 = G[5];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            N[3 * i + j] = g2 * sym_at(d.s, i, j) - g5 * sym_at(s2, i, j) + g6 * sr[3 * i + j];
+    mul_r([&](int i, int j) { return N[3 * i + j]; }, d.w, Nr);
+    const double iso = ((double)G[2] * (s2[0] + s2[3] + s2[5]) + (double)G[3] * (r2[0] + r2[3] + r2[5]) +
+                        2.0 * g6 * tr2(d.s, r2)) / 3.0;
+    constexpr int I[6] = {0, 0, 0, 1, 1, 2}, J[6] = {0, 1, 2, 1, 2, 2};
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+        t[c] = (double)G[0] * d.s[c] + (double)G[2] * s2[c] + (double)G[3] * r2[c] + Nr[3 * I[c] + J[c]] +
+               Nr[3 * J[c] + I[c]];
+        if (I[c] == J[c]) t[c] -= iso;
+    }
 }
 
 // the six basis tensors, components (11 12 13 22 23 33)
@@ -190,55 +297,107 @@ __global__ void __launch_bounds__(256) k_closure_features(const TS *__restrict__
 {
     const double inv = inv_scale(sumsq, nnorm);
     for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
-        M3 s, r;
-        strain_rotation(g, t, stride, inv, s, r);
+        double A[9];
+#pragma unroll
+        for (int c = 0; c < 9; ++c) A[c] = inv * (double)g[t + c * stride];
         float x[10];
-        features_of(s, r, dratio, x);
+        features_of(split_of(A), dratio, x);
 #pragma unroll
         for (int k = 0; k < 10; ++k) X[t * 10 + k] = x[k];
         if (A9) {
 #pragma unroll
-            for (int c = 0; c < 9; ++c) A9[t * 9 + c] = (float)(inv * (double)g[t + c * stride]);
+            for (int c = 0; c < 9; ++c) A9[t * 9 + c] = (float)A[c];
         }
     }
 }
 
 // ---------------------------------------------------------------------------
-// stress of the network outputs G (n, 6).  which = 0: write tau 11 12 22 33
+// stress: features, network and basis of a point in one pass.  A wave takes 64
+// points; its lanes form the features of one point each, hand them (BF16)
+// through LDS to the network's operands, 32 points at a time, and take the
+// outputs (FP32) back the same way.  which = 0: write tau 11 12 22 33
 // to tau (4 components, stride apart, cells); 1: tau 13 23 (2, edges);
 // 2: all six (11 12 13 22 23 33).  fallback: keep the value already in tau
 // wherever the network's dissipation -tau_ij S_ij is negative; the number
 // of such points of each block goes to nfall[blockIdx.x].
+// Bound by the vector unit: the GELUs of the network, then the FP64 algebra.
+// 256^3 FP32: features 335, network 1600 and stress 350 us as three passes
+// that moved 224 bytes per point, now 1.4 ms in one that moves 60.
 // ---------------------------------------------------------------------------
 template <typename TS>
-__global__ void __launch_bounds__(256) k_closure_stress(const TS *__restrict__ g, long n, long stride,
-                                                       const double *__restrict__ sumsq, long nnorm, double delta2,
-                                                       const float *__restrict__ G, int which, int fallback,
-                                                       TS *__restrict__ tau, long tstride,
-                                                       unsigned *__restrict__ nfall)
+__global__ void __launch_bounds__(256, 4)
+k_closure_stress(const TS *g, long n, long stride, const double *__restrict__ sumsq, long nnorm, double delta2,
+                 double dratio, const unsigned short *__restrict__ Wb, const float *__restrict__ P, int which,
+                 int fallback, TS *tau, long tstride, unsigned *__restrict__ nfall)
 {
-    __shared__ unsigned cnt[256];
+    __shared__ MlpLds L;
+    __shared__ u32x4 rows[256 * 2];  // 32 bytes per point: features, then outputs
+    __shared__ unsigned cnt[4];
+    mlp_stage(L, Wb, P);
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, gq = lane >> 4;
+    unsigned *mine = (unsigned *)(rows + (wave * 64 + lane) * 2);
     const double inv = inv_scale(sumsq, nnorm);
     // tau = Delta^2 g^2 sum G_n T_n(a), a = A / g
     const double scale = inv > 0 ? delta2 / (inv * inv) : 0.0;
-    unsigned mine = 0;
-    for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
-        M3 s, r;
-        strain_rotation(g, t, stride, inv, s, r);
-        double T[6][6];
-        basis_of(s, r, T);
-        double tv[6] = {0, 0, 0, 0, 0, 0};
+    unsigned kept = 0;
+    const long chunks = (n + 63) / 64;
+    for (long ch = (long)blockIdx.x * 4 + wave; ch < chunks; ch += (long)gridDim.x * 4) {
+        const long t = 64 * ch + lane;
+        TS a[9];
 #pragma unroll
-        for (int k = 0; k < 6; ++k) {
-            const double gk = (double)G[t * 6 + k];
+        for (int c = 0; c < 9; ++c) a[c] = t < n ? g[t + c * stride] : TS(0);
+        {
+            double A[9];
+            float x[10];
 #pragma unroll
-            for (int c = 0; c < 6; ++c) tv[c] = fma(gk, T[k][c], tv[c]);
+            for (int c = 0; c < 9; ++c) A[c] = inv * (double)a[c];
+            features_of(split_of(A), dratio, x);
+            ((u32x4 *)mine)[0] = (u32x4){pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7])};
+            ((u32x4 *)mine)[1] = (u32x4){pack2(x[8], x[9]), 0u, 0u, 0u};
         }
+        // the lanes of a wave exchange through its own rows: LDS operations
+        // of a wave complete in order, the fences keep them in program order
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+        for (int half = 0; half < 2; ++half) {
+            u32x2 x[2];
+            f32x4 y[2];
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                x[q] = ((const u32x2 *)(rows + (wave * 64 + 32 * half + 16 * q + (lane & 15)) * 2))[gq];
+            mlp_eval<2>(L, x, y);
+            // the rows read above belong to these 32 points alone
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                if (gq < 2)
+                    rows[(wave * 64 + 32 * half + 16 * q + (lane & 15)) * 2 + gq] = __builtin_bit_cast(u32x4, y[q]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        float G[6];
+        {
+            const f32x4 y0 = __builtin_bit_cast(f32x4, ((u32x4 *)mine)[0]);
+            const u32x2 y1 = ((u32x2 *)mine)[2];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) G[i] = y0[i];
+            G[4] = __uint_as_float(y1[0]);
+            G[5] = __uint_as_float(y1[1]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        double A[9], tv[6];
+#pragma unroll
+        for (int c = 0; c < 9; ++c) A[c] = inv * (double)a[c];
+        const Split d = split_of(A);
+        stress_of(d, G, tv);
+        if (t >= n) continue;
         // dissipation sign of the normalised stress against the strain
-        const double pi = -(tv[0] * s.a[0][0] + tv[3] * s.a[1][1] + tv[5] * s.a[2][2] +
-                            2.0 * (tv[1] * s.a[0][1] + tv[2] * s.a[0][2] + tv[4] * s.a[1][2]));
-        if (fallback && pi < 0) {
-            ++mine;
+        if (fallback && -tr2(tv, d.s) < 0) {
+            ++kept;
             continue;
         }
         if (which == 0) {
@@ -255,13 +414,11 @@ __global__ void __launch_bounds__(256) k_closure_stress(const TS *__restrict__ g
         }
     }
     if (!nfall) return;
-    cnt[threadIdx.x] = mine;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) kept += __shfl_xor(kept, o);
+    if (lane == 0) cnt[wave] = kept;
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) cnt[threadIdx.x] += cnt[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) nfall[blockIdx.x] = cnt[0];
+    if (threadIdx.x == 0) nfall[blockIdx.x] = cnt[0] + cnt[1] + cnt[2] + cnt[3];
 }
 
 // ---------------------------------------------------------------------------
@@ -315,8 +472,6 @@ __global__ void __launch_bounds__(256) k_closure_loss(const float *__restrict__ 
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-int closure_blocks(long n) { return (int)grid_of(n); }
-
 hipError_t launch_grad_sumsq(bool dbl, const void *g, long n, long stride, double *partial, double *out,
                              hipStream_t st)
 {
@@ -342,18 +497,29 @@ hipError_t launch_closure_features(bool dbl, const void *g, long n, long stride,
     return hipGetLastError();
 }
 
-hipError_t launch_closure_stress(bool dbl, const void *g, long n, long stride, const double *sumsq, long nnorm,
-                                 double delta2, const float *G, int which, int fallback, void *tau, long tstride,
-                                 unsigned *nfall, hipStream_t st)
+template <typename TS>
+static hipError_t stress_t(const void *g, long n, long stride, const double *sumsq, long nnorm, double delta2,
+                           double dratio, const unsigned short *Wb, const float *P, int which, int fallback, void *tau,
+                           long tstride, unsigned *nfall, int *blocks, hipStream_t st)
 {
-    const unsigned nb = grid_of(n);
-    if (dbl)
-        hipLaunchKernelGGL(k_closure_stress<double>, dim3(nb), dim3(256), 0, st, (const double *)g, n, stride, sumsq,
-                           nnorm, delta2, G, which, fallback, (double *)tau, tstride, nfall);
-    else
-        hipLaunchKernelGGL(k_closure_stress<float>, dim3(nb), dim3(256), 0, st, (const float *)g, n, stride, sumsq,
-                           nnorm, delta2, G, which, fallback, (float *)tau, tstride, nfall);
+    static Resident resident;
+    int res = 0;
+    const hipError_t e = resident_blocks(resident, (const void *)k_closure_stress<TS>, 256, &res);
+    if (e != hipSuccess) return e;
+    const long need = (n + 255) / 256;
+    const long nb = std::min(std::min(need, (long)res), 8192L);
+    *blocks = (int)nb;
+    hipLaunchKernelGGL(k_closure_stress<TS>, dim3((unsigned)nb), dim3(256), 0, st, (const TS *)g, n, stride, sumsq,
+                       nnorm, delta2, dratio, Wb, P, which, fallback, (TS *)tau, tstride, nfall);
     return hipGetLastError();
+}
+
+hipError_t launch_closure_stress(bool dbl, const void *g, long n, long stride, const double *sumsq, long nnorm,
+                                 double delta2, double dratio, const unsigned short *Wb, const float *P, int which,
+                                 int fallback, void *tau, long tstride, unsigned *nfall, int *blocks, hipStream_t st)
+{
+    return (dbl ? stress_t<double> : stress_t<float>)(g, n, stride, sumsq, nnorm, delta2, dratio, Wb, P, which,
+                                                      fallback, tau, tstride, nfall, blocks, st);
 }
 
 hipError_t launch_closure_loss(const float *G, const float *A9, const float *T, long B, float *dG, double *partial,

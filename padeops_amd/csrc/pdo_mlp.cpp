@@ -36,6 +36,12 @@ struct MlpObject {
 
 struct pdo_mlp_s : public pdo::MlpObject {};
 
+void pdo::mlp_params(pdo_mlp h, const unsigned short **Wb, const float **P)
+{
+    *Wb = h->Wb;
+    *P = h->P;
+}
+
 using namespace pdo;
 
 static int ok(hipError_t e, const char *w) { return e == hipSuccess ? 0 : hip_fail(e, w); }

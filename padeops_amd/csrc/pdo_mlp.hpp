@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "../../include/padeops_hip.h"
+
 namespace pdo {
 
 // 10 inputs (padded to 16) -> 64 -> 64 -> 64 -> 6 outputs (padded to 16).
@@ -25,6 +27,9 @@ struct MlpCache {
     unsigned short *H[4];
     unsigned short *Z[3];
 };
+
+// the network's parameters on the device: BF16 weights and FP32 vector
+void mlp_params(pdo_mlp h, const unsigned short **Wb, const float **P);
 
 hipError_t launch_mlp_forward(const float *X, float *Y, const unsigned short *Wb, const float *P, long B,
                               const MlpCache &cache, hipStream_t st);

@@ -158,3 +158,29 @@ def test_mlp_backward_from_dy(cuda):
     # the batch of the last forward_train is enforced
     with pytest.raises(P.PdoError):
         net.backward(torch.from_numpy(dYg[:100]).to(cuda))
+
+
+@pytest.mark.parametrize("dt", ["f64", "f32"])
+@pytest.mark.parametrize("n", [1, 15, 31, 33, 63, 65, 255, 257, 321])
+def test_stress_at_the_edges_of_waves(cuda, n, dt):
+    """the stress kernel takes 64 points per wave and 32 per network pass"""
+    import torch
+    dtype = torch.float64 if dt == "f64" else torch.float32
+    A = _field(n, n).astype(np.float32).astype(np.float64)
+    net = P.SGSNet(64)
+    net.set_params(P.SGSNet.pack(M.init_params(6)))
+    cl = P.Closure(net, n)
+    g = _planes(A, cuda, dtype)
+    tau = torch.full((6 * n + 64,), 77.0, dtype=dtype, device=cuda)
+    X, Y = torch.empty((n, 10), device=cuda), torch.empty((n, 6), device=cuda)
+    assert cl.stress(g, n, 0.4, 0.5, tau, which=2) == 0
+    assert cl.features(g, n, 0.5, X) == 0 and net.forward(X, Y) == 0
+    torch.cuda.synchronize()
+    ref = C.stress(A, Y.cpu().numpy(), 0.4)
+    got = tau.cpu().numpy().astype(np.float64)
+    assert (got[6 * n:] == 77.0).all()
+    # FP64 sums of the same outputs, rounded to the storage type
+    assert np.abs(got[:6 * n].reshape(6, n).T - ref).max() <= (1e-12 if dt == "f64" else 1e-7) * np.abs(ref).max()
+    mark = torch.full((6 * n,), 1234.5, dtype=dtype, device=cuda)
+    assert cl.stress(g, n, 0.4, 0.5, mark, which=2, fallback=True) == 0
+    assert cl.fallback_count() == int((C.dissipation_sign(A, Y.cpu().numpy()) < 0).sum())
