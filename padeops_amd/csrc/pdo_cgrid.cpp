@@ -74,34 +74,7 @@ int cg(pdo_cgrid h, CgOp op, const CgArgs &a, hipStream_t st)
     return e == hipSuccess ? 0 : hip_fail(e, "cgrid kernel");
 }
 
-// derivatives%dd{x,y,z} / d2d{x,y,z}2 along direction d (0, 1, 2)
-int dd(pdo_cgrid h, int d, const void *f, void *df, int bc1, int bcn, hipStream_t st)
-{
-    void *s = (void *)st;
-    if (d == 0) return pdo_derivatives_ddx(h->der, h->prec, f, df, bc1, bcn, s);
-    if (d == 1) return pdo_derivatives_ddy(h->der, h->prec, f, df, bc1, bcn, s);
-    return pdo_derivatives_ddz(h->der, h->prec, f, df, bc1, bcn, s);
-}
-int d2(pdo_cgrid h, int d, const void *f, void *df, int bc1, int bcn, hipStream_t st)
-{
-    void *s = (void *)st;
-    if (d == 0) return pdo_derivatives_d2dx2(h->der, h->prec, f, df, bc1, bcn, s);
-    if (d == 1) return pdo_derivatives_d2dy2(h->der, h->prec, f, df, bc1, bcn, s);
-    return pdo_derivatives_d2dz2(h->der, h->prec, f, df, bc1, bcn, s);
-}
-
 const int *bc_of(pdo_cgrid h, int d) { return d == 0 ? h->p.x_bc : (d == 1 ? h->p.y_bc : h->p.z_bc); }
-
-// gradient (cgrid.F90:446-480); flip[d] negates the bc of direction d
-int gradient(pdo_cgrid h, const void *f, void *out3, int flipdir, hipStream_t st)
-{
-    for (int d = 0; d < 3; d++) {
-        const int *b = bc_of(h, d);
-        const int sg = d == flipdir ? -1 : 1;
-        PDO_TRY(dd(h, d, f, (char *)out3 + (size_t)d * h->n * h->W, sg * b[0], sg * b[1], st));
-    }
-    return 0;
-}
 
 // the fourth derivatives along each direction (two second-derivative passes)
 // of the functions of the coefficients [k0, k1) into F_D4 + 3 k + d
@@ -109,8 +82,11 @@ int fourth(pdo_cgrid h, const void *const f[3], int k0, int k1, hipStream_t st)
 {
     for (int d = 0; d < 3; d++) {
         const int *b = bc_of(h, d);
-        for (int k = k0; k < k1; k++) PDO_TRY(d2(h, d, f[k], h->f(F_T1 + k), b[0], b[1], st));
-        for (int k = k0; k < k1; k++) PDO_TRY(d2(h, d, h->f(F_T1 + k), h->f(F_D4 + 3 * k + d), b[0], b[1], st));
+        DerivTask t[3];
+        for (int k = k0; k < k1; k++) t[k - k0] = {f[k], h->f(F_T1 + k), b[0], b[1]};
+        PDO_TRY(derivatives_many(h->der, d, 2, h->prec, t, k1 - k0, nullptr, st));
+        for (int k = k0; k < k1; k++) t[k - k0] = {h->f(F_T1 + k), h->f(F_D4 + 3 * k + d), b[0], b[1]};
+        PDO_TRY(derivatives_many(h->der, d, 2, h->prec, t, k1 - k0, nullptr, st));
     }
     return 0;
 }
@@ -120,7 +96,6 @@ int fourth(pdo_cgrid h, const void *const f[3], int k0, int k1, hipStream_t st)
 // applications along a direction go together where the filter can.
 int filter3(pdo_cgrid h, pdo_filters fl, void *const *arr, int count, int numtimes, hipStream_t st)
 {
-    void *s = (void *)st;
     const int order[3] = {1, 0, 2};
     int total = 0;
     for (int d : order) total += filters_twice(fl, d, h->prec) ? (numtimes + 1) / 2 : numtimes;
@@ -134,15 +109,10 @@ int filter3(pdo_cgrid h, pdo_filters fl, void *const *arr, int count, int numtim
             const int times = two && left > 1 ? 2 : 1;
             // out of place: the last pass writes arr unless it also reads it
             const bool home = pass == total - 1 && cur[0] != arr[0];
-            for (int k = 0; k < count; k++) {
-                void *dst = home ? arr[k] : h->f(F_FIL + 2 * k + buf);
-                const int e = times == 2 ? filters_apply_twice(fl, d, h->prec, cur[k], dst, b[0], b[1], st)
-                            : d == 0     ? pdo_filters_filterx(fl, h->prec, cur[k], dst, b[0], b[1], s)
-                            : d == 1     ? pdo_filters_filtery(fl, h->prec, cur[k], dst, b[0], b[1], s)
-                                         : pdo_filters_filterz(fl, h->prec, cur[k], dst, b[0], b[1], s);
-                if (e) return e;
-                cur[k] = dst;
-            }
+            void *dst[3];
+            for (int k = 0; k < count; k++) dst[k] = home ? arr[k] : h->f(F_FIL + 2 * k + buf);
+            PDO_TRY(filters_many(fl, d, h->prec, cur, dst, count, times, b[0], b[1], st));
+            for (int k = 0; k < count; k++) cur[k] = dst[k];
             buf ^= 1;
             left -= times;
         }
@@ -159,8 +129,7 @@ int filter3(pdo_cgrid h, pdo_filters fl, void *const *arr, int count, int numtim
 }
 
 // getLAD (cgrid.F90:1058-1257), one species: the filtered artificial shear
-// and bulk viscosity and conductivity into F_STAR.  Gradients of rho and e
-// precede it.
+// and bulk viscosity and conductivity into F_STAR
 int lad(pdo_cgrid h, hipStream_t st)
 {
     const pdo_cgrid_params &p = h->p;
@@ -174,8 +143,6 @@ int lad(pdo_cgrid h, hipStream_t st)
     a.out[1] = h->f(F_DIL);
     a.n = n;
     PDO_TRY(cg(h, CG_STRAIN, a, st));
-    PDO_TRY(gradient(h, h->f(F_PRIM), h->f(F_DRHO), -1, st));
-    PDO_TRY(gradient(h, h->f(F_PRIM + 4), h->f(F_DE), -1, st));
     const void *const func[3] = {h->f(F_FUNC), h->f(F_DIL), h->f(F_PRIM + 4)};
     auto star = [&](int k) -> int {
         CgArgs c;
@@ -203,13 +170,18 @@ int lad(pdo_cgrid h, hipStream_t st)
         for (int i = 0; i < 8; i++) c.c[i] = v[i];
         return cg(h, CG_KAPSTAR, c, st);
     };
-    // one coefficient after the other: a pass finds what the last one wrote
-    // in the Infinity Cache
-    for (int k = 0; k < 3; k++) {
-        PDO_TRY(fourth(h, func, k, k + 1, st));
-        PDO_TRY(star(k));
-        void *s = h->f(F_STAR + k);
-        PDO_TRY(filter3(h, h->gfil, &s, 1, 2, st));
+    // small fields: the three coefficients' passes share launches; others:
+    // one coefficient after the other, so that a pass finds what the last one
+    // wrote in the Infinity Cache
+    const int step = small_field(n, h->prec) ? 3 : 1;
+    for (int k = 0; k < 3; k += step) {
+        PDO_TRY(fourth(h, func, k, k + step, st));
+        void *s[3];
+        for (int q = k; q < k + step; q++) {
+            PDO_TRY(star(q));
+            s[q - k] = h->f(F_STAR + q);
+        }
+        PDO_TRY(filter3(h, h->gfil, s, step, 2, st));
     }
     return 0;
 }
@@ -264,8 +236,19 @@ int pdo_cgrid_rhs(pdo_cgrid h, int prec, const void *Wc, void *rhs, void *stream
         a.c[1] = 1.0 / p.Rgas;
         PDO_TRY(cg(h, CG_PRIMITIVE, a, st));
     }
-    // velocity gradients: u with -x_bc, v with -y_bc, w with -z_bc
-    for (int c = 0; c < 3; c++) PDO_TRY(gradient(h, h->f(F_PRIM + 1 + c), h->f(F_G + 3 * c), c, st));
+    // gradients (cgrid.F90:446-480) of u, v, w, rho and e: antisymmetric ends
+    // for u along x, v along y and w along z
+    for (int d = 0; d < 3; d++) {
+        const int *b = bc_of(h, d);
+        DerivTask t[5];
+        for (int c = 0; c < 3; c++) {
+            const int sg = c == d ? -1 : 1;
+            t[c] = {h->f(F_PRIM + 1 + c), h->f(F_G + 3 * c + d), sg * b[0], sg * b[1]};
+        }
+        t[3] = {h->f(F_PRIM), h->f(F_DRHO + d), b[0], b[1]};
+        t[4] = {h->f(F_PRIM + 4), h->f(F_DE + d), b[0], b[1]};
+        PDO_TRY(derivatives_many(h->der, d, 1, h->prec, t, 5, nullptr, st));
+    }
     PDO_TRY(lad(h, st));
     // transport properties, tau, q and the fluxes along every direction
     {
@@ -293,14 +276,14 @@ int pdo_cgrid_rhs(pdo_cgrid h, int prec, const void *Wc, void *rhs, void *stream
     // along d, antisymmetric for the others
     for (int d = 0; d < 3; d++) {
         const int *b = bc_of(h, d);
+        DerivTask t[5];
         for (int c = 0; c < 5; c++) {
             const int sg = c == 1 + d ? 1 : -1;
-            void *r = (char *)rhs + (size_t)c * n * h->W;
             // the mass flux is the momentum
             const void *f = c == 0 ? (const char *)Wc + (size_t)(1 + d) * n * h->W : h->f(F_FLUX + 4 * d + c - 1);
-            PDO_TRY(derivatives_subtract(h->der, d, h->prec, f, r, d == 0, sg * b[0], sg * b[1],
-                                         h->f(F_STAR), st));
+            t[c] = {f, (char *)rhs + (size_t)c * n * h->W, sg * b[0], sg * b[1], d == 0 ? 3 : 2};
         }
+        PDO_TRY(derivatives_many(h->der, d, 1, h->prec, t, 5, h->f(F_STAR), st));
     }
     return 0;
 }

@@ -29,10 +29,21 @@ struct CgArgs {
 
 hipError_t launch_cgrid(bool dbl, CgOp op, const CgArgs &a, hipStream_t st);
 
-// of the derivatives and filters objects (pdo_dispatch.cpp)
-int derivatives_subtract(pdo_derivatives h, int d, int prec, const void *f, void *out, bool first, int bc1, int bcn,
-                         void *work, hipStream_t st);
+// of the derivatives and filters objects (pdo_dispatch.cpp): independent
+// passes along direction d (0, 1, 2), several per launch for small fields
+struct DerivTask {
+    const void *f;
+    void *out;
+    int bc1, bcn;
+    int sub = 0;  // 2: out -= df, 3: out = -df
+};
+// order 1 or 2, at most 8 tasks; work holds one field (null without sub)
+int derivatives_many(pdo_derivatives h, int d, int order, int prec, const DerivTask *t, int count, void *work,
+                     hipStream_t st);
+// whether one pass along d can apply the filter twice
 bool filters_twice(pdo_filters h, int d, int prec);
-int filters_apply_twice(pdo_filters h, int d, int prec, const void *f, void *ff, int bc1, int bcn, hipStream_t st);
+// at most 3 fields, the filter applied `times` (1, or 2 where filters_twice) times
+int filters_many(pdo_filters h, int d, int prec, const void *const *f, void *const *ff, int count, int times, int bc1,
+                 int bcn, hipStream_t st);
 
 }  // namespace pdo

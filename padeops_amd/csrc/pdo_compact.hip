@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "pdo_stencil.hpp"
 
@@ -438,9 +439,10 @@ __device__ __forceinline__ void strided_store(const ApplyArgs &A, const typename
 
 // LB: workgroup size bound, 1024 (up to 16 segments) or 512 (up to 8, which
 // leaves the compiler 256 vector registers per lane)
-template <int FAM, int MODE, int NPW, bool PER, bool EPI, int XR, int LB>
-__global__ void __launch_bounds__(LB) k_strided(ApplyArgs A)
+template <int FAM, int MODE, int NPW, bool PER, bool EPI, int XR, int LB, typename ARGS>
+__global__ void __launch_bounds__(LB) k_strided(ARGS B)
 {
+    const ApplyArgs &A = pass_of(B);
     using TS = typename Mode<MODE>::TS;
     using TC = typename Mode<MODE>::TC;
     using F = Fam<FAM>;
@@ -707,9 +709,10 @@ __device__ __forceinline__ void xdir_store(const ApplyArgs &A, typename Mode<MOD
     }
 }
 
-template <int FAM, int MODE, bool EPI>
-__global__ void __launch_bounds__(256) k_xdir(ApplyArgs A, int TP, int LD)
+template <int FAM, int MODE, bool EPI, typename ARGS>
+__global__ void __launch_bounds__(256) k_xdir(ARGS B, int TP, int LD)
 {
+    const ApplyArgs &A = pass_of(B);
     // periodic pencils only: every segment has the same factors (type 1)
     extern __shared__ unsigned char smem[];
     constexpr bool PER = true;
@@ -864,15 +867,23 @@ hipError_t launch_zero_words(void *p, long words, hipStream_t st)
 // launchers
 // ---------------------------------------------------------------------------
 template <int FAM, int MODE, int NPW, bool PER, bool EPI, int XR = 0, int LB = 1024>
-static hipError_t launch_strided_k(const ApplyArgs &A, hipStream_t st)
+static hipError_t launch_strided_k(const ApplyBatch &B, int count, hipStream_t st)
 {
     using TC = typename Mode<MODE>::TC;
     constexpr int K = Fam<FAM>::K;
-    dim3 grid((unsigned)((A.na + NPW - 1) / NPW), (unsigned)A.nb);
+    const ApplyArgs &A = B.a[0];
+    dim3 grid((unsigned)((A.na + NPW - 1) / NPW), (unsigned)A.nb, (unsigned)count);
     dim3 block(NPW * A.P);
     if ((int)block.x > LB || A.xr != XR) return hipErrorInvalidValue;
     size_t lds = (size_t)A.P * 2 * K * NPW * sizeof(TC) * (Mode<MODE>::REFINE ? 3 : 1);
-    hipLaunchKernelGGL((k_strided<FAM, MODE, NPW, PER, EPI, XR, LB>), grid, block, lds, st, A);
+    if (count > 1) {
+        if constexpr (can_batch(K, MODE))
+            hipLaunchKernelGGL((k_strided<FAM, MODE, NPW, PER, EPI, XR, LB, ApplyBatch>), grid, block, lds, st, B);
+        else
+            return hipErrorInvalidValue;
+    } else {
+        hipLaunchKernelGGL((k_strided<FAM, MODE, NPW, PER, EPI, XR, LB, ApplyArgs>), grid, block, lds, st, A);
+    }
     return hipGetLastError();
 }
 
@@ -892,45 +903,47 @@ template <int FAM> constexpr bool has_epilogue() { return FAM == 0 || FAM == 2; 
 #endif
 
 template <int FAM, int MODE>
-static hipError_t launch_strided_t(const ApplyArgs &A, hipStream_t st)
+static hipError_t launch_strided_t(const ApplyBatch &B, int count, hipStream_t st)
 {
+    const ApplyArgs &A = B.a[0];
     if (!A.periodic && A.epi) return hipErrorInvalidValue;
     if constexpr (MODE == MODE_F32R) if (!A.periodic) {
         // refined non-periodic passes run on overlapping segments, but for
         // the 513 rows (32 x 16 + 1) of the tridiagonal families: one segment
         // more than those take
         if constexpr (has_extra_row<FAM>())
-            if (A.xr && A.P > 8) return launch_strided_k<FAM, MODE, 64, false, false, 1, 1024>(A, st);
+            if (A.xr && A.P > 8) return launch_strided_k<FAM, MODE, 64, false, false, 1, 1024>(B, count, st);
         return hipErrorInvalidValue;
     }
     if constexpr (MODE != MODE_F32R) if (!A.periodic) {
         if (A.xr) {
             if constexpr (has_extra_row<FAM>()) {
-                if (A.P <= 8) return launch_strided_k<FAM, MODE, 64, false, false, 1, 512>(A, st);
-                return launch_strided_k<FAM, MODE, 64, false, false, 1, 1024>(A, st);
+                if (A.P <= 8) return launch_strided_k<FAM, MODE, 64, false, false, 1, 512>(B, count, st);
+                return launch_strided_k<FAM, MODE, 64, false, false, 1, 1024>(B, count, st);
             }
             return hipErrorInvalidValue;
         }
-        if (A.P <= 8) return launch_strided_k<FAM, MODE, 64, false, false, 0, 512>(A, st);
-        return launch_strided_k<FAM, MODE, 64, false, false, 0, 1024>(A, st);
+        if (A.P <= 8) return launch_strided_k<FAM, MODE, 64, false, false, 0, 512>(B, count, st);
+        return launch_strided_k<FAM, MODE, 64, false, false, 0, 1024>(B, count, st);
     }
     if (A.epi) {
         if constexpr (has_epilogue<FAM>()) {
-            if (PDO_STRIDED_NPW_PER == 32 && A.P % 2 == 0) return launch_strided_k<FAM, MODE, 32, true, true>(A, st);
-            return launch_strided_k<FAM, MODE, 64, true, true>(A, st);
+            if (PDO_STRIDED_NPW_PER == 32 && A.P % 2 == 0) return launch_strided_k<FAM, MODE, 32, true, true>(B, count, st);
+            return launch_strided_k<FAM, MODE, 64, true, true>(B, count, st);
         }
         return hipErrorInvalidValue;
     }
-    if (PDO_STRIDED_NPW_PER == 32 && A.P % 2 == 0) return launch_strided_k<FAM, MODE, 32, true, false>(A, st);
-    return launch_strided_k<FAM, MODE, 64, true, false>(A, st);
+    if (PDO_STRIDED_NPW_PER == 32 && A.P % 2 == 0) return launch_strided_k<FAM, MODE, 32, true, false>(B, count, st);
+    return launch_strided_k<FAM, MODE, 64, true, false>(B, count, st);
 }
 
 template <int FAM, int MODE>
-static hipError_t launch_x_t(const ApplyArgs &A, hipStream_t st)
+static hipError_t launch_x_t(const ApplyBatch &B, int count, hipStream_t st)
 {
     using TS = typename Mode<MODE>::TS;
     using TC = typename Mode<MODE>::TC;
     constexpr int K = Fam<FAM>::K;
+    const ApplyArgs &A = B.a[0];
     const int P = A.P;
     int TP = 256 / P;
     // pencil pitch n + n/32 = 33 P: the P segments of consecutive pencils in
@@ -943,23 +956,31 @@ static hipError_t launch_x_t(const ApplyArgs &A, hipStream_t st)
     while (TP > 1 && lds_of(TP) > 80 * 1024) TP >>= 1;
     if (TP * P != 256) return hipErrorInvalidValue;
     const long npen = A.na * A.nb;
-    dim3 grid((unsigned)((npen + TP - 1) / TP));
+    dim3 grid((unsigned)((npen + TP - 1) / TP), 1u, (unsigned)count);
     dim3 block(TP * P);
-    if (A.epi) {
-        if constexpr (has_epilogue<FAM>())
-            hipLaunchKernelGGL((k_xdir<FAM, MODE, true>), grid, block, lds_of(TP), st, A, TP, LD);
-        else
-            return hipErrorInvalidValue;
-    } else {
-        hipLaunchKernelGGL((k_xdir<FAM, MODE, false>), grid, block, lds_of(TP), st, A, TP, LD);
-    }
-    return hipGetLastError();
+    auto go = [&](auto epi) -> hipError_t {
+        constexpr bool EPI = decltype(epi)::value;
+        if (count > 1) {
+            if constexpr (can_batch(K, MODE))
+                hipLaunchKernelGGL((k_xdir<FAM, MODE, EPI, ApplyBatch>), grid, block, lds_of(TP), st, B, TP, LD);
+            else
+                return hipErrorInvalidValue;
+        } else {
+            hipLaunchKernelGGL((k_xdir<FAM, MODE, EPI, ApplyArgs>), grid, block, lds_of(TP), st, A, TP, LD);
+        }
+        return hipGetLastError();
+    };
+    if (!A.epi) return go(std::false_type{});
+    if constexpr (has_epilogue<FAM>()) return go(std::true_type{});
+    return hipErrorInvalidValue;
 }
 
 template <int FAM, int MODE>
-static hipError_t launch_general_t(const ApplyArgs &A, double *scratch, hipStream_t st)
+static hipError_t launch_general_t(const ApplyBatch &B, int count, double *scratch, hipStream_t st)
 {
     using TS = typename Mode<MODE>::TS;
+    const ApplyArgs &A = B.a[0];
+    if (count != 1) return hipErrorInvalidValue;  // one work area
     const long npen = A.na * A.nb;
     dim3 grid((unsigned)((npen + 255) / 256));
     hipLaunchKernelGGL((k_general<FAM, TS>), grid, dim3(256), 0, st, A, scratch);
@@ -967,46 +988,46 @@ static hipError_t launch_general_t(const ApplyArgs &A, double *scratch, hipStrea
 }
 
 template <int FAM>
-static hipError_t dispatch_mode(int shape, int mode, const ApplyArgs &A, double *scratch, hipStream_t st)
+static hipError_t dispatch_mode(int shape, int mode, const ApplyBatch &B, int count, double *scratch, hipStream_t st)
 {
     switch (shape) {
     case SHAPE_STRIDED:
         switch (mode) {
-        case MODE_F64: return launch_strided_t<FAM, MODE_F64>(A, st);
-        case MODE_F32R: return launch_strided_t<FAM, MODE_F32R>(A, st);
-        case MODE_F32S: return launch_strided_t<FAM, MODE_F32S>(A, st);
-        case MODE_F32: return launch_strided_t<FAM, MODE_F32>(A, st);
+        case MODE_F64: return launch_strided_t<FAM, MODE_F64>(B, count, st);
+        case MODE_F32R: return launch_strided_t<FAM, MODE_F32R>(B, count, st);
+        case MODE_F32S: return launch_strided_t<FAM, MODE_F32S>(B, count, st);
+        case MODE_F32: return launch_strided_t<FAM, MODE_F32>(B, count, st);
         }
         break;
     case SHAPE_X:
         if constexpr (Fam<FAM>::SHIFT == 0) {
             switch (mode) {
-            case MODE_F64: return launch_x_t<FAM, MODE_F64>(A, st);
-            case MODE_F32R: return launch_x_t<FAM, MODE_F32R>(A, st);
-            case MODE_F32S: return launch_x_t<FAM, MODE_F32S>(A, st);
-            case MODE_F32: return launch_x_t<FAM, MODE_F32>(A, st);
+            case MODE_F64: return launch_x_t<FAM, MODE_F64>(B, count, st);
+            case MODE_F32R: return launch_x_t<FAM, MODE_F32R>(B, count, st);
+            case MODE_F32S: return launch_x_t<FAM, MODE_F32S>(B, count, st);
+            case MODE_F32: return launch_x_t<FAM, MODE_F32>(B, count, st);
             }
         }
         break;
     case SHAPE_GENERAL:
-        if (mode == MODE_F64) return launch_general_t<FAM, MODE_F64>(A, scratch, st);
-        return launch_general_t<FAM, MODE_F32S>(A, scratch, st);
+        if (mode == MODE_F64) return launch_general_t<FAM, MODE_F64>(B, count, scratch, st);
+        return launch_general_t<FAM, MODE_F32S>(B, count, scratch, st);
     }
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_compact(int family, int shape, int mode, const ApplyArgs &A, double *scratch, hipStream_t st)
+hipError_t launch_compact(int family, int shape, int mode, const ApplyBatch &B, int count, double *scratch, hipStream_t st)
 {
     switch (family) {
-    case 0: return dispatch_mode<0>(shape, mode, A, scratch, st);
-    case 1: return dispatch_mode<1>(shape, mode, A, scratch, st);
-    case 2: return dispatch_mode<2>(shape, mode, A, scratch, st);
-    case 3: return dispatch_mode<3>(shape, mode, A, scratch, st);
-    case 4: return dispatch_mode<4>(shape, mode, A, scratch, st);
-    case 5: return dispatch_mode<5>(shape, mode, A, scratch, st);
-    case 6: return dispatch_mode<6>(shape, mode, A, scratch, st);
-    case 7: return dispatch_mode<7>(shape, mode, A, scratch, st);
-    case 8: return dispatch_mode<8>(shape, mode, A, scratch, st);
+    case 0: return dispatch_mode<0>(shape, mode, B, count, scratch, st);
+    case 1: return dispatch_mode<1>(shape, mode, B, count, scratch, st);
+    case 2: return dispatch_mode<2>(shape, mode, B, count, scratch, st);
+    case 3: return dispatch_mode<3>(shape, mode, B, count, scratch, st);
+    case 4: return dispatch_mode<4>(shape, mode, B, count, scratch, st);
+    case 5: return dispatch_mode<5>(shape, mode, B, count, scratch, st);
+    case 6: return dispatch_mode<6>(shape, mode, B, count, scratch, st);
+    case 7: return dispatch_mode<7>(shape, mode, B, count, scratch, st);
+    case 8: return dispatch_mode<8>(shape, mode, B, count, scratch, st);
     }
     return hipErrorInvalidValue;
 }

@@ -233,39 +233,59 @@ using namespace pdo;
 
 namespace pdo {
 
-// out -= df/dx_d (first: out = -df/dx_d); work holds one field
-int derivatives_subtract(pdo_derivatives h, int d, int prec, const void *f, void *out, bool first, int bc1, int bcn,
-                         void *work, hipStream_t st)
+int derivatives_many(pdo_derivatives h, int d, int order, int prec, const DerivTask *t, int count, void *work,
+                     hipStream_t st)
 {
     int na, nb, r;
     h->pencils(d, na, nb);
-    if (h->n_of(d) > 1 && (h->method[d] == METHOD_CD10 || h->method[d] == METHOD_CD06)) {
-        if (h->method[d] == METHOD_CD06) bc1 = bcn = 0;
-        return apply(h->op[d], KIND_D1, bc1, bcn, d + 1, prec, f, out, na, nb, st, first ? 3 : 2, out);
+    const bool cd10 = h->method[d] == METHOD_CD10;
+    bool direct = h->n_of(d) > 1 && (cd10 || (h->method[d] == METHOD_CD06 && order == 1)) && count <= 8;
+    for (int i = 0; i < count; i++)  // the operators' own entry points refuse other flags
+        if (cd10 && (t[i].bc1 < -1 || t[i].bc1 > 1 || t[i].bcn < -1 || t[i].bcn > 1)) direct = false;
+    if (direct) {
+        ApplyTask a[8];
+        for (int i = 0; i < count; i++)
+            a[i] = {h->op[d], order == 1 ? KIND_D1 : KIND_D2, cd10 ? t[i].bc1 : 0, cd10 ? t[i].bcn : 0, t[i].f,
+                    t[i].out, t[i].sub, t[i].sub ? t[i].out : nullptr};
+        return apply_many(a, count, d + 1, prec, na, nb, st);
     }
     const long N = (long)h->nx * h->ny * h->nz;
     const bool dbl = prec == PDO_F64;
-    if (first) {
-        const hipError_t e = launch_zero_words(out, N * (dbl ? 2 : 1), st);
-        if (e != hipSuccess) return hip_fail(e, "zero fill");
+    for (int i = 0; i < count; i++) {
+        if (!t[i].sub) {
+            if ((r = h->apply(d, order, prec, t[i].f, t[i].out, t[i].bc1, t[i].bcn, st))) return r;
+            continue;
+        }
+        if (t[i].sub == 3) {
+            const hipError_t e = launch_zero_words(t[i].out, N * (dbl ? 2 : 1), st);
+            if (e != hipSuccess) return hip_fail(e, "zero fill");
+        }
+        if (h->n_of(d) == 1) continue;
+        if ((r = h->apply(d, order, prec, t[i].f, work, t[i].bc1, t[i].bcn, st))) return r;
+        const hipError_t e = launch_axpy(dbl, t[i].out, t[i].out, work, -1.0, N, st);
+        if (e != hipSuccess) return hip_fail(e, "derivative sum");
     }
-    if (h->n_of(d) == 1) return 0;
-    if ((r = h->apply(d, 1, prec, f, work, bc1, bcn, st))) return r;
-    const hipError_t e = launch_axpy(dbl, out, out, work, -1.0, N, st);
-    return e == hipSuccess ? 0 : hip_fail(e, "derivative sum");
+    return 0;
 }
 
-// whether one pass along d can apply the filter twice, and that pass
 bool filters_twice(pdo_filters h, int d, int prec)
 {
     if (h->method[d] == FIL_CF90 || prec_mode(prec) < 0) return false;
     return xfilter_can_twice(h->xf[d], d + 1);
 }
-int filters_apply_twice(pdo_filters h, int d, int prec, const void *f, void *ff, int bc1, int bcn, hipStream_t st)
+int filters_many(pdo_filters h, int d, int prec, const void *const *f, void *const *ff, int count, int times, int bc1,
+                 int bcn, hipStream_t st)
 {
-    int na, nb;
+    int na, nb, r;
     h->pencils(d, na, nb);
-    return xfilter_twice(h->xf[d], d + 1, prec, f, ff, na, nb, bc1, bcn, st);
+    if (h->method[d] != FIL_CF90) {
+        ExplicitFields F{};
+        for (int i = 0; i < count; i++) F.f[i] = f[i], F.out[i] = ff[i];
+        return xfilter_many(h->xf[d], d + 1, prec, F, count, times, na, nb, bc1, bcn, st);
+    }
+    for (int i = 0; i < count; i++)
+        if ((r = h->apply(d, prec, f[i], ff[i], bc1, bcn, st))) return r;
+    return 0;
 }
 
 }  // namespace pdo

@@ -61,8 +61,10 @@ __device__ __forceinline__ void filter_rows(const ExplicitArgs &E, const TW (&in
 
 // y and z: lanes over the pencils, blockIdx.y over chunks of T rows (chunked(n))
 template <typename TS, int NP>
-__global__ void __launch_bounds__(256) k_expl_strided(ExplicitArgs E, const TS *__restrict__ f, TS *__restrict__ out)
+__global__ void __launch_bounds__(256) k_expl_strided(ExplicitArgs E, ExplicitFields F)
 {
+    const TS *f = (const TS *)F.f[blockIdx.z];
+    TS *out = (TS *)F.out[blockIdx.z];
     const unsigned id = blockIdx.x * 256 + threadIdx.x, na = (unsigned)E.na;
     const unsigned pencils = na * (unsigned)E.nb;
     if (id >= pencils) return;
@@ -102,9 +104,10 @@ __global__ void __launch_bounds__(256) k_expl_strided(ExplicitArgs E, const TS *
 // x: `lines` whole lines per workgroup in LDS; element e is point
 // e % n of line e / n (magic: the rounded-up reciprocal of n)
 template <typename TS, int NP>
-__global__ void __launch_bounds__(256) k_expl_x(ExplicitArgs E, const TS *__restrict__ f, TS *__restrict__ out,
-                                               int lines, unsigned magic)
+__global__ void __launch_bounds__(256) k_expl_x(ExplicitArgs E, ExplicitFields F, int lines, unsigned magic)
 {
+    const TS *f = (const TS *)F.f[blockIdx.z];
+    TS *out = (TS *)F.out[blockIdx.z];
     extern __shared__ double lds[];
     const int n = E.n;
     const long l0 = (long)blockIdx.x * lines, left = (long)E.na * E.nb - l0;
@@ -204,13 +207,13 @@ static bool chunked(const ExplicitArgs &E)
 }
 
 template <typename TS, int NP>
-static bool launch_fast(const ExplicitArgs &E, const void *f, void *out, hipStream_t st)
+static bool launch_fast(const ExplicitArgs &E, const ExplicitFields &F, int count, hipStream_t st)
 {
     const long pencils = (long)E.na * E.nb;
     if (E.dir != 1) {
         if (!chunked(E)) return false;
-        const dim3 grid((unsigned)((pencils + 255) / 256), (unsigned)((E.n + EXPL_T - 1) / EXPL_T));
-        hipLaunchKernelGGL((k_expl_strided<TS, NP>), grid, dim3(256), 0, st, E, (const TS *)f, (TS *)out);
+        const dim3 grid((unsigned)((pencils + 255) / 256), (unsigned)((E.n + EXPL_T - 1) / EXPL_T), (unsigned)count);
+        hipLaunchKernelGGL((k_expl_strided<TS, NP>), grid, dim3(256), 0, st, E, F);
         return true;
     }
     // about 2048 points a workgroup (8 per thread), at most 64 KiB of LDS
@@ -218,29 +221,32 @@ static bool launch_fast(const ExplicitArgs &E, const void *f, void *out, hipStre
     const int lines = E.n < 2048 ? 2048 / E.n : 1;
     const size_t lds = (size_t)lines * E.n * (sizeof(TS) + (NP == 2 ? 8 : 0));
     const unsigned magic = (unsigned)(((unsigned long long)1 << 32) / E.n + 1);
-    hipLaunchKernelGGL((k_expl_x<TS, NP>), dim3((unsigned)((pencils + lines - 1) / lines)), dim3(256), lds, st, E,
-                       (const TS *)f, (TS *)out, lines, magic);
+    hipLaunchKernelGGL((k_expl_x<TS, NP>), dim3((unsigned)((pencils + lines - 1) / lines), 1, (unsigned)count),
+                       dim3(256), lds, st, E, F, lines, magic);
     return true;
 }
 
 bool explicit_twice(const ExplicitArgs &E) { return E.dir == 1 ? E.n <= 4096 : chunked(E); }
 
-hipError_t launch_explicit(bool dbl, const ExplicitArgs &E, const void *f, void *out, hipStream_t st, int times)
+hipError_t launch_explicit(bool dbl, const ExplicitArgs &E, const ExplicitFields &F, int count, hipStream_t st,
+                           int times)
 {
     const long total = (long)E.n * E.na * E.nb;
     if (total <= 0) return hipSuccess;
-    const bool done = times == 2 ? (dbl ? launch_fast<double, 2>(E, f, out, st) : launch_fast<float, 2>(E, f, out, st))
-                                 : (dbl ? launch_fast<double, 1>(E, f, out, st) : launch_fast<float, 1>(E, f, out, st));
+    const bool done = times == 2 ? (dbl ? launch_fast<double, 2> : launch_fast<float, 2>)(E, F, count, st)
+                                 : (dbl ? launch_fast<double, 1> : launch_fast<float, 1>)(E, F, count, st);
     if (done) return hipGetLastError();
     if (times == 2) return hipErrorInvalidValue;
     long blocks = (total + 255) / 256;
     if (blocks > 1 << 20) blocks = 1 << 20;
-    if (dbl)
-        hipLaunchKernelGGL((k_explicit<double, double>), dim3((unsigned)blocks), dim3(256), 0, st, E,
-                           (const double *)f, (double *)out);
-    else
-        hipLaunchKernelGGL((k_explicit<float, double>), dim3((unsigned)blocks), dim3(256), 0, st, E,
-                           (const float *)f, (float *)out);
+    for (int i = 0; i < count; i++) {
+        if (dbl)
+            hipLaunchKernelGGL((k_explicit<double, double>), dim3((unsigned)blocks), dim3(256), 0, st, E,
+                               (const double *)F.f[i], (double *)F.out[i]);
+        else
+            hipLaunchKernelGGL((k_explicit<float, double>), dim3((unsigned)blocks), dim3(256), 0, st, E,
+                               (const float *)F.f[i], (float *)F.out[i]);
+    }
     return hipGetLastError();
 }
 

@@ -20,14 +20,21 @@ struct ExplicitArgs {
     double right[EXPL_NB * EXPL_WB];      // rows n-4..n-1 against points n-8..n-1
 };
 
-// the filter applied `times` (1, or 2 where explicit_twice) times
-hipError_t launch_explicit(bool dbl, const ExplicitArgs &E, const void *f, void *out, hipStream_t st, int times = 1);
+// up to three fields of one call (grid z)
+struct ExplicitFields {
+    const void *f[3];
+    void *out[3];
+};
+
+// the filter applied `times` (1, or 2 where explicit_twice) times to each field
+hipError_t launch_explicit(bool dbl, const ExplicitArgs &E, const ExplicitFields &F, int count, hipStream_t st,
+                           int times);
 bool explicit_twice(const ExplicitArgs &E);
-// two applications of an explicit filter along dir in one pass, where
-// xfilter_can_twice
+// the filter along dir, `times` times (1, or 2 where xfilter_can_twice), on
+// each of count (at most 3) fields
 bool xfilter_can_twice(pdo_xfilter h, int dir);
-int xfilter_twice(pdo_xfilter h, int dir, int prec, const void *f, void *fil, long na, long nb, int bc1, int bcn,
-                  hipStream_t st);
+int xfilter_many(pdo_xfilter h, int dir, int prec, const ExplicitFields &F, int count, int times, long na, long nb,
+                 int bc1, int bcn, hipStream_t st);
 // out = a + s b, elementwise over n values (FP64 arithmetic)
 hipError_t launch_axpy(bool dbl, void *out, const void *a, const void *b, double s, long n, hipStream_t st);
 

@@ -43,6 +43,7 @@ __global__ void __launch_bounds__(1024) k_fft_strided(const TS *src, TS *dst, lo
     const long a = (long)bx * TX + ln;
     const bool act = a < na;
     const long off = 2 * ((act ? a : 0) + (long)by * sb);
+    if (MODE == 2 && blockIdx.z) src = dst = (TS *)pm.more[blockIdx.z - 1];
     const TS *const lin = src + off;
     TS *const lout = dst + off;
     const C2<TC> *tw = (const C2<TC> *)twL;
@@ -335,7 +336,7 @@ static void launch_strided_fft(const TS *src, TS *dst, long na, long sb, long se
 {
     constexpr size_t ce = 2 * sizeof(TC);
     constexpr int TX = strided_fft_lines<L, ce, MODE>();
-    dim3 grid((unsigned)((na + TX - 1) / TX), (unsigned)nb);
+    dim3 grid((unsigned)((na + TX - 1) / TX), (unsigned)nb, MODE == 2 ? (unsigned)pm.fields : 1u);
     hipLaunchKernelGGL((k_fft_strided<TS, TC, MODE, L, TX>), grid, dim3(TX * (L / 8)),
                        (size_t)(TX + (PDO_FFT_TW_LDS ? 1 : 0)) * L * ce +
                            ((PDO_FFT_TW_LDS && MODE == 2) ? (size_t)L * sizeof(TC) : 0),

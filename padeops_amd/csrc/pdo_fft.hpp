@@ -17,6 +17,9 @@ struct SpecMul {
     const double *ax, *ay, *az;
     int kind;
     double scale;
+    // run_zmul: further fields of the same launch, in place (grid z)
+    void *more[2] = {nullptr, nullptr};
+    int fields = 1;
 };
 
 struct PoissonPlanDev {

@@ -183,32 +183,29 @@ int igrid_fields(pdo_duidxj h, int prec, const pdo_interp_fields &I, const pdo_d
     auto HC = [&](int k) { return at(D.duidxjChat, cC, k); };
     auto HE = [&](int k) { return at(D.duidxjEhat, cE, k); };
     const int *bc = h->bc;
-    auto z = [&](int kind, int b, int t, const void *in, void *out) {
-        return pdo_pade6stagg_apply(h->dz, kind, b, t, prec, in, out, nxh, ny, 1, (void *)st);
+    auto z = [&](std::initializer_list<StaggTask> t) {
+        return pade6stagg_many(h->dz, t.begin(), (int)t.size(), prec, nxh, ny, st);
     };
     int r;
 #define PDO_TRY(x)               \
     do {                         \
         if ((r = (x))) return r; \
     } while (0)
-    // igrid.F90:1423-1463 and :2621-2679 in spectral space
-    PDO_TRY(z(14, bc[4], bc[5], I.what, I.whatC));
-    PDO_TRY(z(15, bc[0], bc[1], I.uhat, I.uEhat));
-    PDO_TRY(z(15, bc[2], bc[3], I.vhat, I.vEhat));
-    PDO_TRY(z(10, bc[4], bc[5], I.what, HC(9)));
-    PDO_TRY(z(15, bc[10], bc[11], HC(9), HE(9)));
-    if (!h->inviscid) PDO_TRY(z(13, bc[4], bc[5], I.what, D.d2wdz2hatE));
-    const void *uv[2] = {I.uhat, I.vhat};
-    void *d2[2] = {D.d2udz2hatC, D.d2vdz2hatC};
-    for (int q = 0; q < 2; q++) {
-        const int b = bc[2 * q], t = bc[2 * q + 1], db = bc[6 + 2 * q], dt = bc[7 + 2 * q], k = 3 + 3 * q;
-        PDO_TRY(z(11, b, t, uv[q], HE(k)));
-        if (!h->inviscid) {
-            // a one-sided boundary takes the second derivative as E2C(C2E(.))
-            if (t == 0 || b == 0) PDO_TRY(z(10, db, dt, HE(k), d2[q]));
-            else PDO_TRY(z(12, b, t, uv[q], d2[q]));
-        }
-        PDO_TRY(z(14, db, dt, HE(k), HC(k)));
+    // igrid.F90:1423-1463 and :2621-2679 in spectral space, calls of a kind
+    // together
+    PDO_TRY(z({{10, bc[4], bc[5], I.what, HC(9)}}));
+    PDO_TRY(z({{11, bc[0], bc[1], I.uhat, HE(3)}, {11, bc[2], bc[3], I.vhat, HE(6)}}));
+    PDO_TRY(z({{15, bc[0], bc[1], I.uhat, I.uEhat}, {15, bc[2], bc[3], I.vhat, I.vEhat}, {15, bc[10], bc[11], HC(9), HE(9)}}));
+    PDO_TRY(z({{14, bc[4], bc[5], I.what, I.whatC}, {14, bc[6], bc[7], HE(3), HC(3)}, {14, bc[8], bc[9], HE(6), HC(6)}}));
+    if (!h->inviscid) {
+        // a one-sided boundary takes the second derivative as E2C(C2E(.))
+        auto second = [&](int q, const void *f, const void *fz, void *out) {
+            const bool sided = bc[2 * q] == 0 || bc[2 * q + 1] == 0;
+            return sided ? StaggTask{10, bc[6 + 2 * q], bc[7 + 2 * q], fz, out}
+                         : StaggTask{12, bc[2 * q], bc[2 * q + 1], f, out};
+        };
+        PDO_TRY(z({second(0, I.uhat, HE(3), D.d2udz2hatC), second(1, I.vhat, HE(6), D.d2vdz2hatC),
+                   {13, bc[4], bc[5], I.what, D.d2wdz2hatE}}));
     }
 #undef PDO_TRY
     const InvTask task[12] = {
@@ -415,9 +412,8 @@ static int sgsrhs_compute(pdo_sgsrhs h, int prec, const void *duidxjC, const voi
         task[q].planes = q < 4 ? nz : nz + 1;
     }
     PDO_HIP(run_fwd_multi(C.plan, mode, task, 6, st), "stress transforms");
-    for (int q = 0; q < 2; q++)
-        PDO_TRY(pdo_pade6stagg_apply(h->dz, 10, 0, 0, prec, h->hE[q], h->zC[q], nxh, ny, 1, stream));
-    PDO_TRY(pdo_pade6stagg_apply(h->dz, 11, 0, 0, prec, h->hC[3], h->zE, nxh, ny, 1, stream));
+    const StaggTask zt[3] = {{10, 0, 0, h->hE[0], h->zC[0]}, {10, 0, 0, h->hE[1], h->zC[1]}, {11, 0, 0, h->hC[3], h->zE}};
+    PDO_TRY(pade6stagg_many(h->dz, zt, 3, prec, nxh, ny, st));
     const StressSpectra S{h->hC[0], h->hC[1], h->hC[2], h->zC[0], h->zC[1], h->zE, h->hE[0], h->hE[1]};
     PDO_HIP(launch_stress_div(mode, urhs, vrhs, wrhs, S, C.d_k1, C.d_k2, nxh, ny, (long)h->sC, (long)h->sE, st), "rhs");
 #undef PDO_TRY

@@ -63,6 +63,14 @@ hipError_t launch_wall_model(int mode, const void *u, const void *v, void *tauE,
                              int nb, double kappa, double lg, double *wm, hipStream_t st);
 // whether a Pade6stagg object is periodic (pdo_pade6.cpp)
 bool pade6stagg_periodic(pdo_pade6stagg h);
+// independent pdo_pade6stagg_apply calls on complex (n1, n2) lines, those of
+// one kind sharing launches for small fields (at most 8)
+struct StaggTask {
+    int kind, bot, top;
+    const void *in;
+    void *out;
+};
+int pade6stagg_many(pdo_pade6stagg h, const StaggTask *t, int count, int prec, int n1, int n2, hipStream_t st);
 
 struct BandLimit;
 // interp_PrimitiveVars and compute_duidxj of dealiased spectra in one go: the

@@ -133,8 +133,11 @@ int dealias_fields(pdo_igrid h, void *uh, void *vh, void *wh, bool masked, hipSt
     }
     if (h->p.walls) return 0;
     const SpectralObject &C = *h->spC;
-    const SpecMul m{C.d_g1, C.d_g2, C.d_g3, 2, 1.0 / h->nz};
-    for (void *f : {uh, vh, wh}) PDO_HIP(run_zmul(C.plan, h->mode, f, f, m, st, h->band.kxc), "dealias");
+    SpecMul m{C.d_g1, C.d_g2, C.d_g3, 2, 1.0 / h->nz};
+    m.more[0] = vh;
+    m.more[1] = wh;
+    m.fields = 3;
+    PDO_HIP(run_zmul(C.plan, h->mode, uh, uh, m, st, h->band.kxc), "dealias");
     // edge nz + 1 repeats edge 1
     const size_t plane = (size_t)h->nxh * h->ny * 2 * h->W;
     PDO_HIP(hipMemcpyAsync((char *)wh + plane * h->nz, wh, plane, hipMemcpyDeviceToDevice, st), "dealias");
@@ -183,8 +186,8 @@ int populate_rhs(pdo_igrid h, void *ur, void *vr, void *wr, hipStream_t st)
                              {gE(8), gE(6), h->w, nullptr, nullptr, nullptr, fE[1], h->nz + 1},
                              {gE(3), gE(7), h->uE, gE(6), gE(8), h->vE, wr, h->nz + 1}};
     PDO_HIP(run_fwd_multi(h->spC->plan, mode, task, 5, st), "nonlinear");
-    PDO_TRY(pdo_pade6stagg_apply(h->d6, 14, 0, 0, h->prec, fE[0], ur, h->nxh, h->ny, 1, s));
-    PDO_TRY(pdo_pade6stagg_apply(h->d6, 14, 0, 0, h->prec, fE[1], vr, h->nxh, h->ny, 1, s));
+    const StaggTask zt[2] = {{14, 0, 0, fE[0], ur}, {14, 0, 0, fE[1], vr}};
+    PDO_TRY(pade6stagg_many(h->d6, zt, 2, h->prec, h->nxh, h->ny, st));
     // ... and Step 5: addViscousTerm (:1914-1959)
     const RhsTerms T{{ur, vr, wr}, {fC[0], fC[1], nullptr}, {h->cur_u, h->cur_v, h->cur_w}, {h->d2u, h->d2v, h->d2w}};
     PDO_HIP(launch_rhs_terms(mode, T, h->spC->d_k1, h->spC->d_k2, h->nxh, h->ny, (long)(h->sC / 2), (long)(h->sE / 2),

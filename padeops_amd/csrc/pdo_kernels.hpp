@@ -45,9 +45,24 @@ struct ApplyArgs {
     double band[5];    // interior LHS band (offsets -2..2), used by periodic systems
 };
 
+// passes of one launch: independent, of one system size, family and direction
+// (grid z picks the pass).  Kernels take the arguments of a single pass or of
+// several: with the pass picked at run time some need 3 to 20 registers more,
+// and the refined pentadiagonal solves spill (cd10 strided 772 bytes).
+constexpr int MAX_BATCH = 5;
+struct ApplyBatch {
+    ApplyArgs a[MAX_BATCH];
+};
+__device__ __forceinline__ const ApplyArgs &pass_of(const ApplyArgs &A) { return A; }
+__device__ __forceinline__ const ApplyArgs &pass_of(const ApplyBatch &B) { return B.a[blockIdx.z]; }
+
+// modes and families with kernels for several passes
+constexpr bool can_batch(int K, int mode) { return mode == MODE_F64 || (mode == MODE_F32R && K == 1); }
+
 hipError_t launch_absmax(const void *x, bool is_double, long n, double *partial, int nblocks, hipStream_t st);
 hipError_t launch_zero_words(void *p, long words, hipStream_t st);
-hipError_t launch_overlap(int family, int shape, bool dbl, const ApplyArgs &A, hipStream_t st);
-hipError_t launch_compact(int family, int shape, int mode, const ApplyArgs &A, double *scratch, hipStream_t st);
+hipError_t launch_overlap(int family, int shape, bool dbl, ApplyBatch &B, int count, hipStream_t st);
+hipError_t launch_compact(int family, int shape, int mode, const ApplyBatch &B, int count, double *scratch,
+                          hipStream_t st);
 
 }  // namespace pdo

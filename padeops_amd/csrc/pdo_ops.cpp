@@ -189,7 +189,7 @@ static bool overlap_fits(const Variant &v, int dir, long na, long nb, size_t wor
 // Validate one apply call and fill its launch arguments; *empty is set when
 // there is nothing to do (na or nb zero).
 static int prepare(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, const void *f, void *out, long na,
-                   long nb, int epi, const void *aux, int force_shape, ApplyArgs &A, int &shape, int &mode,
+                   long nb, int epi, const void *aux, int force_shape, bool several, ApplyArgs &A, int &shape, int &mode,
                    int &family, size_t &scratch_elems, bool *empty, bool noalloc = false)
 {
     *empty = false;
@@ -236,11 +236,13 @@ static int prepare(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, 
     // an extra row in the last segment only in the tridiagonal families
     if (shape == SHAPE_STRIDED && !s.periodic && (epi || (v->fast.tab.xr && family_shape(s.family).K != 1)))
         shape = SHAPE_GENERAL;
+    // only the first derivatives of cd06 and cd10 have epilogues there
+    const bool epi_ok = !epi || s.family == FAM_CD06_D1 || s.family == FAM_CD10_D1;
     // sizes and ends without a register kernel of their own: overlapping
     // segments, where they fit (n >= 16, at most 512 rows, 1024 of the
     // collocated operators), else one lane per pencil
     scratch_elems = (shape == SHAPE_GENERAL) ? (size_t)s.n_sys * (size_t)(na * nb) : 0;
-    if (shape == SHAPE_GENERAL && force_shape != SHAPE_GENERAL && (!epi || s.n_out == s.n_sys) &&
+    if (shape == SHAPE_GENERAL && force_shape != SHAPE_GENERAL && epi_ok &&
         overlap_fits(*v, dir, na, nb, word))
         shape = dir == 1 ? SHAPE_OVL_X : SHAPE_OVL_STRIDED;
     // FP32 + refinement without periodicity: the refined kernels carry two
@@ -252,6 +254,12 @@ static int prepare(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, 
     if (shape == SHAPE_STRIDED && !s.periodic && mode == MODE_F32R && v->ovl.P <= PMAX &&
         overlap_fits(*v, dir, na, nb, word))
         shape = SHAPE_OVL_STRIDED;
+    // several refined pentadiagonal passes over a small field: the register
+    // kernels have no launch of several passes (can_batch)
+    if (several && (shape == SHAPE_STRIDED || shape == SHAPE_X) && mode == MODE_F32R &&
+        !can_batch(family_shape(s.family).K, mode) && v->ovl.P <= PMAX && epi_ok &&
+        small_field(s.n_sys * na * nb, prec) && overlap_fits(*v, dir, na, nb, word))
+        shape = dir == 1 ? SHAPE_OVL_X : SHAPE_OVL_STRIDED;
     TabSet *ts = &v->fast;
     if (shape == SHAPE_GENERAL && !v->fast.tab.general) {
         // built with the variant
@@ -300,40 +308,78 @@ static int prepare(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, 
     return 0;
 }
 
-// launch of a prepared call; `work` serves the general kernel
-static hipError_t launch(int family, int shape, int mode, const ApplyArgs &A, double *work, hipStream_t stream)
+// launch of prepared calls; `work` serves the general kernel
+static hipError_t launch(int family, int shape, int mode, ApplyBatch &B, int count, double *work, hipStream_t stream)
 {
     if (shape == SHAPE_OVL_X || shape == SHAPE_OVL_STRIDED)
-        return launch_overlap(family, shape, mode == MODE_F64, A, stream);
-    return launch_compact(family, shape, mode, A, work, stream);
+        return launch_overlap(family, shape, mode == MODE_F64, B, count, stream);
+    return launch_compact(family, shape, mode, B, count, work, stream);
+}
+
+// whether a shape has kernels for several passes
+static bool may_join(int shape, int mode, int family)
+{
+    if (shape == SHAPE_OVL_X || shape == SHAPE_OVL_STRIDED) return true;
+    return shape != SHAPE_GENERAL && can_batch(family_shape(family).K, mode);
+}
+
+bool small_field(long points, int prec)
+{
+    return prec == PDO_F64 ? points * 8 <= (long)SMALL_F64 : points * 4 <= (long)SMALL_F32;
+}
+
+int apply_many(const ApplyTask *tasks, int count, int dir, int prec, long na, long nb, hipStream_t stream)
+{
+    ApplyBatch B;
+    int held = 0, shape0 = 0, mode0 = 0, family0 = 0;
+    auto flush = [&]() -> int {
+        if (!held) return 0;
+        const hipError_t e = launch(family0, shape0, mode0, B, held, nullptr, stream);
+        held = 0;
+        return e == hipSuccess ? 0 : hip_fail(e, "kernel launch");
+    };
+    for (int i = 0; i < count; i++) {
+        const ApplyTask &t = tasks[i];
+        ApplyArgs A;
+        int shape = 0, mode = 0, family = 0;
+        size_t scratch_elems = 0;
+        bool empty = false;
+        int st = prepare(t.op, t.kind, t.bc1, t.bcn, dir, prec, t.f, t.out, na, nb, t.epi, t.aux, t.force_shape,
+                         count > 1, A, shape, mode, family, scratch_elems, &empty);
+        if (st) return st;
+        if (empty) continue;
+        // one launch serves passes whose grid, workgroup and kernel agree
+        const ApplyArgs &F = B.a[0];
+        const bool join = held > 0 && held < MAX_BATCH && may_join(shape, mode, family) && shape == shape0 && mode == mode0 && family == family0 &&
+                          small_field(A.n_sys * na * nb, prec) && A.periodic == F.periodic &&
+                          A.n_sys == F.n_sys && A.n_in == F.n_in && A.n_out == F.n_out && A.m == F.m && A.P == F.P &&
+                          A.xr == F.xr && (A.epi != 0) == (F.epi != 0);
+        if (!join && (st = flush())) return st;
+        if (shape == SHAPE_GENERAL) {
+            // the general kernel's work area is stream-ordered memory of this
+            // pass alone: no host synchronisation, and no sharing between
+            // launches that run concurrently on different streams
+            double *scratch = nullptr;
+            hipError_t e = hipMallocAsync((void **)&scratch, scratch_elems * sizeof(double), stream);
+            if (e != hipSuccess) return hip_fail(e, "hipMallocAsync(general-kernel work area)");
+            B.a[0] = A;
+            e = launch(family, shape, mode, B, 1, scratch, stream);
+            const hipError_t ef = hipFreeAsync(scratch, stream);
+            if (e == hipSuccess) e = ef;
+            if (e != hipSuccess) return hip_fail(e, "kernel launch");
+            continue;
+        }
+        B.a[held++] = A;
+        shape0 = shape; mode0 = mode; family0 = family;
+    }
+    return flush();
 }
 
 int apply(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, const void *f, void *out, long na, long nb,
           hipStream_t stream, int epi, const void *aux, int force_shape)
 {
-    ApplyArgs A;
-    int shape = 0, mode = 0, family = 0;
-    size_t scratch_elems = 0;
-    bool empty = false;
-    int st = prepare(op, kind, bc1, bcn, dir, prec, f, out, na, nb, epi, aux, force_shape, A, shape, mode, family,
-                     scratch_elems, &empty);
-    if (st || empty) return st;
-    // the general kernel's work area is stream-ordered memory of this call
-    // alone: no host synchronisation, and no sharing between launches that
-    // run concurrently on different streams
-    double *scratch = nullptr;
-    hipError_t e = hipSuccess;
-    if (shape == SHAPE_GENERAL) {
-        e = hipMallocAsync((void **)&scratch, scratch_elems * sizeof(double), stream);
-        if (e != hipSuccess) return hip_fail(e, "hipMallocAsync(general-kernel work area)");
-    }
-    e = launch(family, shape, mode, A, scratch, stream);
-    if (scratch) {
-        const hipError_t ef = hipFreeAsync(scratch, stream);
-        if (e == hipSuccess) e = ef;
-    }
-    if (e != hipSuccess) return hip_fail(e, "kernel launch");
-    return 0;
+    const ApplyTask t{op, kind, bc1, bcn, f, out, epi, aux, force_shape};
+    return apply_many(&t, 1, dir, prec, na, nb, stream);
 }
 
 int apply_noalloc(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, const void *f, void *out, long na,
@@ -364,7 +410,7 @@ int apply_noalloc(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, c
     int shape = 0, mode = 0, family = 0;
     size_t scratch_elems = 0;
     bool empty = false;
-    int st = prepare(op, kind, bc1, bcn, dir, prec, f, out, na, nb, 0, nullptr, -1, A, shape, mode, family,
+    int st = prepare(op, kind, bc1, bcn, dir, prec, f, out, na, nb, 0, nullptr, -1, false, A, shape, mode, family,
                      scratch_elems, &empty, true);
     if (st || empty) return st;
     // the limit is the entry point's contract for every call outside the fixed
@@ -374,7 +420,9 @@ int apply_noalloc(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, c
                   std::to_string(scratch_elems) + " > " + std::to_string(work_elems) + " FP64 words)");
         return PDO_ERR_ARG;
     }
-    const hipError_t e = launch(family, shape, mode, A, shape == SHAPE_GENERAL ? work : nullptr, stream);
+    ApplyBatch B;
+    B.a[0] = A;
+    const hipError_t e = launch(family, shape, mode, B, 1, shape == SHAPE_GENERAL ? work : nullptr, stream);
     if (e != hipSuccess) return hip_fail(e, "kernel launch");
     return 0;
 }

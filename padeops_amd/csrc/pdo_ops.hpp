@@ -61,6 +61,31 @@ struct OpObject {
 int apply(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, const void *f, void *out, long na, long nb,
           hipStream_t stream, int epi = 0, const void *aux = nullptr, int force_shape = -1);
 
+// Independent passes along one direction of fields of one shape (no output
+// read by another), in order but for those that share a launch: see
+// small_field.
+struct ApplyTask {
+    OpObject *op;
+    int kind, bc1, bcn;
+    const void *f;
+    void *out;
+    int epi = 0;
+    const void *aux = nullptr;
+    int force_shape = -1;
+};
+int apply_many(const ApplyTask *tasks, int count, int dir, int prec, long na, long nb, hipStream_t stream);
+
+// whether passes over fields of this size share launches: a launch of one pass
+// over a small field leaves most of the chip idle for its latency.  A cgrid
+// RHS in launches of one pass and of up to MAX_BATCH (us): FP64 64^3 471 ->
+// 192, 128^3 1107 -> 810, 160^3 2118 -> 1744, 192^3 3249 -> 3004 (54 MiB per
+// field; beyond, passes over one field after the other find it in the Infinity
+// Cache); FP32 + refine 96^3 716 -> 369, 128^3 853 -> 675, 160^3 1417 -> 1295
+// and 192^3 1893 -> 2102 (27 MiB; several pentadiagonal passes run on
+// overlapping segments).
+constexpr size_t SMALL_F64 = 64u << 20, SMALL_F32 = 16u << 20;  // bytes per field
+bool small_field(long points, int prec);
+
 // apply() without any device allocation, for pdo_op_apply_noalloc: the
 // variant must already be built, and the general kernel's work area is
 // `work` (work_elems FP64 words); larger inputs are rejected

@@ -225,9 +225,10 @@ struct NotStaged {
     __device__ __forceinline__ void write(double *) const {}
 };
 
-template <int FAM, typename TS, int M, int NPW, bool LT>
-__global__ void __launch_bounds__(1024) k_ovl_strided(ApplyArgs A)
+template <int FAM, typename TS, int M, int NPW, bool LT, bool EPI, typename ARGS>
+__global__ void __launch_bounds__(1024) k_ovl_strided(ARGS B)
 {
+    const ApplyArgs &A = pass_of(B);
     using F = Fam<FAM>;
     constexpr int K = F::K, R = F::R, W = M + 2 * R;
     constexpr bool UNI = NPW == 64;
@@ -287,7 +288,7 @@ __global__ void __launch_bounds__(1024) k_ovl_strided(ApplyArgs A)
     if (!act) return;
     const unsigned vo = (a + b * (unsigned)A.sb_out) * (unsigned)sizeof(TS);
     char *ob = (char *)A.out + (size_t)blockIdx.y * A.sb_out * sizeof(TS);
-    if (A.epi) {
+    if constexpr (EPI) {
         // the operand's rows in chunks, read before the chunk's rows are
         // written (it may be the output)
         const char *xb = (const char *)A.aux + (size_t)blockIdx.y * A.sb_out * sizeof(TS);
@@ -326,9 +327,10 @@ __global__ void __launch_bounds__(1024) k_ovl_strided(ApplyArgs A)
 // odd pitch LD sends the lanes of a half-wave, which read one row each of
 // neighbouring pencils, to distinct banks.
 // ---------------------------------------------------------------------------
-template <int FAM, typename TS, int M, bool LT>
-__global__ void __launch_bounds__(512) k_ovl_x(ApplyArgs A, int TP, int LD, unsigned magic)
+template <int FAM, typename TS, int M, bool LT, bool EPI, typename ARGS>
+__global__ void __launch_bounds__(512) k_ovl_x(ARGS B, int TP, int LD, unsigned magic)
 {
+    const ApplyArgs &A = pass_of(B);
     using F = Fam<FAM>;
     constexpr int K = F::K, R = F::R, W = M + 2 * R;
     const int P = A.P, n = A.n_sys, nt = TP * P;
@@ -377,16 +379,55 @@ __global__ void __launch_bounds__(512) k_ovl_x(ApplyArgs A, int TP, int LD, unsi
     for (int j = 0; j < M; ++j)
         if (j < own) line[r0 + j] = (TS)d[j];
     __syncthreads();
-    TS *out = (TS *)A.out + pen0 * n;
-    const TS *aux = (const TS *)A.aux + (A.epi == 1 || A.epi == 2 ? pen0 * n : 0);  // may be out
+    TS *__restrict__ out = (TS *)A.out + pen0 * n;
+    if constexpr (!EPI) {
 #pragma unroll 8
-    for (int e = threadIdx.x; e < total; e += nt) {
-        const int q = (int)__umulhi((unsigned)e, magic);
-        const TS y = tile[e + (q & -pad)];
-        out[e] = A.epi == 0 ? y
-                            : (A.epi == 1 ? (TS)((double)aux[e] + (double)y)
-                                          : (TS)((A.epi == 2 ? (double)aux[e] : 0.0) - (double)y));
+        for (int e = threadIdx.x; e < total; e += nt) {
+            const int q = (int)__umulhi((unsigned)e, magic);
+            out[e] = tile[e + (q & -pad)];
+        }
+        return;
     }
+    TS *o = (TS *)A.out + pen0 * n;  // may be the operand
+    const TS *aux = (const TS *)A.aux + (A.epi == 3 ? 0 : pen0 * n);
+    for (int e0 = threadIdx.x; e0 < total; e0 += 4 * nt) {
+        double x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = e0 + i * nt;
+            x[i] = A.epi != 3 && e < total ? (double)aux[e] : 0.0;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = e0 + i * nt;
+            if (e >= total) break;
+            const int q = (int)__umulhi((unsigned)e, magic);
+            const double y = (double)tile[e + (q & -pad)];
+            o[e] = (TS)(A.epi == 1 ? x[i] + y : x[i] - y);
+        }
+    }
+}
+
+// the kernel for one pass or for several
+template <class K1, class KB, class... X>
+void go(K1 one, KB several, int count, dim3 grid, dim3 block, size_t lds, hipStream_t st, const ApplyBatch &B, X... x)
+{
+    if (count > 1) hipLaunchKernelGGL(several, grid, block, lds, st, B, x...);
+    else hipLaunchKernelGGL(one, grid, block, lds, st, B.a[0], x...);
+}
+
+// f(EPI): the first derivatives have kernels with an epilogue operand
+template <int FAM, class F> hipError_t with_epilogue(const ApplyArgs &A, F f)
+{
+    if constexpr (FAM == 0 || FAM == 2) {
+        if (A.epi) {
+            f(std::true_type{});
+            return hipGetLastError();
+        }
+    }
+    if (A.epi) return hipErrorInvalidValue;
+    f(std::false_type{});
+    return hipGetLastError();
 }
 
 // coupling rows staged in LDS up to 4 KiB: the ones of long pencils would
@@ -397,86 +438,108 @@ template <int K> int staged_words(const ApplyArgs &A)
     return words <= 512 ? words : 0;
 }
 
-template <int FAM, typename TS, int M> hipError_t strided_m(ApplyArgs A, hipStream_t st)
+template <int FAM, typename TS, int M> hipError_t strided_m(ApplyBatch &B, int count, hipStream_t st)
 {
     constexpr int K = Fam<FAM>::K;
-    A.glds = A.P > PMAX ? staged_words<K>(A) : 0;
+    const ApplyArgs &A = B.a[0];
+    int glds = 0;
+    for (int i = 0; i < count; i++) {
+        B.a[i].glds = A.P > PMAX ? staged_words<K>(B.a[i]) : 0;
+        glds = B.a[i].glds > glds ? B.a[i].glds : glds;
+    }
     // pencils numbered through where 32-bit offsets reach the whole field
     const size_t nmax = (size_t)(A.n_in > A.n_out ? A.n_in : A.n_out);
     const size_t bytes = (size_t)A.na * A.nb * nmax * sizeof(TS);
-    A.lgn = bytes < ((size_t)1 << 32) ? 1 : 0;
+    for (int i = 0; i < count; i++) B.a[i].lgn = bytes < ((size_t)1 << 32) ? 1 : 0;
     const size_t pen = A.lgn ? (size_t)A.na * A.nb : (size_t)A.na;
     if (!A.lgn && (A.nb > 65535 || (size_t)A.na * sizeof(TS) >= ((size_t)1 << 32))) return hipErrorInvalidValue;
     if (A.P <= PMAX) {
-        const dim3 grid((unsigned)((pen + 63) / 64), A.lgn ? 1u : (unsigned)A.nb);
-        hipLaunchKernelGGL((k_ovl_strided<FAM, TS, M, 64, false>), grid, dim3(64 * A.P),
-                           (size_t)A.P * 2 * K * 64 * sizeof(double), st, A);
-        return hipGetLastError();
+        const dim3 grid((unsigned)((pen + 63) / 64), A.lgn ? 1u : (unsigned)A.nb, (unsigned)count);
+        const size_t red = (size_t)A.P * 2 * K * 64 * sizeof(double);
+        return with_epilogue<FAM>(A, [&](auto e) {
+            constexpr bool E = decltype(e)::value;
+            go(k_ovl_strided<FAM, TS, M, 64, false, E, ApplyArgs>, k_ovl_strided<FAM, TS, M, 64, false, E, ApplyBatch>,
+               count, grid, dim3(64 * A.P), red, st, B);
+        });
     }
     if constexpr (M == MAXM && Fam<FAM>::SHIFT == 0) {
         if (!A.lgn) return hipErrorInvalidValue;
-        const dim3 grid((unsigned)((pen + 31) / 32));
-        const size_t red = ((size_t)A.P * 2 * K * 32 + A.glds) * sizeof(double);
-        if (A.periodic)
-            hipLaunchKernelGGL((k_ovl_strided<FAM, TS, M, 32, false>), grid, dim3(32 * A.P), red, st, A);
-        else
-            hipLaunchKernelGGL((k_ovl_strided<FAM, TS, M, 32, true>), grid, dim3(32 * A.P),
-                               red + sizeof(double) * 3 * (type_words<K, M>()), st, A);
-        return hipGetLastError();
+        const dim3 grid((unsigned)((pen + 31) / 32), 1u, (unsigned)count);
+        const size_t red = ((size_t)A.P * 2 * K * 32 + glds) * sizeof(double);
+        const size_t tabs = sizeof(double) * 3 * type_words<K, M>();
+        return with_epilogue<FAM>(A, [&](auto e) {
+            constexpr bool E = decltype(e)::value;
+            if (A.periodic)
+                go(k_ovl_strided<FAM, TS, M, 32, false, E, ApplyArgs>,
+                   k_ovl_strided<FAM, TS, M, 32, false, E, ApplyBatch>, count, grid, dim3(32 * A.P), red, st, B);
+            else
+                go(k_ovl_strided<FAM, TS, M, 32, true, E, ApplyArgs>,
+                   k_ovl_strided<FAM, TS, M, 32, true, E, ApplyBatch>, count, grid, dim3(32 * A.P), red + tabs, st, B);
+        });
     }
     return hipErrorInvalidValue;
 }
 
-template <int FAM, typename TS, int M> hipError_t x_m(ApplyArgs A, hipStream_t st)
+template <int FAM, typename TS, int M> hipError_t x_m(ApplyBatch &B, int count, hipStream_t st)
 {
     constexpr int K = Fam<FAM>::K;
-    A.glds = staged_words<K>(A);
+    const ApplyArgs &A = B.a[0];
+    int glds = 0;
+    for (int i = 0; i < count; i++) {
+        B.a[i].glds = staged_words<K>(B.a[i]);
+        glds = B.a[i].glds > glds ? B.a[i].glds : glds;
+    }
     const int n = A.n_sys, LD = n | 1;
-    const size_t tabs = ((A.periodic ? 0 : (A.P == 1 ? 1 : 3) * type_words<K, M>()) + (size_t)A.glds) * sizeof(double);
+    const size_t tabs = ((A.periodic ? 0 : (A.P == 1 ? 1 : 3) * type_words<K, M>()) + (size_t)glds) * sizeof(double);
     auto lds = [&](int tp) { return (size_t)tp * (LD * sizeof(TS) + A.P * 2 * K * sizeof(double)) + tabs; };
     // two workgroups on a CU (80 KiB each), at most 512 threads
     int TP = 32;
     while (TP > 8 && (TP * A.P > 512 || lds(TP) > 80 * 1024)) TP >>= 1;
     if (TP * A.P > 512 || lds(TP) > 160 * 1024) return hipErrorInvalidValue;
     const unsigned magic = (unsigned)(((unsigned long long)1 << 32) / n + 1);
-    const dim3 grid((unsigned)((A.na * A.nb + TP - 1) / TP));
-    if (A.periodic)
-        hipLaunchKernelGGL((k_ovl_x<FAM, TS, M, false>), grid, dim3(TP * A.P), lds(TP), st, A, TP, LD, magic);
-    else
-        hipLaunchKernelGGL((k_ovl_x<FAM, TS, M, true>), grid, dim3(TP * A.P), lds(TP), st, A, TP, LD, magic);
-    return hipGetLastError();
+    const dim3 grid((unsigned)((A.na * A.nb + TP - 1) / TP), 1u, (unsigned)count);
+    return with_epilogue<FAM>(A, [&](auto e) {
+        constexpr bool E = decltype(e)::value;
+        if (A.periodic)
+            go(k_ovl_x<FAM, TS, M, false, E, ApplyArgs>, k_ovl_x<FAM, TS, M, false, E, ApplyBatch>, count, grid,
+               dim3(TP * A.P), lds(TP), st, B, TP, LD, magic);
+        else
+            go(k_ovl_x<FAM, TS, M, true, E, ApplyArgs>, k_ovl_x<FAM, TS, M, true, E, ApplyBatch>, count, grid,
+               dim3(TP * A.P), lds(TP), st, B, TP, LD, magic);
+    });
 }
 
-template <int FAM, typename TS> hipError_t launch_t(int shape, const ApplyArgs &A, hipStream_t st)
+template <int FAM, typename TS> hipError_t launch_t(int shape, ApplyBatch &B, int count, hipStream_t st)
 {
-    if (shape == SHAPE_OVL_STRIDED) return A.m == MAXM ? strided_m<FAM, TS, MAXM>(A, st) : strided_m<FAM, TS, MAXM / 2>(A, st);
+    const ApplyArgs &A = B.a[0];
+    if (shape == SHAPE_OVL_STRIDED) return A.m == MAXM ? strided_m<FAM, TS, MAXM>(B, count, st) : strided_m<FAM, TS, MAXM / 2>(B, count, st);
     if constexpr (Fam<FAM>::SHIFT == 0) {
-        if (shape == SHAPE_OVL_X) return A.m == MAXM ? x_m<FAM, TS, MAXM>(A, st) : x_m<FAM, TS, MAXM / 2>(A, st);
+        if (shape == SHAPE_OVL_X) return A.m == MAXM ? x_m<FAM, TS, MAXM>(B, count, st) : x_m<FAM, TS, MAXM / 2>(B, count, st);
     }
     return hipErrorInvalidValue;
 }
 
-template <typename TS> hipError_t launch_f(int family, int shape, const ApplyArgs &A, hipStream_t st)
+template <typename TS> hipError_t launch_f(int family, int shape, ApplyBatch &B, int count, hipStream_t st)
 {
     switch (family) {
-    case 0: return launch_t<0, TS>(shape, A, st);
-    case 1: return launch_t<1, TS>(shape, A, st);
-    case 2: return launch_t<2, TS>(shape, A, st);
-    case 3: return launch_t<3, TS>(shape, A, st);
-    case 4: return launch_t<4, TS>(shape, A, st);
-    case 5: return launch_t<5, TS>(shape, A, st);
-    case 6: return launch_t<6, TS>(shape, A, st);
-    case 7: return launch_t<7, TS>(shape, A, st);
-    case 8: return launch_t<8, TS>(shape, A, st);
+    case 0: return launch_t<0, TS>(shape, B, count, st);
+    case 1: return launch_t<1, TS>(shape, B, count, st);
+    case 2: return launch_t<2, TS>(shape, B, count, st);
+    case 3: return launch_t<3, TS>(shape, B, count, st);
+    case 4: return launch_t<4, TS>(shape, B, count, st);
+    case 5: return launch_t<5, TS>(shape, B, count, st);
+    case 6: return launch_t<6, TS>(shape, B, count, st);
+    case 7: return launch_t<7, TS>(shape, B, count, st);
+    case 8: return launch_t<8, TS>(shape, B, count, st);
     }
     return hipErrorInvalidValue;
 }
 
 }  // namespace
 
-hipError_t launch_overlap(int family, int shape, bool dbl, const ApplyArgs &A, hipStream_t st)
+hipError_t launch_overlap(int family, int shape, bool dbl, ApplyBatch &B, int count, hipStream_t st)
 {
-    return dbl ? launch_f<double>(family, shape, A, st) : launch_f<float>(family, shape, A, st);
+    return dbl ? launch_f<double>(family, shape, B, count, st) : launch_f<float>(family, shape, B, count, st);
 }
 
 }  // namespace pdo

@@ -37,6 +37,24 @@ struct pdo_pade6stagg_s : public pdo::Pade6Object {};
 
 namespace pdo {
 bool pade6stagg_periodic(pdo_pade6stagg h) { return h && h->periodic; }
+
+int pade6stagg_many(pdo_pade6stagg h, const StaggTask *t, int count, int prec, int n1, int n2, hipStream_t st)
+{
+    ApplyTask a[8];
+    int m = 0, r;
+    for (int i = 0; i < count; i++) {
+        const StaggTask &q = t[i];
+        const bool d2 = q.kind == KIND_STG_D2_C2C || q.kind == KIND_STG_D2_E2E;
+        const bool ok = q.bot >= -1 && q.bot <= 1 && q.top >= -1 && q.top <= 1 && !(d2 && (q.bot == 0 || q.top == 0));
+        if ((!h->periodic && !ok) || m == 8) {
+            // the ends without an operator
+            if ((r = pdo_pade6stagg_apply(h, q.kind, q.bot, q.top, prec, q.in, q.out, n1, n2, 1, (void *)st))) return r;
+            continue;
+        }
+        a[m++] = {h->periodic ? h->per : h->obj[q.bot + 1][q.top + 1], q.kind, 0, 0, q.in, q.out};
+    }
+    return apply_many(a, m, 3, prec, 2L * n1, n2, st);
+}
 }  // namespace pdo
 
 using namespace pdo;

@@ -118,6 +118,8 @@ int pdo_rhs_eval(pdo_rhs h, const void *u, const void *v, const void *w, void *g
     auto op = [&](OpObject *o, int kind, int d, const void *f, void *out, int epi, const void *aux) {
         return op_on(st, o, kind, d, f, out, epi, aux);
     };
+    // small fields: one launch per direction for the three components
+    const bool small = small_field(nn * n, h->prec);
     // the 9 velocity-gradient components run on the side stream (they only
     // read u_i): those of the first PDO_RHS_GRAD_EARLY components beside the
     // filter chain, the others beside the divergence / Poisson / projection
@@ -127,17 +129,34 @@ int pdo_rhs_eval(pdo_rhs h, const void *u, const void *v, const void *w, void *g
         hipError_t ee = hipEventRecord(fork, st);
         if (ee == hipSuccess) ee = hipStreamWaitEvent(h->side, fork, 0);
         if (ee != hipSuccess) return hip_fail(ee, "stream fork");
+        hipStream_t gs = PDO_RHS_SIDE_STREAM ? h->side : st;
+        if (small) {
+            for (int j = 0; j < 3; j++) {
+                ApplyTask t[3];
+                for (int i = i0; i < i1; i++)
+                    t[i - i0] = {&h->d1g, KIND_D1, 0, 0, ui[i], h->field(grad, 3 * i + j)};
+                if (const int rr = apply_many(t, i1 - i0, j + 1, h->prec, j == 2 ? nn : n, j == 2 ? 1 : n, gs)) return rr;
+            }
+            return 0;
+        }
         for (int i = i0; i < i1; i++)
             for (int j = 0; j < 3; j++) {
-                const int rr = op_on(PDO_RHS_SIDE_STREAM ? h->side : st, &h->d1g, KIND_D1, j + 1, ui[i],
+                const int rr = op_on(gs, &h->d1g, KIND_D1, j + 1, ui[i],
                                      h->field(grad, 3 * i + j), 0, nullptr);
                 if (rr) return rr;
             }
         return 0;
     };
     if ((r = gradients(0, PDO_RHS_GRAD_EARLY, h->ev_fork))) return r;
-    // filtered velocity ut_i = F_z F_y F_x u_i (uo_i is the x-pass scratch)
-    for (int i = 0; i < 3; i++) {
+    // filtered velocity ut_i = F_z F_y F_x u_i (uo_i and, for
+    // small fields, ut_i hold the passes between)
+    for (int d = 1; small && d <= 3; d++) {
+        ApplyTask t[3];
+        for (int i = 0; i < 3; i++)
+            t[i] = {&h->fil, KIND_FILTER, 0, 0, d == 1 ? ui[i] : (d == 2 ? h->ut[i] : uoi[i]), d == 2 ? uoi[i] : h->ut[i]};
+        if ((r = apply_many(t, 3, d, h->prec, d == 3 ? nn : n, d == 3 ? 1 : n, st))) return r;
+    }
+    for (int i = 0; !small && i < 3; i++) {
         if ((r = op(&h->fil, KIND_FILTER, 1, ui[i], uoi[i], 0, nullptr))) return r;
         if ((r = op(&h->fil, KIND_FILTER, 2, uoi[i], h->tmp, 0, nullptr))) return r;
         if ((r = op(&h->fil, KIND_FILTER, 3, h->tmp, h->ut[i], 0, nullptr))) return r;

@@ -102,10 +102,12 @@ static void fill_args(const XFilterObject *h, int bc1, int bcn, ExplicitArgs &E)
     }
 }
 
-static int xfilter_apply(pdo_xfilter h, int dir, int prec, const void *f, void *fil, long na, long nb, int bc1,
-                         int bcn, void *stream, int times = 1)
+static int xfilter_apply(pdo_xfilter h, int dir, int prec, const ExplicitFields &F, int count, int times, long na,
+                         long nb, int bc1, int bcn, hipStream_t st)
 {
-    if (!h || !f || !fil || na < 0 || nb < 0) { set_error("invalid argument"); return PDO_ERR_ARG; }
+    bool null = false;
+    for (int i = 0; i < count; i++) null = null || !F.f[i] || !F.out[i];
+    if (!h || null || na < 0 || nb < 0) { set_error("invalid argument"); return PDO_ERR_ARG; }
     const int mode = prec_mode(prec);
     if (mode < 0) { set_error("unknown precision mode"); return PDO_ERR_ARG; }
     if (h->gaussian) {
@@ -118,12 +120,14 @@ static int xfilter_apply(pdo_xfilter h, int dir, int prec, const void *f, void *
         bc1 = bcn = 0;  // the least-squares filter has no boundary options
     }
     const bool dbl = mode == MODE_F64;
-    hipStream_t st = (hipStream_t)stream;
-    const long count = (long)h->n * na * nb;
-    if (count == 0) return 0;
+    const long total = (long)h->n * na * nb;
+    if (total == 0) return 0;
     if (h->n == 1) {
-        hipError_t e = hipMemcpyAsync(fil, f, count * (dbl ? 8 : 4), hipMemcpyDeviceToDevice, st);
-        return e == hipSuccess ? 0 : hip_fail(e, "hipMemcpyAsync");
+        for (int i = 0; i < count; i++) {
+            hipError_t e = hipMemcpyAsync(F.out[i], F.f[i], total * (dbl ? 8 : 4), hipMemcpyDeviceToDevice, st);
+            if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync");
+        }
+        return 0;
     }
     if (na * nb * (long)h->n >= (1L << 31)) { set_error("field too large"); return PDO_ERR_ARG; }
     ExplicitArgs E;
@@ -131,7 +135,7 @@ static int xfilter_apply(pdo_xfilter h, int dir, int prec, const void *f, void *
     E.na = (int)na;
     E.nb = (int)nb;
     E.dir = dir;
-    hipError_t e = launch_explicit(dbl, E, f, fil, st, times);
+    hipError_t e = launch_explicit(dbl, E, F, count, st, times);
     return e == hipSuccess ? 0 : hip_fail(e, "explicit filter launch");
 }
 
@@ -144,10 +148,10 @@ bool xfilter_can_twice(pdo_xfilter h, int dir)
     E.dir = dir;
     return explicit_twice(E);
 }
-int xfilter_twice(pdo_xfilter h, int dir, int prec, const void *f, void *fil, long na, long nb, int bc1, int bcn,
-                  hipStream_t st)
+int xfilter_many(pdo_xfilter h, int dir, int prec, const ExplicitFields &F, int count, int times, long na, long nb,
+                 int bc1, int bcn, hipStream_t st)
 {
-    return xfilter_apply(h, dir, prec, f, fil, na, nb, bc1, bcn, (void *)st, 2);
+    return xfilter_apply(h, dir, prec, F, count, times, na, nb, bc1, bcn, st);
 }
 }  // namespace pdo
 
@@ -160,26 +164,26 @@ int pdo_lstsq_init(pdo_xfilter *h, int n, int periodic) { return make_xfilter(h,
 int pdo_xfilter_filter1(pdo_xfilter h, int prec, const void *f, void *fil, int na, int nb, int bc1, int bcn,
                         void *stream)
 {
-    return xfilter_apply(h, 1, prec, f, fil, na, nb, bc1, bcn, stream);
+    return xfilter_apply(h, 1, prec, {{f}, {fil}}, 1, 1, na, nb, bc1, bcn, (hipStream_t)stream);
 }
 
 int pdo_xfilter_filter2(pdo_xfilter h, int prec, const void *f, void *fil, int na, int nb, int bc1, int bcn,
                         void *stream)
 {
-    return xfilter_apply(h, 2, prec, f, fil, na, nb, bc1, bcn, stream);
+    return xfilter_apply(h, 2, prec, {{f}, {fil}}, 1, 1, na, nb, bc1, bcn, (hipStream_t)stream);
 }
 
 int pdo_xfilter_filter3(pdo_xfilter h, int prec, const void *f, void *fil, int na, int nb, int bc1, int bcn,
                         void *stream)
 {
-    return xfilter_apply(h, 3, prec, f, fil, na, nb, bc1, bcn, stream);
+    return xfilter_apply(h, 3, prec, {{f}, {fil}}, 1, 1, na, nb, bc1, bcn, (hipStream_t)stream);
 }
 
 int pdo_xfilter_filter3_cmplx(pdo_xfilter h, int prec, const void *f, void *fil, int na, int nb, int bc1, int bcn,
                               void *stream)
 {
     // interleaved (re, im): a real z filter of (2 na, nb, n)
-    return xfilter_apply(h, 3, prec, f, fil, 2L * na, nb, bc1, bcn, stream);
+    return xfilter_apply(h, 3, prec, {{f}, {fil}}, 1, 1, 2L * na, nb, bc1, bcn, (hipStream_t)stream);
 }
 
 int pdo_xfilter_dense(pdo_xfilter h, int bc1, int bcn, double *W)

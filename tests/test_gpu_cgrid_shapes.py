@@ -102,3 +102,23 @@ def test_rhs(cuda, shape, periodic):
                 # one-sided closure rows
                 top = 1.5 + np.abs(parts["tau"]).max() + np.abs(parts["q"]).max()
                 assert err <= 2.0 ** -24 * top * np.sqrt(sum((4.0 / d) ** 2 for d in D)), c
+
+
+def test_rhs_beyond_shared_launches(cuda):
+    """FP32 fields above 16 MiB take one pass per launch, the FP64 ones of the
+    same grid (below 64 MiB) several: the two agree to FP32 rounding"""
+    import torch
+    shape = (170, 160, 160)
+    W = _state(shape).astype(np.float32).astype(np.float64)
+    out = {}
+    for prec, dt in (("f64", torch.float64), ("f32_refine", torch.float32)):
+        cg = P.cgrid()
+        assert cg.init(shape, D, prec=prec, inviscid=False, mu_ref=0.02, T_ref=0.9, visc_n=0.7, Pr=0.72) == 0
+        wd = to_dev(W, dt, cuda)
+        rhs = torch.empty_like(wd)
+        assert cg.getRHS(wd, rhs) == 0
+        torch.cuda.synchronize()
+        out[prec] = rhs.double().reshape(5, -1)
+    err = (out["f32_refine"] - out["f64"]).square().mean(dim=1).sqrt()
+    # the bound of test_rhs inside the domain, 2.6 / dx, fluxes of at most 1.5
+    assert err.max().item() <= 2.0 ** -24 * 1.5 * np.sqrt(sum((2.6 / d) ** 2 for d in D))
