@@ -220,15 +220,12 @@ def filter_errors(P, n, f64, f32, stream):
     return out
 
 
-# algorithmic words per point of one cgrid RHS evaluation: 69 compact passes
-# (9 velocity gradients; the artificial shear viscosity's 6 second-derivative
-# and 6 Gaussian passes; the bulk viscosity's 3 + 6 + 6 and the conductivity's
-# 3 + 6 + 6; 3 temperature gradients; 15 flux derivatives) of 2 words each,
-# and the pointwise kernels' reads and writes (primitives 12, transport 4,
-# strain magnitude 10, mustar 5, dilatation 4, bulkstar 15, kapstar 10,
-# coefficient sums 9, tau 17, heat flux 9, fluxes 3 x 15, rhs updates
-# 10 + 2 x 15)
-CGRID_WORDS = 69 * 2 + 12 + 4 + 10 + 5 + 4 + 15 + 10 + 9 + 17 + 9 + 45 + 40
+# words per point of one cgrid RHS evaluation: 48 compact passes (15 gradients,
+# 18 second derivatives, 5 flux derivatives that write and 10 that add to the
+# right-hand side), 9 filter passes of two applications each, and the pointwise
+# kernels' reads and writes (primitives 12, strain magnitude and dilatation 11,
+# mustar 5, bulkstar 15, kapstar 10, stresses and fluxes 48)
+CGRID_WORDS = (15 + 18 + 5 + 9) * 2 + 10 * 3 + 12 + 11 + 5 + 15 + 10 + 48
 
 
 def cgrid_bench(P, dev, stream, steps):
@@ -260,7 +257,7 @@ def cgrid_bench(P, dev, stream, steps):
     del X, Y, Z, rho, u, v, w, p, e, comps
     W = W.float().double()
     N = n ** 3
-    out = {"grid": n, "words_per_point": CGRID_WORDS, "compact_passes": 69}
+    out = {"grid": n, "words_per_point": CGRID_WORDS, "compact_passes": 48}
     res = {}
     for prec, dt in (("f64", torch.float64), ("f32_refine", torch.float32)):
         cg = P.cgrid()

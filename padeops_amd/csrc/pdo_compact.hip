@@ -112,10 +112,8 @@ __device__ __forceinline__ T rhs_row(const TW (&win)[W], int j, const T *c, cons
 // residual) for the wide stencils of periodic systems, in FP32 otherwise.
 // 512^3 periodic passes: cf90 x/y/z 0.246/0.266/0.270 ms with FP64,
 // 0.273/0.288/0.300 with FP32; cd06 x/y 0.207/0.222 with FP64, 0.195/0.217
-// with FP32 (88 instead of 108 VGPRs).  Non-periodic systems (closure rows,
-// more live registers) gain most from FP32: the 512 x 512 x 256 wall-normal
-// cd06stagg passes went from 0.43 / 0.37 ms to 0.23 / 0.13 ms.  Tuning
-// choice.
+// with FP32 (88 instead of 108 VGPRs).  The non-periodic ones (513 rows)
+// carry closure rows in the registers this saves.  Tuning choice.
 template <int FAM, bool PER> constexpr bool rhs1_fp64() { return PER && Fam<FAM>::R > 2; }
 
 // the same for segments of MAXM rows, or MAXM + 1 when `ext` (MM = MAXM + 1)
