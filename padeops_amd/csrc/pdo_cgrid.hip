@@ -132,8 +132,8 @@ __global__ void __launch_bounds__(256) k_kapstar(const TS *X, const TS *Y, const
 //   momentum rho u_d u_i + p delta_id - tau_id;
 //   energy (TE + p - tau_dd) u_d - sum_{i != d} u_i tau_id + q_d
 // (that of mass is the momentum itself).  Bound by HBM: 24 words read and 24
-// written per point, where the steps one by one moved 88 (256^3 FP64: 1.3 ms
-// at 5.3 TB/s with three fluxes more).
+// written per point, where the steps one by one moved 88 (256^3 FP64: 1.24
+// ms, 5.2 TB/s).
 // flux may overlie anything but the inputs.
 template <typename TS>
 __global__ void __launch_bounds__(256) k_fluxes(const TS *W, const TS *prim, const TS *g, const TS *star, const TS *de,
