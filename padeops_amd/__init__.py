@@ -1044,7 +1044,8 @@ class igrid:
         return _check(lib().pdo_igrid_step(self._h, nsteps, _stream(stream)))
 
     def field(self, name):
-        """a torch view of one of the object's fields (FIELDS)"""
+        """a torch view of one of the object's fields (FIELDS): the memory is the
+        object's, which the view keeps alive, until destroy()"""
         import torch
         ptr = ctypes.c_void_p()
         _check(lib().pdo_igrid_field(self._h, self.FIELDS[name], ctypes.byref(ptr)))
@@ -1061,8 +1062,7 @@ class igrid:
         dt = cplx if spectral_ else real
         n = sizes[name]
         W = torch.empty((), dtype=dt).element_size()
-        # wrap the device memory without copying (the object owns it)
-        holder = _DeviceView(ptr.value, n * W)
+        holder = _DeviceView(ptr.value, n * W, self)
         t = torch.as_tensor(holder, device="cuda").view(dt)
         return t[:n]
 
@@ -1153,9 +1153,11 @@ class Closure:
 
 class _DeviceView:
     """__cuda_array_interface__ of a byte range of device memory owned by a
-    library object (torch.as_tensor wraps it without a copy)."""
+    library object.  torch.as_tensor wraps it without a copy, and its storage
+    holds the view, so the owner lives as long as any tensor over its memory."""
 
-    def __init__(self, ptr, nbytes):
+    def __init__(self, ptr, nbytes, owner):
+        self.owner = owner
         self.__cuda_array_interface__ = {"shape": (nbytes,), "typestr": "|u1", "data": (ptr, False), "version": 3}
 
 
