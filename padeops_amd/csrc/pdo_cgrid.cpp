@@ -7,6 +7,7 @@
 // solves of the collocated drop-in carry the work; the rest are pointwise
 // kernels (pdo_cgrid.hip).  All fields live in device memory for the life of
 // the object.
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -26,16 +27,15 @@ enum {
     F_STAR = F_Q + 3,      // mustar, bulkstar, kapstar
     F_DE = F_STAR + 3,     // gradient of e
     // of the artificial coefficients alone: the fluxes overlie them
-    F_T1 = F_DE + 3,       // a second derivative per coefficient
-    F_D4 = F_T1 + 3,       // fourth derivatives along x, y, z of each
-    F_FIL = F_D4 + 9,      // two filter buffers for each
-    F_DRHO = F_FIL + 6,    // gradient of rho
+    F_DRHO = F_DE + 3,     // gradient of rho
     F_FUNC = F_DRHO + 3,   // strain-rate magnitude
     F_DIL = F_FUNC + 1,    // dilatation
-    F_COUNT = F_DIL + 1,
-    F_FLUX = F_T1          // momentum and energy fluxes per direction
+    F_PASS = F_DIL + 1,    // fields of the coefficients formed together
+    F_FLUX = F_DRHO        // momentum and energy fluxes, four per direction
 };
-static_assert(F_COUNT - F_FLUX >= 12, "the fluxes overlie 12 work fields");
+// of each coefficient formed at a time: a second derivative, the fourth
+// derivatives along x, y, z, and two filter buffers
+enum { P_T1 = 0, P_D4 = P_T1 + 1, P_FIL = P_D4 + 3, P_COUNT = P_FIL + 2 };
 
 struct CgridObject {
     pdo_cgrid_params p{};
@@ -44,6 +44,7 @@ struct CgridObject {
     long n = 0;
     pdo_derivatives der = nullptr;
     pdo_filters fil = nullptr, gfil = nullptr;
+    int together = 1;  // artificial coefficients formed at a time: 1 or 3
     void *buf = nullptr;
     ~CgridObject()
     {
@@ -53,6 +54,10 @@ struct CgridObject {
         if (buf) (void)hipFree(buf);
     }
     void *f(int i) { return (char *)buf + (size_t)i * n * W; }
+    // of the q-th coefficient of those formed together
+    void *pass(int q, int i) { return f(F_PASS + q * P_COUNT + i); }
+    // 46 fields, 57 with the three coefficients together
+    int fields() const { return std::max(F_PASS + together * P_COUNT, F_FLUX + 12); }
 };
 
 }  // namespace pdo
@@ -77,16 +82,16 @@ int cg(pdo_cgrid h, CgOp op, const CgArgs &a, hipStream_t st)
 const int *bc_of(pdo_cgrid h, int d) { return d == 0 ? h->p.x_bc : (d == 1 ? h->p.y_bc : h->p.z_bc); }
 
 // the fourth derivatives along each direction (two second-derivative passes)
-// of the functions of the coefficients [k0, k1) into F_D4 + 3 k + d
-int fourth(pdo_cgrid h, const void *const f[3], int k0, int k1, hipStream_t st)
+// of count functions f
+int fourth(pdo_cgrid h, const void *const *f, int count, hipStream_t st)
 {
     for (int d = 0; d < 3; d++) {
         const int *b = bc_of(h, d);
         DerivTask t[3];
-        for (int k = k0; k < k1; k++) t[k - k0] = {f[k], h->f(F_T1 + k), b[0], b[1]};
-        PDO_TRY(derivatives_many(h->der, d, 2, h->prec, t, k1 - k0, nullptr, st));
-        for (int k = k0; k < k1; k++) t[k - k0] = {h->f(F_T1 + k), h->f(F_D4 + 3 * k + d), b[0], b[1]};
-        PDO_TRY(derivatives_many(h->der, d, 2, h->prec, t, k1 - k0, nullptr, st));
+        for (int q = 0; q < count; q++) t[q] = {f[q], h->pass(q, P_T1), b[0], b[1]};
+        PDO_TRY(derivatives_many(h->der, d, 2, h->prec, t, count, nullptr, st));
+        for (int q = 0; q < count; q++) t[q] = {h->pass(q, P_T1), h->pass(q, P_D4 + d), b[0], b[1]};
+        PDO_TRY(derivatives_many(h->der, d, 2, h->prec, t, count, nullptr, st));
     }
     return 0;
 }
@@ -110,7 +115,7 @@ int filter3(pdo_cgrid h, pdo_filters fl, void *const *arr, int count, int numtim
             // out of place: the last pass writes arr unless it also reads it
             const bool home = pass == total - 1 && cur[0] != arr[0];
             void *dst[3];
-            for (int k = 0; k < count; k++) dst[k] = home ? arr[k] : h->f(F_FIL + 2 * k + buf);
+            for (int k = 0; k < count; k++) dst[k] = home ? arr[k] : h->pass(k, P_FIL + buf);
             PDO_TRY(filters_many(fl, d, h->prec, cur, dst, count, times, b[0], b[1], st));
             for (int k = 0; k < count; k++) cur[k] = dst[k];
             buf ^= 1;
@@ -144,9 +149,10 @@ int lad(pdo_cgrid h, hipStream_t st)
     a.n = n;
     PDO_TRY(cg(h, CG_STRAIN, a, st));
     const void *const func[3] = {h->f(F_FUNC), h->f(F_DIL), h->f(F_PRIM + 4)};
-    auto star = [&](int k) -> int {
+    // coefficient k, the q-th of those formed together
+    auto star = [&](int k, int q) -> int {
         CgArgs c;
-        for (int d = 0; d < 3; d++) c.in[d] = h->f(F_D4 + 3 * k + d);
+        for (int d = 0; d < 3; d++) c.in[d] = h->pass(q, P_D4 + d);
         c.out[0] = h->f(F_STAR + k);
         c.n = n;
         if (k == 0) {
@@ -173,13 +179,13 @@ int lad(pdo_cgrid h, hipStream_t st)
     // small fields: the three coefficients' passes share launches; others:
     // one coefficient after the other, so that a pass finds what the last one
     // wrote in the Infinity Cache
-    const int step = small_field(n, h->prec) ? 3 : 1;
+    const int step = h->together;
     for (int k = 0; k < 3; k += step) {
-        PDO_TRY(fourth(h, func, k, k + step, st));
+        PDO_TRY(fourth(h, func + k, step, st));
         void *s[3];
-        for (int q = k; q < k + step; q++) {
-            PDO_TRY(star(q));
-            s[q - k] = h->f(F_STAR + q);
+        for (int q = 0; q < step; q++) {
+            PDO_TRY(star(k + q, q));
+            s[q] = h->f(F_STAR + k + q);
         }
         PDO_TRY(filter3(h, h->gfil, s, step, 2, st));
     }
@@ -213,7 +219,8 @@ int pdo_cgrid_init(pdo_cgrid *out, const pdo_cgrid_params *p, int prec)
     const int gauss[3] = {2, 2, 2};
     if (!st) st = pdo_filters_init(&h->gfil, p->nx, p->ny, p->nz, p->periodic, gauss);
     if (st) { delete h; return st; }
-    hipError_t e = hipMalloc(&h->buf, (size_t)F_COUNT * h->n * h->W);
+    h->together = small_field(h->n, prec) ? 3 : 1;
+    hipError_t e = hipMalloc(&h->buf, (size_t)h->fields() * h->n * h->W);
     if (e != hipSuccess) { delete h; return hip_fail(e, "hipMalloc(cgrid work)"); }
     *out = h;
     return 0;

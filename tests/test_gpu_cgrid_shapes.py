@@ -122,3 +122,20 @@ def test_rhs_beyond_shared_launches(cuda):
     err = (out["f32_refine"] - out["f64"]).square().mean(dim=1).sqrt()
     # the bound of test_rhs inside the domain, 2.6 / dx, fluxes of at most 1.5
     assert err.max().item() <= 2.0 ** -24 * 1.5 * np.sqrt(sum((2.6 / d) ** 2 for d in D))
+
+
+@pytest.mark.parametrize("prec,n", [("f64", 208), ("f32_refine", 164)])
+def test_work_memory_of_large_fields(cuda, prec, n):
+    """fields beyond the shared launches (64 MiB, 16 MiB) form one artificial
+    coefficient at a time and hold work for one: 46 fields"""
+    import gc
+
+    import torch
+    gc.collect()  # no earlier object's memory comes back in between
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    cg = P.cgrid()
+    assert cg.init((n, n, n), D, prec=prec) == 0
+    used = free - torch.cuda.mem_get_info()[0]
+    field = n ** 3 * (8 if prec == "f64" else 4)
+    assert used <= 47 * field, used / field
