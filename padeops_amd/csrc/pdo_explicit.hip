@@ -16,6 +16,8 @@
 // lines staged in LDS.  One thread per point with nine loads each, before,
 // spent its time on 64-bit index divisions: 256^3 FP64, two applications
 // 2 x 116 us, now in one pass 52 us along y and z, 81 us along x.
+#include <algorithm>
+
 #include "pdo_explicit.hpp"
 
 namespace pdo {
@@ -102,10 +104,12 @@ __global__ void __launch_bounds__(256) k_expl_strided(ExplicitArgs E, ExplicitFi
 }
 
 // x: `lines` whole lines per workgroup in LDS; element e is point
-// e % n of line e / n (magic: the rounded-up reciprocal of n)
-template <typename TS, int NP>
-__global__ void __launch_bounds__(256) k_expl_x(ExplicitArgs E, ExplicitFields F, int lines, unsigned magic)
+// e % n of line e / n (magic: the rounded-up reciprocal of n).  NT: 256
+// threads, or up to 1024
+template <typename TS, int NP, int NT>
+__global__ void __launch_bounds__(NT) k_expl_x(ExplicitArgs E, ExplicitFields F, int lines, unsigned magic)
 {
+    const int nt = NT == 256 ? 256 : blockDim.x;
     const TS *f = (const TS *)F.f[blockIdx.z];
     TS *out = (TS *)F.out[blockIdx.z];
     extern __shared__ double lds[];
@@ -116,11 +120,11 @@ __global__ void __launch_bounds__(256) k_expl_x(ExplicitArgs E, ExplicitFields F
     f += l0 * n;
     out += l0 * n;
 #pragma unroll 4
-    for (int e = threadIdx.x; e < total; e += 256) tile[e] = f[e];
+    for (int e = threadIdx.x; e < total; e += nt) tile[e] = f[e];
     __syncthreads();
     auto apply = [&](const auto *src, auto put) {
 #pragma unroll 2
-        for (int e = threadIdx.x; e < total; e += 256) {
+        for (int e = threadIdx.x; e < total; e += nt) {
             const int r = e - (int)__umulhi((unsigned)e, magic) * n;
             const auto *p = src + (e - r);
             double acc;
@@ -153,9 +157,9 @@ __global__ void __launch_bounds__(256) k_expl_x(ExplicitArgs E, ExplicitFields F
     }
 }
 
-// the lengths the two others don't take (y, z: 8 .. 15 rows, 17 .. 23 without
-// periodicity; x: above 4096), one application: one thread per output point
-// along the contiguous index
+// one application, what the two others don't take (y, z: 8 .. 15 rows, 17 ..
+// 23 without periodicity; x: above 4096) or take longer for (launch_fast): one
+// thread per output point along the contiguous index
 template <typename TS, typename TA>
 __global__ void __launch_bounds__(256) k_explicit(ExplicitArgs E, const TS *__restrict__ f, TS *__restrict__ out)
 {
@@ -206,23 +210,48 @@ static bool chunked(const ExplicitArgs &E)
     return E.n >= EXPL_T && E.n <= 1 << 17 && (E.periodic || C == 1 || (E.n - EXPL_T) / (C - 1) >= 2 * EXPL_R);
 }
 
+// Fields of few points leave most of the chip idle, and a pass takes as long
+// as the chain of one thread, which is shortest with a point per thread
+// (k_explicit): one application along z and y of 32^3 FP64 points takes 2.4
+// us there and 3.2 in chunks of 16 rows, of 64^3 3.2 and 3.3, of 80^3 5.7 and
+// 3.7; FP32 2.2 and 3.1, 3.1 and 3.2, 3.9 and 3.4.
+constexpr long FEW_POINTS = 1 << 18;
+// Lines along x: as many per workgroup as make 1024 workgroups, within 256 to
+// 2048 points (1 to 8 per thread): 32^3 FP64 2.0 us with 256 points, 4.2 with
+// 2048; 64^3 2.6 and 4.5; 128^3 9.1 both.  Long lines without 512 workgroups
+// take a thread per point (4096 x 16 FP64 lines 2.3 us against 6.5 in lines,
+// 3000 x 256 5.9 and 6.7, 2000 x 512 7.4 and 6.6), and for two applications up
+// to 1024 threads (3000 x 256 FP64, the filter twice along each direction,
+// 23.3 us, with 256 threads 27.5).
+constexpr long LINE_GROUPS = 1024, FEW_LINES = 512;
+
 template <typename TS, int NP>
 static bool launch_fast(const ExplicitArgs &E, const ExplicitFields &F, int count, hipStream_t st)
 {
-    const long pencils = (long)E.na * E.nb;
+    const long pencils = (long)E.na * E.nb * count;  // of all fields
+    const unsigned nz = (unsigned)count;
     if (E.dir != 1) {
-        if (!chunked(E)) return false;
-        const dim3 grid((unsigned)((pencils + 255) / 256), (unsigned)((E.n + EXPL_T - 1) / EXPL_T), (unsigned)count);
+        if (!chunked(E) || (NP == 1 && pencils * E.n <= FEW_POINTS)) return false;
+        const dim3 grid((unsigned)(((long)E.na * E.nb + 255) / 256), (unsigned)((E.n + EXPL_T - 1) / EXPL_T), nz);
         hipLaunchKernelGGL((k_expl_strided<TS, NP>), grid, dim3(256), 0, st, E, F);
         return true;
     }
-    // about 2048 points a workgroup (8 per thread), at most 64 KiB of LDS
-    if (E.n > 4096) return false;
-    const int lines = E.n < 2048 ? 2048 / E.n : 1;
+    const bool few = E.n > 256 && pencils < FEW_LINES;
+    if (E.n > 4096 || (NP == 1 && few)) return false;
+    // at most 64 KiB of LDS
+    const long lo = E.n < 256 ? 256 / E.n : 1, hi = E.n < 2048 ? 2048 / E.n : 1;
+    const int lines = (int)std::min(std::max(pencils / LINE_GROUPS, lo), hi);
     const size_t lds = (size_t)lines * E.n * (sizeof(TS) + (NP == 2 ? 8 : 0));
     const unsigned magic = (unsigned)(((unsigned long long)1 << 32) / E.n + 1);
-    hipLaunchKernelGGL((k_expl_x<TS, NP>), dim3((unsigned)((pencils + lines - 1) / lines), 1, (unsigned)count),
-                       dim3(256), lds, st, E, F, lines, magic);
+    const dim3 grid((unsigned)(((long)E.na * E.nb + lines - 1) / lines), 1, nz);
+    if constexpr (NP == 2) {
+        if (few) {
+            const dim3 block(std::min((E.n + 63) / 64 * 64, 1024));
+            hipLaunchKernelGGL((k_expl_x<TS, NP, 1024>), grid, block, lds, st, E, F, lines, magic);
+            return true;
+        }
+    }
+    hipLaunchKernelGGL((k_expl_x<TS, NP, 256>), grid, dim3(256), lds, st, E, F, lines, magic);
     return true;
 }
 

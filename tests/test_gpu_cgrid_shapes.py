@@ -21,27 +21,80 @@ D = (0.1, 0.13, 0.17)
 @pytest.mark.parametrize("periodic,bc", [(True, (0, 0)), (False, (0, 0)), (False, (1, -1)), (False, (-1, 1))])
 @pytest.mark.parametrize("n", [8, 9, 15, 16, 17, 23, 24, 25, 32, 33, 49, 100])
 @pytest.mark.parametrize("axis", [0, 1, 2])
-def test_filter_once_and_twice(cuda, axis, n, periodic, bc):
+@pytest.mark.parametrize("prec", ["f64", "f32_refine"])
+def test_filter_once_and_twice(cuda, axis, n, periodic, bc, prec):
     import torch
+    dt = torch.float64 if prec == "f64" else torch.float32
     shape = [11, 9, 10]
     shape[axis] = n
     shape = tuple(shape)
     per, bcs = [True] * 3, [(0, 0)] * 3
     per[axis], bcs[axis] = periodic, bc
-    f = random_field(shape, seed=n + axis)
+    f = from_dev(to_dev(random_field(shape, seed=n + axis), dt, cuda), shape)
     for kind in ("gaussian", "lstsq"):
         cg = P.cgrid()
-        assert cg.init(shape, D, prec="f64", periodic=tuple(per), bc=tuple(bcs), filter=(kind,) * 3) == 0
+        assert cg.init(shape, D, prec=prec, periodic=tuple(per), bc=tuple(bcs), filter=(kind,) * 3) == 0
         for times in (1, 2, 3, 4):
             ref = f
             for ax in (1, 0, 2):
                 for _ in range(times):
                     ref = X.filter_axis(ref, ax, kind, per[ax], *bcs[ax])
-            fd = to_dev(f, torch.float64, cuda)
+            fd = to_dev(f, dt, cuda)
             assert cg.filter(fd, numtimes=times, gaussian=kind == "gaussian") == 0
             torch.cuda.synchronize()
-            # 9-point sums with weights of at most 1 in magnitude, FP64
-            assert rel_l2(from_dev(fd, shape), ref) <= 1e-14 * 3 * times, (kind, times)
+            # 9-point sums with weights of at most 1 in magnitude, FP64; FP32
+            # storage rounds each of at most 3 times fields by 2^-24, which
+            # the filters that follow damp like the field
+            tol = 1e-14 if prec == "f64" else 2.0 ** -24
+            assert rel_l2(from_dev(fd, shape), ref) <= tol * 3 * times, (kind, times)
+
+
+@pytest.mark.parametrize("axis,n,other", [(a, n, (128, 129)) for a in (1, 2) for n in (16, 17, 24, 25, 33, 100)]
+                         + [(0, n, (23, 23)) for n in (255, 256, 257, 300)] + [(0, 512, (16, 32)), (0, 4096, (16, 32)),
+                                                                             (0, 16, (64, 129))])
+@pytest.mark.parametrize("prec", ["f64", "f32_refine"])
+def test_filter_large_fields(cuda, axis, n, other, prec):
+    """one application in chunks along y and z and in lines along x: more than
+    2^18 points, and 512 lines or more of above 256 points (smaller fields
+    take a thread per point)"""
+    import torch
+    dt = torch.float64 if prec == "f64" else torch.float32
+    shape = list(other)
+    shape.insert(axis, n)
+    f = random_field(shape, seed=n + axis)
+    ft = to_dev(f, dt, cuda)
+    f = from_dev(ft, tuple(shape))
+    for periodic, bc in ((True, (0, 0)), (False, (0, 0)), (False, (1, -1))):
+        o = P.gaussian()
+        o.init(n, periodic)
+        out = torch.full_like(ft, float("nan"))
+        (o.filter1, o.filter2, o.filter3)[axis](ft, out, *other, *bc, prec=prec)
+        torch.cuda.synchronize()
+        ref = X.filter_axis(f, axis, "gaussian", periodic, *bc)
+        # a 9-point sum in FP64; FP32 storage rounds the output alone
+        assert rel_l2(from_dev(out, tuple(shape)), ref) <= (1e-14 if prec == "f64" else 2.0 ** -24), (periodic, bc)
+
+
+@pytest.mark.parametrize("n", [257, 300, 1023, 1025, 4096, 4097])
+@pytest.mark.parametrize("periodic,bc", [(True, (0, 0)), (False, (1, -1))])
+@pytest.mark.parametrize("prec", ["f64", "f32_refine"])
+def test_filter_long_lines_twice(cuda, n, periodic, bc, prec):
+    """few long lines: two applications with up to 1024 threads and 64 KiB of
+    LDS up to 4096 points, one after the other beyond"""
+    import torch
+    dt = torch.float64 if prec == "f64" else torch.float32
+    shape = (n, 10, 1)
+    ft = to_dev(random_field(shape, seed=n), dt, cuda)
+    ref = from_dev(ft, shape)
+    cg = P.cgrid()
+    assert cg.init(shape, D, prec=prec, periodic=(periodic, True, True), bc=(bc, (0, 0), (0, 0))) == 0
+    for ax in (1, 0):  # one point along z: no filter
+        for _ in range(2):
+            ref = X.filter_axis(ref, ax, "gaussian", periodic if ax == 0 else True, *(bc if ax == 0 else (0, 0)))
+    assert cg.filter(ft, numtimes=2, gaussian=True) == 0
+    torch.cuda.synchronize()
+    # as above, four applications
+    assert rel_l2(from_dev(ft, shape), ref) <= 4 * (1e-14 if prec == "f64" else 2.0 ** -24)
 
 
 @pytest.mark.parametrize("n", [4095, 4096, 4097, 6000])
