@@ -288,7 +288,10 @@ __global__ void __launch_bounds__(256) k_sum_partials(const double *__restrict__
 }
 
 // ---------------------------------------------------------------------------
-// features X (n, 10) and, optionally, the normalised gradient a (n, 9)
+// features X (n, 10) and, optionally, the normalised gradient a (n, 9).  Bound
+// by HBM (FP32: 76 bytes per point after the scale's 36), so one point per
+// thread: in a loop over points the compiler held 104 registers for 82, four
+// waves per SIMD for five (2^24 FP32 points with their scale 548 us, now 420).
 // ---------------------------------------------------------------------------
 template <typename TS>
 __global__ void __launch_bounds__(256) k_closure_features(const TS *__restrict__ g, long n, long stride,
@@ -296,18 +299,18 @@ __global__ void __launch_bounds__(256) k_closure_features(const TS *__restrict__
                                                          float *__restrict__ X, float *__restrict__ A9)
 {
     const double inv = inv_scale(sumsq, nnorm);
-    for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
-        double A[9];
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    double A[9];
 #pragma unroll
-        for (int c = 0; c < 9; ++c) A[c] = inv * (double)g[t + c * stride];
-        float x[10];
-        features_of(split_of(A), dratio, x);
+    for (int c = 0; c < 9; ++c) A[c] = inv * (double)g[t + c * stride];
+    float x[10];
+    features_of(split_of(A), dratio, x);
 #pragma unroll
-        for (int k = 0; k < 10; ++k) X[t * 10 + k] = x[k];
-        if (A9) {
+    for (int k = 0; k < 10; ++k) X[t * 10 + k] = x[k];
+    if (A9) {
 #pragma unroll
-            for (int c = 0; c < 9; ++c) A9[t * 9 + c] = (float)A[c];
-        }
+        for (int c = 0; c < 9; ++c) A9[t * 9 + c] = (float)A[c];
     }
 }
 
@@ -487,7 +490,7 @@ hipError_t launch_grad_sumsq(bool dbl, const void *g, long n, long stride, doubl
 hipError_t launch_closure_features(bool dbl, const void *g, long n, long stride, const double *sumsq, long nnorm,
                                    double dratio, float *X, float *A9, hipStream_t st)
 {
-    const unsigned nb = grid_of(n);
+    const unsigned nb = (unsigned)((n + 255) / 256);
     if (dbl)
         hipLaunchKernelGGL(k_closure_features<double>, dim3(nb), dim3(256), 0, st, (const double *)g, n, stride,
                            sumsq, nnorm, dratio, X, A9);

@@ -62,6 +62,33 @@ def test_features(cuda, dt):
     assert np.abs(A9.cpu().numpy() - A / g).max() <= 1e-6 * np.abs(A / g).max()
 
 
+@pytest.mark.parametrize("dt", ["f64", "f32"])
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 2097157])
+def test_features_at_the_edges_of_workgroups(cuda, n, dt):
+    """a workgroup takes 256 points: the last one's, and nothing beyond"""
+    import torch
+    dtype = torch.float64 if dt == "f64" else torch.float32
+    A = _field(n, 4).astype(np.float32).astype(np.float64)
+    cl = P.Closure(None, n)
+    X = torch.full((10 * n + 40,), 77.0, device=cuda)
+    A9 = torch.full((9 * n + 40,), 77.0, device=cuda)
+    assert cl.features(_planes(A, cuda, dtype), n, 0.5, X, A9) == 0
+    torch.cuda.synchronize()
+    X, A9 = X.cpu().numpy(), A9.cpu().numpy()
+    assert (X[10 * n:] == 77.0).all() and (A9[9 * n:] == 77.0).all()
+    g = C.scale(A)
+    rows = np.unique(np.r_[np.arange(min(n, 300)), np.arange(max(n - 300, 0), n)])
+    a = A[rows] / g
+    assert np.abs(A9[:9 * n].reshape(n, 9)[rows] - a).max() <= 1e-6 * np.abs(a).max()
+    # the first two features are sqrt(tr s^2) and sqrt(-tr r^2), rounded to FP32
+    M3 = a.reshape(-1, 3, 3)
+    S, R = 0.5 * (M3 + M3.transpose(0, 2, 1)), 0.5 * (M3 - M3.transpose(0, 2, 1))
+    S -= (np.trace(S, axis1=1, axis2=2) / 3)[:, None, None] * np.eye(3)
+    ref = np.stack([np.sqrt((S * S).sum(axis=(1, 2))), np.sqrt((R * R).sum(axis=(1, 2)))], axis=1)
+    assert np.abs(X[:10 * n].reshape(n, 10)[rows, :2] - ref).max() <= 2.0 ** -22 * ref.max()
+    assert (X[:10 * n].reshape(n, 10)[:, 9] == 0.5).all()
+
+
 def test_stress_layouts_and_fallback(cuda):
     import torch
     n = 4096
