@@ -874,9 +874,16 @@ static bool local_tables(const SystemDesc &s, int r0, int m, bool has_prev, bool
 // rows: the coupling rows are then the same for every segment.
 // `exact`: rows beyond the period may not stand in for the first ones (an
 // edge field's last point is read as it is stored), so n is a multiple of m.
+// Non-periodic pencils of 32 and 64 rows take two and four 16-row segments: as
+// one and two 32-row segments their passes last as long as one lane's sweep
+// over 32 rows (staggered z derivative of FP32 lines, 32 rows: 4224 lines 8.5
+// us, with 16-row segments 5.4, refined in registers 7.5; 66048 lines 10.7,
+// 8.1, 9.8; 64 rows: 8.3, 5.7, 7.7 and 13.5, 11.4, 12.9).  From 96 rows on the
+// larger fields take longer in 16-row segments (66048 lines 15.8 and 17.5).
 static bool choose_overlap(int n, int K, int nb, bool periodic, bool exact, int &m, int &P)
 {
-    for (m = MAXM; m >= MAXM / 2; m /= 2) {
+    const bool halves = !periodic && n % MAXM == 0 && n <= 2 * MAXM;
+    for (m = halves ? MAXM / 2 : MAXM; m >= MAXM / 2; m /= 2) {
         if (n < m || (exact && n % m != 0)) continue;
         P = (n + m - 1) / m;
         if (P > OVL_PMAX) return false;

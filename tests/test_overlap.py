@@ -118,7 +118,7 @@ def _fields(n, dir, seed):
 
 # lengths at the edges of the segment counts: one 16- or 32-row segment, one
 # row more, the last and first of a count, primes, above 512
-LENGTHS = [16, 17, 23, 33, 36, 47, 63, 65, 97, 101, 151, 200, 257, 300, 509, 513, 640, 1021]
+LENGTHS = [16, 17, 23, 32, 33, 36, 47, 63, 64, 65, 97, 101, 151, 200, 257, 300, 509, 513, 640, 1021]
 
 
 @pytest.mark.gpu
@@ -158,7 +158,7 @@ def test_against_oracle(cuda, n, dir, prec):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,prec", [(n, "f64") for n in (16, 24, 40, 48, 65, 100)]
-                         + [(n, "f32_refine") for n in (32, 100, 511, 512, 513)])
+                         + [(n, "f32_refine") for n in (32, 64, 96, 100, 511, 512, 513)])
 def test_staggered_against_oracle(cuda, n, prec):
     import torch
 
