@@ -130,30 +130,36 @@ __global__ void __launch_bounds__(256) k_mlp_forward(const float *__restrict__ X
 }
 
 // ---------------------------------------------------------------------------
-// inference forward (no cache): pdo_mlp_dev.hpp on samples in memory, two
+// inference forward (no cache): pdo_mlp_dev.hpp on samples in memory, NT
 // tiles per wave at a time.  At most 128 registers, so that the matrix
 // results stay in vector registers.
 // ---------------------------------------------------------------------------
 constexpr int INFER_WAVES = 4;  // waves per workgroup
+// samples up to which a wave takes one tile, not two: as many tiles as the
+// chip has SIMDs.  A launch lasts as long as one wave then: 1000 samples 5.1
+// us with one tile and 6.6 with two, 16384 5.3 and 6.7; beyond, two tiles
+// share the weights' LDS reads: 65536 10.7 and 9.4.
+constexpr long ONE_TILE = 16 * 1024;
 
+template <int NT>
 __global__ void __launch_bounds__(64 * INFER_WAVES, 4)
 k_mlp_infer(const float *__restrict__ X, float *__restrict__ Y, const unsigned short *__restrict__ Wb,
-            const float *__restrict__ P, long B, long npairs)
+            const float *__restrict__ P, long B, long ngroups)
 {
     __shared__ MlpLds L;
     mlp_stage(L, Wb, P);
     __syncthreads();
     const int lane = threadIdx.x & 63, g = lane >> 4;
     const long stride = (long)gridDim.x * INFER_WAVES;
-    for (long t = (long)blockIdx.x * INFER_WAVES + (threadIdx.x >> 6); t < npairs; t += stride) {
+    for (long t = (long)blockIdx.x * INFER_WAVES + (threadIdx.x >> 6); t < ngroups; t += stride) {
         // keeps the LDS weight reads inside the loop (hoisted, they would
         // occupy the registers the LDS placement is meant to free)
         asm volatile("" ::: "memory");
-        u32x2 x[2];
-        f32x4 y[2];
+        u32x2 x[NT];
+        f32x4 y[NT];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const long s = 32 * t + 16 * q + (lane & 15);  // this lane's sample
+        for (int q = 0; q < NT; ++q) {
+            const long s = 16 * (NT * t + q) + (lane & 15);  // this lane's sample
             f32x4 xv = {0, 0, 0, 0};
             if (s < B) {
 #pragma unroll
@@ -162,10 +168,10 @@ k_mlp_infer(const float *__restrict__ X, float *__restrict__ Y, const unsigned s
             }
             x[q] = (u32x2){pack2(xv[0], xv[1]), pack2(xv[2], xv[3])};
         }
-        mlp_eval<2>(L, x, y);
+        mlp_eval<NT>(L, x, y);
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const long s = 32 * t + 16 * q + (lane & 15);
+        for (int q = 0; q < NT; ++q) {
+            const long s = 16 * (NT * t + q) + (lane & 15);
             // outputs 4 g .. 4 g + 3 of sample s; 6 are used
             if (s < B && g < 2) {
 #pragma unroll
@@ -307,6 +313,17 @@ hipError_t resident_blocks(Resident &r, const void *kernel, int threads, int *bl
 
 static unsigned nblocks(long B) { return (unsigned)((B + TILE - 1) / TILE); }
 
+template <int NT>
+static hipError_t launch_infer(const float *X, float *Y, const unsigned short *Wb, const float *P, long B, long blocks,
+                               hipStream_t st)
+{
+    const long ngroups = (B + 16 * NT - 1) / (16 * NT);
+    const long need = (ngroups + INFER_WAVES - 1) / INFER_WAVES;
+    hipLaunchKernelGGL(k_mlp_infer<NT>, dim3((unsigned)(need < blocks ? need : blocks)), dim3(64 * INFER_WAVES), 0, st,
+                       X, Y, Wb, P, B, ngroups);
+    return hipGetLastError();
+}
+
 hipError_t launch_mlp_forward(const float *X, float *Y, const unsigned short *Wb, const float *P, long B,
                               const MlpCache &cache, hipStream_t st)
 {
@@ -315,13 +332,9 @@ hipError_t launch_mlp_forward(const float *X, float *Y, const unsigned short *Wb
         // inference: as many persistent workgroups as are resident at once
         static Resident resident;
         int res = 0;
-        const hipError_t e = resident_blocks(resident, (const void *)k_mlp_infer, 64 * INFER_WAVES, &res);
+        const hipError_t e = resident_blocks(resident, (const void *)k_mlp_infer<2>, 64 * INFER_WAVES, &res);
         if (e != hipSuccess) return e;
-        const long npairs = (B + 31) / 32;  // 32 samples per wave
-        const long need = (npairs + INFER_WAVES - 1) / INFER_WAVES;
-        const long nwg = need < res ? need : res;
-        hipLaunchKernelGGL(k_mlp_infer, dim3((unsigned)nwg), dim3(64 * INFER_WAVES), 0, st, X, Y, Wb, P, B, npairs);
-        return hipGetLastError();
+        return B <= ONE_TILE ? launch_infer<1>(X, Y, Wb, P, B, res, st) : launch_infer<2>(X, Y, Wb, P, B, res, st);
     }
     hipLaunchKernelGGL(k_mlp_forward, dim3(nblocks(B)), dim3(256), 0, st, X, Y, Wb, P, B, cache);
     return hipGetLastError();

@@ -54,11 +54,11 @@ def test_forward_and_gradients(cuda, B):
     assert np.all(after[pad] == 0) and np.all(lib_before[pad] == 0)
 
 
-@pytest.mark.parametrize("B", [5, 400003])
+@pytest.mark.parametrize("B", [5, 16, 17, 16384, 16385, 400003])
 def test_inference_kernel(cuda, B):
     """The inference forward (persistent workgroups, several 16-sample tiles
-    per wave at B = 400003, a partial last tile, and a single partial tile at
-    B = 5) against the oracle and against the training forward, which keeps
+    per wave at B = 400003, a partial last tile, a single partial tile at
+    B = 5, one tile per wave up to 16384 and two beyond) against the oracle and against the training forward, which keeps
     its activations and evaluates GELU through tanh."""
     import torch
     rng = np.random.default_rng(11)
