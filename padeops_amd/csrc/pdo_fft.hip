@@ -652,23 +652,22 @@ __global__ void __launch_bounds__(1024) k_pp_walls(TS *f, TS *w, long na, long s
     }
 }
 
-template <int L, size_t CE> constexpr int pp_walls_lines()
+// lines per workgroup of the wall projection: two line tiles and the twiddles
+// in at most `kib` KiB, 8 points per thread; above 256 threads only for rows
+// of up to 64 bytes (VAL: bytes of a stored value)
+template <int L, size_t CE, size_t VAL, size_t KIB> constexpr int pp_walls_lines()
 {
     int tx = 512 / (L / 8);
     if (tx < 1) tx = 1;
-    while (tx > 1 && (2 * (size_t)tx + 1) * L * CE > 80 * 1024) tx >>= 1;
+    while (tx > 1 && ((2 * (size_t)tx + 1) * L * CE > KIB * 1024 || (tx * (L / 8) > 256 && tx * VAL > 64))) tx >>= 1;
     return tx;
 }
 
-template <typename TS, typename TC, int L>
-static void launch_pp_walls(TS *f, TS *w, long na, long sb, long se, const TC *tw, const PadeWallTables &t, int nb,
-                            bool upd, hipStream_t st)
+template <typename TS, typename TC, int L, int TX>
+static void launch_pp_walls_tx(TS *f, TS *w, long na, long sb, long se, const TC *tw, const PadeWallTables &t, int nb,
+                               bool upd, hipStream_t st)
 {
-    constexpr size_t ce = 2 * sizeof(TC);
-    // two line tiles and the twiddles: at most 80 KiB, two workgroups to a CU
-    // (8 instead of 4 lines of 512 FP32 points: rows of 64 bytes)
-    constexpr int TX = pp_walls_lines<L, ce>();
-    const size_t lds = (2 * (size_t)TX + 1) * L * ce;
+    const size_t lds = (2 * (size_t)TX + 1) * L * 2 * sizeof(TC);
     dim3 grid((unsigned)((na + TX - 1) / TX), (unsigned)nb);
     if (upd)
         hipLaunchKernelGGL((k_pp_walls<TS, TC, L, TX, true>), grid, dim3(TX * (L / 8)), lds, st, f, w, na, sb, (int)se,
@@ -676,6 +675,27 @@ static void launch_pp_walls(TS *f, TS *w, long na, long sb, long se, const TC *t
     else
         hipLaunchKernelGGL((k_pp_walls<TS, TC, L, TX, false>), grid, dim3(TX * (L / 8)), lds, st, f, w, na, sb,
                            (int)se, tw, t.ax, t.ay, t.az, t.kcm, t.kcp);
+}
+
+// 80 KiB (two workgroups to a CU) doubles the rows of the longer lines, which
+// fields beyond the caches need: 256 x 256 planes, a projection with 512-point
+// lines, FP64 680 us in 64 KiB and 568 in 80, FP32 236 and 234 (in the band of
+// 512 x 512 planes more).  Where that leaves a few workgroups per CU the last
+// ones cost more: 64 x 64 x 256 FP32 25.1 and 28.7, 128 x 128 x 256 FP32 64 and
+// 69, 128 x 128 x 32 FP64 19.9 and 21.1; at most one per CU, 64 x 64 x 64 FP64
+// 19.4 and 17.5.
+template <typename TS, typename TC, int L>
+static void launch_pp_walls(TS *f, TS *w, long na, long sb, long se, const TC *tw, const PadeWallTables &t, int nb,
+                            bool upd, hipStream_t st)
+{
+    constexpr int BIG = pp_walls_lines<L, 2 * sizeof(TC), 2 * sizeof(TS), 80>();
+    constexpr int SMALL = pp_walls_lines<L, 2 * sizeof(TC), 2 * sizeof(TS), 64>();
+    const long groups = (na + BIG - 1) / BIG * nb;
+    if constexpr (BIG != SMALL) {
+        if (groups > 256 && groups < 2048)
+            return launch_pp_walls_tx<TS, TC, L, SMALL>(f, w, na, sb, se, tw, t, nb, upd, st);
+    }
+    launch_pp_walls_tx<TS, TC, L, BIG>(f, w, na, sb, se, tw, t, nb, upd, st);
 }
 
 template <typename TS, typename TC>

@@ -101,6 +101,20 @@ def test_walls_fp32(cuda, prec):
         assert e <= 2e-6
 
 
+@pytest.mark.parametrize("shape,prec", [((128, 128, 32), "f64"), ((64, 64, 128), "f64"), ((32, 32, 256), "f64"),
+                                        ((64, 64, 256), "f32_refine"), ((64, 64, 256), "f32_store"),
+                                        ((256, 16, 256), "f32_refine"), ((256, 256, 32), "f64")])
+def test_walls_workgroup_sizes(cuda, shape, prec):
+    """both sizes of the line tiles, chosen by the number of workgroups
+    (at most 256, below 2048)"""
+    nx, ny, nz = shape
+    d, spC, uh, vh, wh = _fields(nx, ny, nz, sum(shape))
+    got = _gpu(nx, ny, nz, d, uh, vh, wh, prec, cuda)
+    ref = PadePoissonWalls(spC, *d).projection(uh, vh, wh)
+    for g, r in zip(got[:3], ref):
+        assert rel_l2(g, r) <= (1e-12 if prec == "f64" else 2e-6)
+
+
 STOKES = [(32, 16, 32, 1.0), (64, 32, 16, 2.0), (16, 16, 256, 1.0)]
 
 
