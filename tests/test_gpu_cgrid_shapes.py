@@ -127,7 +127,10 @@ def _state(shape):
 
 
 @pytest.mark.parametrize("periodic", [(True, True, True), (False, True, False), (False, False, False)])
-@pytest.mark.parametrize("shape", [(32, 64, 32), (33, 17, 20), (16, 40, 49), (12, 10, 14), (32, 36, 1)])
+@pytest.mark.parametrize("shape", [(32, 64, 32), (33, 17, 20), (16, 40, 49), (12, 10, 14), (32, 36, 1),
+                                   # above 512 rows: two segments per wave, in several passes per launch and
+                                   # with the flux sums
+                                   (20, 544, 12), (12, 10, 600), (600, 10, 12), (10, 12, 1023)])
 def test_rhs(cuda, shape, periodic):
     import torch
     bc = tuple((0, 0) if q else (1, -1) for q in periodic)

@@ -183,3 +183,41 @@ def test_staggered_against_oracle(cuda, n, prec):
             getattr(s, name)(to_dev(f, dt, cuda), out, n1, n2, prec=prec)
             torch.cuda.synchronize()
             assert rel_l2(from_dev(out, (n1, n2, n + eout)), ref) < tol, (name, per)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dir,prec,per", [(1, "f32_refine", False), (2, "f32_refine", False), (2, "f32_refine", True),
+                                          (2, "f64", False), (3, "f32_refine", False), (3, "f64", True)])
+def test_fields_of_4_gib(cuda, dir, prec, per):
+    """fields whose byte offsets pass 32 bits: planes (y) or rows (z) of their
+    own 64-bit offsets, and whole lines along x, against the same passes over
+    parts of the field, which are addressed within 32 bits"""
+    import torch
+    n, dt = 400, torch.float64 if prec == "f64" else torch.float32
+    pencils = (2 ** 32 // dt.itemsize + (1 << 22)) // n
+    na = 1 << 12
+    nb = pencils // na + 1
+    f = torch.empty(n * na * nb, dtype=dt, device=cuda)
+    assert f.numel() * f.element_size() > 2 ** 32
+    g = torch.Generator(device=cuda).manual_seed(dir)
+    for part in f.chunk(64):
+        part.normal_(generator=g)
+    out = torch.full_like(f, float("nan"))
+    op = P.cd10()
+    assert op.init(n, 0.1, per) == 0
+    fn = (op.dd1, op.dd2, op.dd3)[dir - 1]
+    fn(f, out, na, nb, prec=prec)
+    # x, y: whole planes (nb the slowest index); z: pencils of one plane index
+    axis = 0 if dir < 3 else 1
+    shape = (nb, n * na) if dir < 3 else (n, nb, na)
+    F, G = f.view(shape), out.view(shape)
+    for b in (0, 1, nb // 2, nb - 2):
+        part = F.narrow(axis, b, 2).contiguous().flatten()
+        ref = torch.full_like(part, float("nan"))
+        fn(part, ref, na, 2, prec=prec)
+        got = G.narrow(axis, b, 2).contiguous().flatten()
+        torch.cuda.synchronize()
+        assert torch.equal(got, ref), (b, (got - ref).abs().max().item())
+    assert all(bool(torch.isfinite(part).all()) for part in out.chunk(16))
+    del f, out, F, G
+    torch.cuda.empty_cache()
