@@ -93,7 +93,7 @@ __global__ void __launch_bounds__(256) k_edge_tau(const TS *__restrict__ g, TS *
 }
 
 // the stress divergence of the three components in one pass (it was a
-// read-modify-write of the right-hand side per term: 27 words, now 15)
+// read-modify-write of the right-hand side per term: 27 words, now 14)
 template <typename TS, typename TC>
 __global__ void __launch_bounds__(256) k_stress_div(TS *u, TS *v, TS *w, StressSpectra S,
                                                    const double *__restrict__ k1, const double *__restrict__ k2,

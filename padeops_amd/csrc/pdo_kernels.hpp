@@ -35,10 +35,10 @@ struct ApplyArgs {
     const double *tab_d;
     const float *tab_f;
     int o_fac, o_spk, o_lhs, o_G, o_sp;
-    // overlapping segments (SHAPE_OVL_*): rows between segment starts (q0 or
-    // q0 + 1), segments coupled to one (nd, from d0 relative to it), and
-    // whether every segment has the same coupling rows
-    int q0, nd, d0, guni;
+    // overlapping segments (SHAPE_OVL_*): segments coupled to one (nd, from d0
+    // relative to it), and whether every segment has the same coupling rows
+    int nd, d0, guni;
+    int flat;          // strided: pencils numbered through all planes (0: grid y is the plane)
     int glds;          // words of coupling rows the workgroup stages in LDS (0: read from memory)
     unsigned smul, sdiv;  // start of segment s: s smul / D by the reciprocal sdiv = 2^31 / D + 1 (2^31: D = 1)
     double c[5];

@@ -298,7 +298,7 @@ static int prepare(OpObject *op, int kind, int bc1, int bcn, int dir, int prec, 
     if (shape == SHAPE_OVL_X || shape == SHAPE_OVL_STRIDED) {
         const OverlapTables &o = v->ovl;
         A.m = o.m; A.P = o.P; A.xr = 0; A.nbl = o.nbl; A.nbr = o.nbr;
-        A.q0 = o.q0; A.nd = o.nd; A.d0 = o.d0; A.guni = o.guni;
+        A.nd = o.nd; A.d0 = o.d0; A.guni = o.guni;
         const int steps = s.periodic ? o.P : std::max(o.P - 1, 1);
         A.smul = s.periodic ? s.n_sys : (o.P > 1 ? s.n_sys - o.m : 0);
         A.sdiv = steps > 1 ? (1u << 31) / steps + 1 : 1u << 31;

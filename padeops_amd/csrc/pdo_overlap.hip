@@ -182,8 +182,8 @@ __device__ __forceinline__ void ovl_solve(const ApplyArgs &A, double (&d)[M], PT
 // types and tables are scalar.  NPW = 32: two segments per wave (P <= 32);
 // tables from LDS when the types differ (LT, no periodicity).  Lanes run over
 // all na nb pencils of a y pass, not over those of one plane, so that a short
-// contiguous index leaves no lane idle (A.nb == 1 in the launch then, and
-// A.lgn == 1 says that pencils are numbered through).
+// contiguous index leaves no lane idle (A.flat); in a field of 4 GiB and more
+// grid y is the plane.
 // ---------------------------------------------------------------------------
 // Tables a workgroup reads from LDS: the coupling rows (A.glds words) and, with
 // LT, types 0, 1, 2 (or 3 alone).  Loaded to registers here, ahead of the field
@@ -237,8 +237,8 @@ __global__ void __launch_bounds__(1024) k_ovl_strided(ARGS B)
     const int pl = threadIdx.x % NPW;
     const unsigned id = blockIdx.x * NPW + pl;
     const unsigned na = (unsigned)A.na;
-    const bool act = A.lgn ? id < na * (unsigned)A.nb : id < na;
-    const unsigned b = A.lgn && act ? id / na : 0, a = act ? id - b * na : 0;
+    const bool act = A.flat ? id < na * (unsigned)A.nb : id < na;
+    const unsigned b = A.flat && act ? id / na : 0, a = act ? id - b * na : 0;
     const int ty = A.periodic ? 1 : (P == 1 ? 3 : (s == 0 ? 0 : (s == P - 1 ? 2 : 1)));
     const Seg g = segment<K>(A, s, M);
     const int r0 = g.r0, own = g.own;
@@ -450,11 +450,11 @@ template <int FAM, typename TS, int M> hipError_t strided_m(ApplyBatch &B, int c
     // pencils numbered through where 32-bit offsets reach the whole field
     const size_t nmax = (size_t)(A.n_in > A.n_out ? A.n_in : A.n_out);
     const size_t bytes = (size_t)A.na * A.nb * nmax * sizeof(TS);
-    for (int i = 0; i < count; i++) B.a[i].lgn = bytes < ((size_t)1 << 32) ? 1 : 0;
-    const size_t pen = A.lgn ? (size_t)A.na * A.nb : (size_t)A.na;
-    if (!A.lgn && (A.nb > 65535 || (size_t)A.na * sizeof(TS) >= ((size_t)1 << 32))) return hipErrorInvalidValue;
+    for (int i = 0; i < count; i++) B.a[i].flat = bytes < ((size_t)1 << 32) ? 1 : 0;
+    const size_t pen = A.flat ? (size_t)A.na * A.nb : (size_t)A.na;
+    if (!A.flat && (A.nb > 65535 || (size_t)A.na * sizeof(TS) >= ((size_t)1 << 32))) return hipErrorInvalidValue;
     if (A.P <= PMAX) {
-        const dim3 grid((unsigned)((pen + 63) / 64), A.lgn ? 1u : (unsigned)A.nb, (unsigned)count);
+        const dim3 grid((unsigned)((pen + 63) / 64), A.flat ? 1u : (unsigned)A.nb, (unsigned)count);
         const size_t red = (size_t)A.P * 2 * K * 64 * sizeof(double);
         return with_epilogue<FAM>(A, [&](auto e) {
             constexpr bool E = decltype(e)::value;
@@ -463,7 +463,7 @@ template <int FAM, typename TS, int M> hipError_t strided_m(ApplyBatch &B, int c
         });
     }
     if constexpr (M == MAXM && Fam<FAM>::SHIFT == 0) {
-        if (!A.lgn) return hipErrorInvalidValue;
+        if (!A.flat) return hipErrorInvalidValue;
         const dim3 grid((unsigned)((pen + 31) / 32), 1u, (unsigned)count);
         const size_t red = ((size_t)A.P * 2 * K * 32 + glds) * sizeof(double);
         const size_t tabs = sizeof(double) * 3 * type_words<K, M>();
