@@ -24,11 +24,11 @@
 //     from LDS (segment rows padded by one element against bank conflicts),
 //     and results go back through LDS to coalesced stores.
 // Other sizes, and the x pencils the x kernel does not take, run on the
-// overlapping segments of pdo_overlap.hip; what those leave (n below 16 or
-// above 1024, above 512 for the staggered operators and along y and z of
-// fields of 4 GiB and more, periodic edge fields of lengths that are no
-// multiple of 16) uses a one-lane-per-pencil kernel with global scratch,
-// computing in FP64.
+// overlapping segments of pdo_overlap.hip; what those leave (n below 16,
+// without periodicity 17 to 19, or above 1024; above 512 for the staggered
+// operators and along y and z of fields of 4 GiB and more; periodic edge
+// fields of lengths that are no multiple of 16) uses a one-lane-per-pencil
+// kernel with global scratch, computing in FP64.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
