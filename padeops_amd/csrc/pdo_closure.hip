@@ -324,9 +324,9 @@ __global__ void __launch_bounds__(256) k_closure_features(const TS *__restrict__
 // wherever the network's dissipation -tau_ij S_ij is negative; the number
 // of such points of each block goes to nfall[blockIdx.x].
 // Bound by the vector unit: the GELUs of the network, then the FP64 algebra.
-// 256^3 FP32: features 335, network 1600 and stress 350 us as three passes
-// that moved 224 bytes per point, now 1.4 ms in one that moves 60 (launches
-// timed by events; a kernel trace shows 1.65).
+// 256^3 FP32: features, network and stress as three passes that moved 224
+// bytes per point took 1.9 ms (2.3 in a kernel trace: 335, 1600 and 350 us),
+// one that moves 60 takes 1.4 (1.65).
 // ---------------------------------------------------------------------------
 template <typename TS>
 __global__ void __launch_bounds__(256, 4)

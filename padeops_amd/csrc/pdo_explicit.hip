@@ -12,10 +12,11 @@
 // it (2 words per point).  y and z: a lane carries T consecutive rows of its
 // pencil in registers and reads 4 NP rows more on either side, which its
 // neighbours in the direction read too (from the cache); the first and last
-// chunk are flush with the pencil, so closure rows sit at fixed registers.  x: whole
-// lines staged in LDS.  One thread per point with nine loads each, before,
-// spent its time on 64-bit index divisions: 256^3 FP64, two applications
-// 2 x 116 us, now in one pass 52 us along y and z, 81 us along x.
+// chunk are flush with the pencil, so closure rows sit at fixed registers.  x:
+// whole lines staged in LDS.  One thread per point with nine loads each spends
+// its time on 64-bit index divisions (256^3 FP64, two applications 2 x 116 us,
+// in one pass 52 us along y and z, 81 us along x); it is the shorter way for
+// fields of few points (launch_fast).
 #include <algorithm>
 
 #include "pdo_explicit.hpp"

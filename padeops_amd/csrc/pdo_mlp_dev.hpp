@@ -20,8 +20,8 @@
 // The 192 GELUs per sample bound it: 7 vector operations (2 of them
 // transcendental, at a quarter of the rate) and 2 for the BF16 roundings,
 // converted in pairs (one by one, with permutes to merge them, K = 16
-// operands and the results in accumulation registers it took 1600 us for
-// 16.8 M samples, now 1380).  Two tiles at a time halve the LDS reads of the
+// operands and the results in accumulation registers it took 1240 us for
+// 16.8 M samples, now 1030).  Two tiles at a time halve the LDS reads of the
 // weights and give the matrix cores and the vector unit independent work.
 #pragma once
 
